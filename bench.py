@@ -43,8 +43,16 @@ ROOT = Path(__file__).resolve().parent
 METRIC = "ResNet-18 fp32 images/s (b1,b32) on 1 GPU; per-op % HBM/MFMA roofline"
 PEAK_HBM_GBS = 8000.0      # MI355X HBM3E
 PEAK_FP32_MFMA_TF = 157.3  # MI355X dense fp32 matrix
+PEAK_SPLIT_TF = 2500.0 / 3  # fp32 products as three f16 products each (csrc/split_tile.h)
 # kernel-table names of the MFMA kernels (their work is priced in FLOP)
-MFMA_KERNELS = ("conv_igemm", "conv_stem", "conv_ws", "gemm_mfma", "gemm_dma", "gemm_skinny", "gemm_ws", "attention")
+MFMA_KERNELS = ("conv_igemm", "conv_stem", "conv_ws", "gemm_mfma", "gemm_split", "gemm_dma", "gemm_skinny", "gemm_ws", "attention")
+
+
+def mfma_peak(name: str) -> float:
+    """Peak of the matrix instruction a kernel of the timing table uses, in
+    fp32 products."""
+    split = name.startswith("gemm_split") or (name.startswith("conv_igemm") and name.endswith("_dma") and "c3" not in name)
+    return PEAK_SPLIT_TF if split else PEAK_FP32_MFMA_TF
 
 
 def load_package():
@@ -204,7 +212,7 @@ def kernel_table(ex, runtime, steps: int) -> list[dict]:
     for r in table:
         avg_ms = r["ms"] / r["launches"]
         if r["flops"] > 0 and r["name"].startswith(MFMA_KERNELS):
-            bound, unit, peak = "mfma", "TFLOP/s", PEAK_FP32_MFMA_TF
+            bound, unit, peak = "mfma", "TFLOP/s", mfma_peak(r["name"])
             achieved = r["flops"] / (r["ms"] * 1e-3) / 1e12
         elif r["name"].endswith("_fixup"):
             # stream-K partial-tile reduction: no algorithmic work of its own,
@@ -294,12 +302,14 @@ COPY_PROBE_BYTES = 256 << 20
 def conv_symbol_pattern(name: str) -> re.Pattern | None:
     """Kernel-table name -> regex over the HIP kernel symbol rocprofv3 reports,
     e.g. conv_igemm_128x128_k3x3_v4 -> conv_streamk_k<nnc::Tile<128, 128, ...>, 3, 3, true>,
-    conv_igemm_128x128_k3x3_dma -> conv_dma_k<nnc::Tile<128, 128, ...>, nnc::DmaPacked<..., 3, 3>, ...>."""
-    m = re.fullmatch(r"conv_igemm_(\d+)x(\d+)_k(\d+)x(\d+)(c3)?_dma", name)
+    conv_igemm_128x128_k3x3_dma -> conv_split_k<nnc::Tile<128, 128, ...>, nnc::SplitTaps<..., 3, 3, false>>."""
+    m = re.fullmatch(r"conv_igemm_(\d+)x(\d+)_k(\d+)x(\d+)(c3|p)?_dma", name)
     if m:
-        bm, bn, kh, kw, c3 = m.groups()
-        loader = rf"DmaSmallC<nnc::Tile<[^>]*>, {kh}, {kw}, 3>" if c3 else rf"DmaPacked<nnc::Tile<[^>]*>, {kh}, {kw}>"
-        return re.compile(rf"conv_dma_k<nnc::Tile<{bm}, {bn},[^>]*>, nnc::{loader}")
+        bm, bn, kh, kw, kind = m.groups()
+        if kind == "c3":
+            return re.compile(rf"conv_dma_k<nnc::Tile<{bm}, {bn},[^>]*>, nnc::DmaSmallC<nnc::Tile<[^>]*>, {kh}, {kw}, 3>")
+        proj = "true" if kind == "p" else "false"
+        return re.compile(rf"conv_split_k<nnc::Tile<{bm}, {bn},[^>]*>, nnc::SplitTaps<nnc::Tile<[^>]*>, {kh}, {kw}, {proj}>")
     m = re.fullmatch(r"conv_igemm_(\d+)x(\d+)_k(\d+|any)(?:x(\d+))?_(v4|s1)", name)
     if m:
         bm, bn, kh, kw, vec = m.groups()
@@ -411,11 +421,11 @@ def _op_roofline(runtime, fn, reps: int = 10, warmup: int = 3) -> dict:
     rows = []
     flops = sum(r["flops"] for r in table) / reps
     nbytes = sum(r["bytes"] for r in table) / reps
-    mfma = False
+    mfma, op_peak = False, 0.0
     for r in table:
         if r["flops"] > 0 and r["name"].startswith(MFMA_KERNELS):
-            achieved, unit, peak = r["flops"] / (r["ms"] * 1e-3) / 1e12, "TFLOP/s", PEAK_FP32_MFMA_TF
-            mfma = True
+            achieved, unit, peak = r["flops"] / (r["ms"] * 1e-3) / 1e12, "TFLOP/s", mfma_peak(r["name"])
+            mfma, op_peak = True, max(op_peak, peak)
         else:
             achieved, unit, peak = (r["bytes"] / (r["ms"] * 1e-3) / 1e9 if r["ms"] > 0 else 0.0), "GB/s", PEAK_HBM_GBS
         rows.append({"kernel": r["name"], "launches": r["launches"] // reps, "avg_us": round(r["ms"] / r["launches"] * 1e3, 2),
@@ -438,7 +448,7 @@ def _op_roofline(runtime, fn, reps: int = 10, warmup: int = 3) -> dict:
     lib.nnc_hip_graph_destroy()
     op_us = graph_ms / (launches * reps) * 1e3
     if mfma:
-        op_ach, unit, peak = flops / (op_us * 1e-6) / 1e12, "TFLOP/s", PEAK_FP32_MFMA_TF
+        op_ach, unit, peak = flops / (op_us * 1e-6) / 1e12, "TFLOP/s", op_peak
     else:
         op_ach, unit, peak = nbytes / (op_us * 1e-6) / 1e9, "GB/s", PEAK_HBM_GBS
     return {"kernels": rows, "op_us": round(op_us, 2), "op_achieved": round(op_ach, 2), "op_unit": unit,
@@ -735,7 +745,7 @@ def main() -> int:
 
     table = tables[args.batch]
     dom = table[0]
-    peak = PEAK_FP32_MFMA_TF if dom["bound"] == "mfma" else PEAK_HBM_GBS
+    peak = mfma_peak(dom["kernel"]) if dom["bound"] == "mfma" else PEAK_HBM_GBS
     traffic = None
     traffic_detail = None
     if not args.no_traffic:

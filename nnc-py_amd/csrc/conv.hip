@@ -1,4 +1,4 @@
-// Convolution entry points of the nnc ABI as implicit GEMM on fp32 MFMA
+// Convolution entry points of the nnc ABI as implicit GEMM on the matrix units
 // (reference: runtime/x86/ops.c:720-1504 and 3122-3227).
 //
 // GEMM view of one convolution (NCHW, weights [Co][Ci][kh][kw]):
@@ -16,15 +16,16 @@
 // Padding follows the reference: only the top/left pads are arguments, the
 // bottom/right extent comes from the output shape (c_emitter.py:1051-1058).
 //
-// Accumulation: one fp32 MFMA chain per workgroup segment (K <= 4608 at
+// Accumulation: fp32, one chain per workgroup segment (K <= 4608 at
 // ResNet-18 scale stays inside 1e-4 abs / 1e-3 rel of the reference's fp64
-// sum); shared tiles add their segments in fixed workgroup order.
+// sum; tap-major convolutions multiply f16 pieces of the fp32 operands, see
+// split_tile.h); shared tiles add their segments in fixed workgroup order.
 #include <math.h>
 #include <stdlib.h>
 
 #include <algorithm>
 
-#include "mfma_tile.h"
+#include "split_tile.h"
 
 namespace nnc {
 
@@ -320,7 +321,7 @@ __device__ void conv_finish_tile(const ConvArgs& a, int t, int g0, int g1, int f
 // and, counting in order, for every earlier store). Out-of-range rows and
 // pixels get an out-of-range buffer offset: loads read 0, stores are
 // dropped. Needs output (and residual) below 2 GiB.
-template <class T, bool RES>
+template <class T>
 __device__ __forceinline__ void store_tile(const ConvArgs& a, int i0, int j0, const floatx16 (&sum)[T::TM][T::TN]) {
     const int hw = a.Ho * a.Wo;
     const __amdgpu_buffer_rsrc_t rb = make_rsrc(a.bias), rr = make_rsrc(a.res), ro = make_rsrc(a.out);
@@ -333,16 +334,17 @@ __device__ __forceinline__ void store_tile(const ConvArgs& a, int i0, int j0, co
     }
     const int co0 = i0 + acc_row<T>(0, 0);  // this lane's first row; row (tm, r) adds a wave-uniform step
     const int act = a.act;
+    const bool has_res = a.res != nullptr;
 #pragma unroll
     for (int tm = 0; tm < T::TM; ++tm) {
         float bv[16];
-        float rv[T::TN][16];
+        float rv[T::TN][16] = {};
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const int co = co0 + tm * 32 + 8 * (r >> 2) + (r & 3);
             bv[r] = a.bias ? load_f32(rb, co < a.Co ? (uint32_t)co * 4u : kOutOfRange) : 0.f;
         }
-        if (RES) {
+        if (has_res) {
 #pragma unroll
             for (int tn = 0; tn < T::TN; ++tn)
 #pragma unroll
@@ -352,15 +354,29 @@ __device__ __forceinline__ void store_tile(const ConvArgs& a, int i0, int j0, co
                     rv[tn][r] = load_f32(rr, ok ? (pbase[tn] + (uint32_t)(co * hw)) * 4u : kOutOfRange);
                 }
         }
+        // relu as a select per element; sigmoid (a call per element) behind
+        // one branch per block
+#pragma unroll
+        for (int tn = 0; tn < T::TN; ++tn)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                float v = sum[tm][tn][r] + bv[r];
+                v = has_res ? v + rv[tn][r] : v;
+                rv[tn][r] = act == kActRelu && !(v > 0.0f) ? 0.0f : v;
+            }
+        if (act == kActSigmoid) {
+#pragma unroll
+            for (int tn = 0; tn < T::TN; ++tn)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) rv[tn][r] = activate(rv[tn][r], kActSigmoid);
+        }
 #pragma unroll
         for (int tn = 0; tn < T::TN; ++tn)
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const int co = co0 + tm * 32 + 8 * (r >> 2) + (r & 3);
                 const bool ok = pbase[tn] != kOutOfRange && co < a.Co;
-                float v = sum[tm][tn][r] + bv[r];
-                if (RES) v += rv[tn][r];
-                v = activate(v, act);
+                const float v = rv[tn][r];
                 __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), ro,
                                                       (int)(ok ? (pbase[tn] + (uint32_t)(co * hw)) * 4u : kOutOfRange),
                                                       0, 0);
@@ -376,10 +392,7 @@ __device__ __forceinline__ void conv_segment_out(const ConvArgs& a, const Stream
                                                  int i0, int j0, const floatx16 (&sum)[T::TM][T::TN]) {
     const int hw = a.Ho * a.Wo;
     if (BATCHED && seg.slot < 0 && a.out32) {
-        if (a.res)
-            store_tile<T, true>(a, i0, j0, sum);
-        else
-            store_tile<T, false>(a, i0, j0, sum);
+        store_tile<T>(a, i0, j0, sum);
         return;
     }
     if (seg.slot < 0) {
@@ -489,13 +502,9 @@ __global__ void __launch_bounds__(256, 2) conv_streamk_k(ConvArgs a, StreamK sk)
 //     k (one channel and tap), so the gather coalesces along image rows; an
 //     MFMA lane reads its k one ds_read_b32 at a time.
 // Out-of-range lanes (co >= Co, pixel >= Npix, tap outside the image, k >=
-// K) get an out-of-range offset, and the hardware writes 0 to LDS. The
-// loader (DmaPacked) needs Ci % 32 == 0 and weights packed tap-major
-// [Co][kh][kw][Ci] (for 1x1 kernels the reference layout). K is walked
-// tap-major: slice s is one tap t and 32 consecutive channels, so the tap -
-// and each pixel's in-image test and offset - is uniform over the slice and
-// channels differ by an SGPR offset. A: one dwordx4 load per 8 rows (lane l:
-// row l / 8, 16 bytes of the packed row).
+// K) get an out-of-range offset, and the hardware writes 0 to LDS. A: one
+// dwordx4 load per 8 rows (lane l: row l / 8, 16 bytes of the packed row).
+// Runs the RGB stem where its row kernels do not (DmaSmallC).
 // ---------------------------------------------------------------------------
 template <class T>
 struct DmaStage {
@@ -520,7 +529,7 @@ struct PixelTaps {
     typedef typename std::conditional<(KH * KW > 32), uint64_t, uint32_t>::type Mask;
     int bpo;
     Mask mask;
-    __device__ void init(const ConvArgs& a, int px) {
+    __device__ __forceinline__ void init(const ConvArgs& a, int px) {
         const bool valid = px < a.Npix;
         const int hw = a.Ho * a.Wo;
         const int p = valid ? px : 0;
@@ -539,168 +548,13 @@ struct PixelTaps {
                 mask |= (Mask)in << (r * KW + c);
             }
     }
-    __device__ bool inside(int tap) const { return ((mask >> tap) & 1u) != 0; }
-    __device__ uint32_t bit(int tap) const { return (uint32_t)(mask >> tap) & 1u; }
-};
-
-template <class T, int KH, int KW>
-struct DmaPacked {
-    typedef DmaStage<T> D;
-    static constexpr bool kFinishInKernel = true;
-    static constexpr int EXTRA_LDS_FLOATS = 0;
-    __device__ void prepare(float*, const ConvArgs&) {}
-    static constexpr int A_LOADS = T::BM / (8 * T::NW);  // dwordx4 loads per wave per slice, 8 rows each
-    static_assert(T::BM % (8 * T::NW) == 0, "A rows split evenly over the waves");
-    __amdgpu_buffer_rsrc_t rin, rw;
-    int wave, b_grp, b_kr0, CB, HW, W, Ci;
-    uint32_t avo[A_LOADS];
-    PixelTaps<KH, KW> px;
-    int t, cb;       // slice cursor: tap, 32-channel block
-    uint32_t bv;     // B offset of the slice being issued
-
-    __device__ void init(const ConvArgs& a, int wave_, int lane) {
-        rin = make_rsrc(a.in);
-        rw = make_rsrc(a.w);
-        wave = wave_;
-        b_grp = wave % D::PX_GROUPS;
-        b_kr0 = (wave / D::PX_GROUPS) * D::B_LOADS;
-        CB = a.Ci >> 5;
-        HW = a.H * a.W;
-        W = a.W;
-        Ci = a.Ci;
-    }
-    __device__ void tile(const ConvArgs& a, int i0, int j0, int lane) {
-        const int a_kc = (lane & 7) ^ ((lane >> 3) & 7);
-#pragma unroll
-        for (int i = 0; i < A_LOADS; ++i) {
-            const int co = i0 + (wave + T::NW * i) * 8 + (lane >> 3);
-            avo[i] = keep_or_oob((uint32_t)(co * a.ldw) * 4u + (uint32_t)a_kc * 16u, co < a.Co);
-        }
-        px.init(a, j0 + b_grp * 64 + lane);
-    }
-    __device__ void begin(int kb) {
-        t = kb / CB;
-        cb = kb - t * CB;
-    }
-    __device__ void step(bool more) {
-        const int cb1 = cb + 1 == CB ? 0 : cb + 1;
-        const int t1 = cb + 1 == CB ? t + 1 : t;
-        t = more ? t1 : t;
-        cb = more ? cb1 : cb;
-    }
-    // part 0: A and the first half of B; part 1: the rest of B
-    __device__ void issue(float* S, bool on, int part) {
-        if (part == 0) {
-            const uint32_t sa = (uint32_t)(t * Ci + cb * 32) * 4u;
-#pragma unroll
-            for (int i = 0; i < A_LOADS; ++i)
-                dma_load16(rw, S + (wave + T::NW * i) * 8 * 32, on ? avo[i] : kOutOfRange, sa);
-            const int r = t / KW, c = t - r * KW;
-            bv = keep_or_oob((uint32_t)(px.bpo + r * W + c) * 4u, on && px.inside(t));
-        }
-        const uint32_t s0 = (uint32_t)((cb * 32 + b_kr0) * HW) * 4u;
-        float* d0 = S + D::A_FLOATS + b_kr0 * T::BN + b_grp * 64;
-        constexpr int H = D::B_LOADS / 2;
-#pragma unroll
-        for (int i = part * H; i < (part + 1) * H; ++i) dma_load4(rin, d0 + i * T::BN, bv, s0 + (uint32_t)(i * HW) * 4u);
-    }
-};
-
-// A KH x KW convolution of `in` and a 1x1 projection of a second input (a
-// residual block's strided downsample) as one contraction, so the
-// projection needs no launch and no tensor of its own: k < KH*KW*Ci walks
-// `in` as DmaPacked does, the last pci k walk `pin` at the output pixel's
-// position times the projection stride (always inside that image). Weights
-// [Co][KH*KW*Ci + pci]: slice s starts at k = 32 s in both parts. Needs Ci
-// and pci multiples of 32.
-template <class T, int KH, int KW>
-struct DmaProj {
-    typedef DmaStage<T> D;
-    static constexpr bool kFinishInKernel = true;
-    static constexpr int EXTRA_LDS_FLOATS = 0;
-    __device__ void prepare(float*, const ConvArgs&) {}
-    static constexpr int A_LOADS = T::BM / (8 * T::NW);
-    static constexpr int TAPS = KH * KW;  // cursor tap TAPS: the projection
-    static_assert(T::BM % (8 * T::NW) == 0, "A rows split evenly over the waves");
-    __amdgpu_buffer_rsrc_t rin, rx, rw;
-    int wave, b_grp, b_kr0, CB, CBX, HW, HWX, W, Ci;
-    uint32_t avo[A_LOADS];
-    PixelTaps<KH, KW> px;
-    uint32_t xvo;  // this lane's pixel in the projection input at channel 0 (bytes; out of range past Npix)
-    int t, cb;     // slice cursor: tap (TAPS: projection), 32-channel block
-    uint32_t bv;
-
-    __device__ void init(const ConvArgs& a, int wave_, int lane) {
-        rin = make_rsrc(a.in);
-        rx = make_rsrc(a.pin);
-        rw = make_rsrc(a.w);
-        wave = wave_;
-        b_grp = wave % D::PX_GROUPS;
-        b_kr0 = (wave / D::PX_GROUPS) * D::B_LOADS;
-        CB = a.Ci >> 5;
-        CBX = a.pci >> 5;
-        HW = a.H * a.W;
-        HWX = a.pH * a.pW;
-        W = a.W;
-        Ci = a.Ci;
-    }
-    __device__ void tile(const ConvArgs& a, int i0, int j0, int lane) {
-        const int a_kc = (lane & 7) ^ ((lane >> 3) & 7);
-#pragma unroll
-        for (int i = 0; i < A_LOADS; ++i) {
-            const int co = i0 + (wave + T::NW * i) * 8 + (lane >> 3);
-            avo[i] = keep_or_oob((uint32_t)(co * a.ldw) * 4u + (uint32_t)a_kc * 16u, co < a.Co);
-        }
-        const int p = j0 + b_grp * 64 + lane;
-        px.init(a, p);
-        const bool valid = p < a.Npix;
-        const int q = valid ? p : 0;
-        const int hw = a.Ho * a.Wo;
-        const int n = q / hw, rem = q - n * hw;
-        const int oh = rem / a.Wo, ow = rem - oh * a.Wo;
-        xvo = keep_or_oob((uint32_t)(n * a.pci * HWX + oh * a.psh * a.pW + ow * a.psw) * 4u, valid);
-    }
-    __device__ void begin(int kb) {
-        const bool proj = kb >= TAPS * CB;
-        t = proj ? TAPS : kb / CB;
-        cb = proj ? kb - TAPS * CB : kb - t * CB;
-    }
-    __device__ void step(bool more) {
-        const bool wrap = t < TAPS && cb + 1 == CB;
-        const int cb1 = wrap ? 0 : cb + 1;
-        const int t1 = wrap ? t + 1 : t;
-        t = more ? t1 : t;
-        cb = more ? cb1 : cb;
-    }
-    // part 0: A and the first half of B; part 1: the rest of B
-    __device__ void issue(float* S, bool on, int part) {
-        const bool proj = t == TAPS;
-        if (part == 0) {
-            const uint32_t sa = (uint32_t)(t * Ci + cb * 32) * 4u;
-#pragma unroll
-            for (int i = 0; i < A_LOADS; ++i)
-                dma_load16(rw, S + (wave + T::NW * i) * 8 * 32, on ? avo[i] : kOutOfRange, sa);
-            const int r = t / KW, c = t - r * KW;
-            const uint32_t tap = keep_or_oob((uint32_t)(px.bpo + r * W + c) * 4u, on && !proj && px.inside(t));
-            bv = proj ? (on ? xvo : kOutOfRange) : tap;
-        }
-        const int hw = proj ? HWX : HW;
-        const uint32_t s0 = (uint32_t)((cb * 32 + b_kr0) * hw) * 4u;
-        float* d0 = S + D::A_FLOATS + b_kr0 * T::BN + b_grp * 64;
-        constexpr int H = D::B_LOADS / 2;
-        if (proj) {
-#pragma unroll
-            for (int i = part * H; i < (part + 1) * H; ++i) dma_load4(rx, d0 + i * T::BN, bv, s0 + (uint32_t)(i * hw) * 4u);
-        } else {
-#pragma unroll
-            for (int i = part * H; i < (part + 1) * H; ++i) dma_load4(rin, d0 + i * T::BN, bv, s0 + (uint32_t)(i * hw) * 4u);
-        }
-    }
+    __device__ __forceinline__ bool inside(int tap) const { return ((mask >> tap) & 1u) != 0; }
+    __device__ __forceinline__ uint32_t bit(int tap) const { return (uint32_t)(mask >> tap) & 1u; }
 };
 
 // Few input channels (the RGB stem): weights packed [Co][Kp], k = tap * CI +
 // ci tap-major, zero past K = kh*kw*CI up to Kp, a multiple of 32. A as in
-// DmaPacked; each B load is one k, whose tap and channel are uniform (the
+// above; each B load is one k, whose tap and channel are uniform (the
 // divisions by compile-time constants run on the scalar unit), and each lane
 // applies its pixel's in-image test for that tap.
 template <class T, int KH, int KW, int CI>
@@ -885,6 +739,142 @@ __global__ void __launch_bounds__(T::THREADS, DmaStage<T>::MIN_WAVES) conv_dma_k
         if (!have_next) break;
         seg = nxt;
     }
+}
+
+// ---------------------------------------------------------------------------
+// The tile engine's convolution on the 16-bit matrix units (split_tile.h),
+// for tap-major weights [Co][kh][kw][Ci] with Ci % 32 == 0 (1x1 weights are
+// tap-major as stored). A: the packed weight rows. B: a thread stages one
+// output pixel of the tile; a slice is one tap and 32 channels, so the tap's
+// in-image test and offset are computed once per slice and channels differ
+// by a wave-uniform offset, each load covering 64 consecutive pixels of one
+// channel. Slices walk the taps of a channel block before the next block
+// (neighbouring taps read the same lines).
+//
+// PROJ: a 1x1 projection of a second input (a residual block's strided
+// downsample) as the end of the same contraction: the last pci k walk `pin`
+// at the output pixel's position times the projection stride (always inside
+// that image). Weights [Co][kh*kw*Ci + pci]; Ci and pci multiples of 32.
+//
+// ResNet-18's 3x3 layers at batch 32, launch and fixup, against the fp32
+// matrix instruction on direct-to-LDS tiles: 64 channels 83 -> 45 us, 128 with
+// residual 75 -> 46, 256 72 -> 45, 512 78 -> 46; error against 64 bits 0.6 of
+// before.
+// ---------------------------------------------------------------------------
+template <class T, int KH, int KW, bool PROJ>
+struct SplitTaps : SplitStaged<T, T::BN, T::BN * 16 / T::THREADS> {
+    typedef SplitStaged<T, T::BN, T::BN * 16 / T::THREADS> S;
+    using S::koff;
+    using S::PER;
+    using S::v;
+    using S::x;
+    static constexpr int TAPS = KH * KW;  // cursor tap TAPS: the projection
+    // the projection's input and plane as differences: a choice between two
+    // members becomes a choice of addresses, which keeps the object in memory
+    const char* in;
+    int64_t to_x;
+    int CB, HW, to_hwx, W;
+    PixelTaps<KH, KW> px;
+    uint32_t xvo;  // this thread's pixel in the projection input (bytes; out of range past Npix)
+    uint32_t bv;   // and in the current slice's tap, or kOutOfRange
+    int t, cb;     // slice cursor: tap, 32-channel block
+    __device__ __forceinline__ void init(const ConvArgs& a) {
+        x = threadIdx.x % T::BN;  // lanes along pixels; channels uniform over a wave
+        koff = __builtin_amdgcn_readfirstlane(threadIdx.x / T::BN) * PER;
+        in = reinterpret_cast<const char*>(a.in);
+        CB = a.Ci >> 5;
+        HW = a.H * a.W;
+        W = a.W;
+        if (PROJ) {
+            to_x = reinterpret_cast<const char*>(a.pin) - in;
+            to_hwx = a.pH * a.pW - HW;
+        }
+    }
+    __device__ __forceinline__ void tile(const ConvArgs& a, int j0) {
+        px.init(a, j0 + x);
+        if (PROJ) {
+            const int p = j0 + x;
+            const bool valid = p < a.Npix;
+            const int q = valid ? p : 0, hw = a.Ho * a.Wo;
+            const int n = q / hw, rem = q - n * hw, oh = rem / a.Wo, ow = rem - oh * a.Wo;
+            xvo = keep_or_oob((uint32_t)(n * a.pci * (a.pH * a.pW) + oh * a.psh * a.pW + ow * a.psw) * 4u, valid);
+        }
+    }
+    __device__ __forceinline__ void begin(int kb) {
+        const bool proj = PROJ && kb >= TAPS * CB;
+        cb = proj ? kb - TAPS * CB : kb / TAPS;
+        t = proj ? TAPS : kb - cb * TAPS;
+    }
+    __device__ __forceinline__ void step() {
+        // the taps of a channel block, then the next block; after the last
+        // the projection's blocks
+        const bool proj = PROJ && t == TAPS;
+        const bool wrap = t + 1 == TAPS;
+        const bool last = PROJ && wrap && cb + 1 == CB;
+        cb = last ? 0 : cb + (proj || wrap);
+        t = last || proj ? TAPS : wrap ? 0 : t + 1;
+    }
+    // first k of the current slice in a packed weight row
+    __device__ __forceinline__ int k0(int ci) const { return t * ci + cb * 32; }
+    template <int Q>
+    __device__ __forceinline__ void load(bool on) {
+        const bool proj = PROJ && t == TAPS;
+        if (Q == 0) {
+            const int r = t / KW, c = t - r * KW;
+            const uint32_t tap = keep_or_oob((uint32_t)(px.bpo + r * W + c) * 4u, px.inside(t));
+            const uint32_t m = 0u - (uint32_t)proj;
+            bv = keep_or_oob(PROJ ? (tap & ~m) | (xvo & m) : tap, on);
+        }
+        const int hw = PROJ ? HW + (to_hwx & -(int)proj) : HW;
+        const __amdgpu_buffer_rsrc_t rs =
+            make_rsrc(reinterpret_cast<const float*>(PROJ ? in + (to_x & -(int64_t)proj) : in));
+        const uint32_t s0 = (uint32_t)((cb * 32 + 16 * Q + koff) * hw) * 4u;
+#pragma unroll
+        for (int i = 0; i < PER; ++i)
+            v[Q][i] = __uint_as_float(
+                __builtin_amdgcn_raw_buffer_load_b32(rs, (int)bv, (int)(s0 + (uint32_t)(i * hw) * 4u), 0));
+    }
+};
+
+template <class T, class B>
+struct ConvSplit {
+    static constexpr bool LOADS_BRANCH = false;
+    const ConvArgs& args;
+    const StreamK& sk;
+    int wg;
+    KcSplit<T, T::BM, true> a;
+    B b;
+    __device__ __forceinline__ ConvSplit(const ConvArgs& c, const StreamK& sk_, int wg_) : args(c), sk(sk_), wg(wg_) {
+        a.init();
+        b.init(c);
+    }
+    __device__ __forceinline__ void tile(int t) {
+        const int i0 = t % args.tiles_m * T::BM, j0 = t / args.tiles_m * T::BN;
+        a.tile(args.w + (int64_t)i0 * args.ldw, args.ldw, args.Co - i0);
+        b.tile(args, j0);
+    }
+    __device__ __forceinline__ void begin(int it) { b.begin(it); }
+    __device__ __forceinline__ void step() { b.step(); }
+    template <int Q>
+    __device__ __forceinline__ void load_a(int, int half, bool on) { a.template load<Q>(b.k0(args.Ci) + half * 16, args.K, on); }
+    template <int Q>
+    __device__ __forceinline__ void load_b(int, int, bool on) { b.template load<Q>(on); }
+    __device__ __forceinline__ void out(const Segment& seg, const floatx16 (&sum)[T::TM][T::TN]) {
+        // a whole tile straight to the output (below 2 GiB: conv_run cuts
+        // larger ones), a partial one to the workgroup's slot
+        if (seg.slot < 0)
+            store_tile<T>(args, seg.tile % args.tiles_m * T::BM, seg.tile / args.tiles_m * T::BN, sum);
+        else
+            store_slot<T>(args.ws, wg, seg.slot, sum);
+    }
+};
+
+template <class T, class B>
+__global__ void __launch_bounds__(T::THREADS, 2) conv_split_k(ConvArgs a, StreamK sk) {
+    extern __shared__ __align__(16) float lds[];
+    const int wg = xcd_remap(blockIdx.x, sk.G);
+    ConvSplit<T, B> p(a, sk, wg);
+    split_run<T>(p, sk, wg, reinterpret_cast<char*>(lds));
 }
 
 // ---------------------------------------------------------------------------
@@ -1356,6 +1346,7 @@ static constexpr int kMaxInKernelParts = 4;
 typedef Tile<128, 128, 32, 2, 2> ConvT128;  // Co >= 128: 2x2 blocks per wave
 typedef Tile<64, 128, 32, 1, 4> ConvT64;    // Co == 64, many pixels: 2x1 blocks per wave
 typedef Tile<64, 64, 32, 2, 2> ConvTSmall;  // short K or few pixels: 1 block per wave
+typedef Tile<64, 256, 32, 1, 4> ConvW64;     // the split kernels' Co <= 64: 2x2 blocks per wave
 
 template <class T, int KH, int KW, bool AVEC>
 static void launch_conv_t(ConvArgs& a, const char* entry) {
@@ -1439,11 +1430,65 @@ static void launch_conv_dma_t(ConvArgs& a, const char* entry, const char* name) 
     if (sk.needs_fixup() && !a.cnt) launch_conv_fixup<T>(a, sk);
 }
 
-template <class T, int KH, int KW>
-static void launch_conv_dma(ConvArgs& a, const char* entry) {
-    char name[64];
-    snprintf(name, sizeof name, "conv_igemm_%dx%d_k%dx%d_dma", T::BM, T::BN, KH, KW);
-    launch_conv_dma_t<T, DmaPacked<T, KH, KW>>(a, entry, name);
+template <class T, int KH, int KW, bool PROJ>
+static void launch_conv_split(ConvArgs& a, const StreamK& sk, const char* entry) {
+    auto kernel = conv_split_k<T, SplitTaps<T, KH, KW, PROJ>>;
+    const size_t lds = (size_t)split_lds_bytes<T>();
+    // once per kernel, thread-safe (C++ static initialisation): the LDS limit
+    static const bool ready = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                  (int)lds) == hipSuccess;
+    if (!ready) return fail(NNC_HIP_EDEVICE, entry, "hipFuncSetAttribute failed");
+    a.tiles_m = (int)ceil_div(a.Co, T::BM);
+    a.tiles_n = (int)ceil_div(a.Npix, T::BN);
+    a.ws = nullptr;
+    a.cnt = nullptr;
+    if (sk.needs_fixup()) {
+        const size_t ws_bytes = (size_t)sk.G * 2 * T::BM * T::BN * sizeof(float);
+        a.ws = workspace(ws_bytes);
+        if (!a.ws) return partials_fail(entry, ws_bytes);
+    }
+    char name[64];  // (the timing table's name of tap-major convolutions)
+    snprintf(name, sizeof name, "conv_igemm_%dx%d_k%dx%d%s_dma", T::BM, T::BN, KH, KW, PROJ ? "p" : "");
+    set_work(2.0 * a.Co * (double)a.Npix * a.K, 0.0);
+    launch(name, kernel, dim3(sk.G), dim3(T::THREADS), lds, a, sk);
+    if (sk.needs_fixup()) launch_conv_fixup<T>(a, sk);
+}
+
+// A tap-major convolution on split_tile.h's tiles (plan_conv_split). Their
+// epilogue stores through 32-bit offsets: an output of 2 GiB or more goes in
+// ranges of images, a single image's in ranges of channels.
+template <int KH, int KW, bool PROJ>
+static void conv_split(ConvArgs& a, const char* entry) {
+    if (!a.out32) {
+        const int64_t hw = (int64_t)a.Ho * a.Wo, most = (((int64_t)1 << 31) - 1) / 4;
+        const bool images = a.N > 1;
+        const int64_t unit = images ? a.Co * hw : hw, total = images ? a.N : a.Co;
+        if (!images && hw > most) return fail(NNC_HIP_EUNSUPP, entry, "an output plane spans 2 GiB or more");
+        const int64_t per = std::max<int64_t>(1, most / unit);
+        for (int64_t u = 0; u < total; u += per) {
+            ConvArgs c = a;
+            const int64_t n = std::min(per, total - u);
+            c.out = a.out + u * unit;
+            if (a.res) c.res = a.res + u * unit;
+            if (images) {
+                c.N = (int)n;
+                c.Npix = (int)(n * hw);
+                c.in = a.in + u * a.Ci * a.H * a.W;
+                if (PROJ) c.pin = a.pin + u * a.pci * a.pH * a.pW;
+            } else {
+                c.Co = (int)n;
+                c.w = a.w + u * a.ldw;
+                if (a.bias) c.bias = a.bias + u;
+            }
+            c.out32 = n * unit <= most;
+            conv_split<KH, KW, PROJ>(c, entry);
+        }
+        return;
+    }
+    const ConvSplitPlan p = plan_conv_split(a.Co, a.Npix, a.K, cu_count());
+    if (p.tile.bn == 256) return launch_conv_split<ConvW64, KH, KW, PROJ>(a, p.sk, entry);
+    if (p.tile.bm == 64) return launch_conv_split<ConvTSmall, KH, KW, PROJ>(a, p.sk, entry);
+    launch_conv_split<ConvT128, KH, KW, PROJ>(a, p.sk, entry);
 }
 
 template <int NS, bool PROJ>
@@ -1869,12 +1914,9 @@ static void launch_conv_stem(ConvArgs& a, const char* entry) {
 template <class T>
 static void launch_conv(ConvArgs& a, bool avec, bool dma, const char* entry) {
     if (dma && launch_conv_ws<false>(a, entry)) return;
+    if (dma) return a.kh == 3 ? conv_split<3, 3, false>(a, entry) : conv_split<1, 1, false>(a, entry);
     a.tiles_m = (int)ceil_div(a.Co, T::BM);
     a.tiles_n = (int)ceil_div(a.Npix, T::BN);
-    if (dma) {
-        if (a.kh == 3) return launch_conv_dma<T, 3, 3>(a, entry);
-        return launch_conv_dma<T, 1, 1>(a, entry);
-    }
 #define NNC_CONV_KS(KH, KW)                                                 \
     if (avec) launch_conv_t<T, KH, KW, true>(a, entry);                     \
     else launch_conv_t<T, KH, KW, false>(a, entry);                         \
@@ -1986,7 +2028,7 @@ static void conv_run(Tensor* in, Tensor* w, Tensor* b, Tensor* out, int kh, int 
             return fail(NNC_HIP_EUNSUPP, name,
                         "packed weights need Ci % 32 == 0, a 1x1 or 3x3 kernel and 16-byte alignment");
     }
-    bool dma = dma_ok && (packed || (kh == 1 && kw == 1));
+    bool dma = dma_ok && K > 0 && (packed || (kh == 1 && kw == 1));
     if (a.N == 0 || a.Co == 0 || a.Ho <= 0 || a.Wo <= 0) return;
     // reference-layout 3x3 weights of a large convolution: a tap-major copy
     // (one small transpose kernel) pays for itself on the direct-to-LDS path
@@ -2130,15 +2172,6 @@ static void conv_maxpool_run(Tensor* in, Tensor* w, Tensor* b, Tensor* out, int 
     }
 }
 
-template <class T>
-static void launch_conv_proj(ConvArgs& a, const char* entry) {
-    a.tiles_m = (int)ceil_div(a.Co, T::BM);
-    a.tiles_n = (int)ceil_div(a.Npix, T::BN);
-    char name[64];
-    snprintf(name, sizeof name, "conv_igemm_%dx%d_k3x3p_dma", T::BM, T::BN);
-    launch_conv_dma_t<T, DmaProj<T, 3, 3>>(a, entry, name);
-}
-
 // nnc_hip_conv_proj: act(conv3x3(in, w[:, :9*Ci]) + conv1x1(x, w[:, 9*Ci:],
 // stride psh x psw) + bias); w packed [Co][9*Ci + Cx].
 static void conv_proj_run(Tensor* in, Tensor* w, Tensor* b, Tensor* x, Tensor* out, int kh, int kw, int sh, int sw,
@@ -2195,10 +2228,7 @@ static void conv_proj_run(Tensor* in, Tensor* w, Tensor* b, Tensor* x, Tensor* o
     a.out32 = (int64_t)a.N * a.Co * a.Ho * a.Wo * 4 < ((int64_t)1 << 31);
     if (a.N == 0 || a.Co == 0 || a.Ho <= 0 || a.Wo <= 0) return;
     if (launch_conv_ws<true>(a, name)) return;
-    // the tile choice of conv_run
-    if (a.K >= 512 && a.Co >= 128 && a.Npix >= 1024) return launch_conv_proj<ConvT128>(a, name);
-    if (a.K >= 512 && a.Co <= 64 && a.Npix >= 4096) return launch_conv_proj<ConvT64>(a, name);
-    launch_conv_proj<ConvTSmall>(a, name);
+    conv_split<3, 3, true>(a, name);
 }
 
 // ---------------------------------------------------------------------------

@@ -217,11 +217,31 @@ bool ws_kernel(const char* op, int kh, int kw, bool proj, int64_t Co, int64_t np
     return true;
 }
 
+constexpr int kMaxInKernelParts = 4;
+
+// conv.hip conv_split, named by the library's tile. Schedule, fixup launches
+// and prices are those of the fp32-MFMA tiles whose measured times the model
+// is fitted to: an upper bound for the library's split kernels.
+void split_conv(const char* op, int kh, int kw, bool proj, int64_t Co, int64_t npix, int64_t K, double flops,
+                double bytes, double weight_bytes) {
+    const nnc::SplitTileCost tile = nnc::plan_conv_split(Co, npix, K, kCUs).tile;
+    char name[64];
+    snprintf(name, sizeof name, "conv_igemm_%dx%d_k%dx%d%s_dma", tile.bm, tile.bn, kh, kw, proj ? "p" : "");
+    const MfmaKind& k = (K >= 512 && Co >= 128 && npix >= 1024) ? kConv128
+                        : (K >= 512 && Co <= 64 && npix >= 4096) ? kConv64x128 : kConv64;
+    const int tiles = (int)(ceil_div(Co, k.bm) * ceil_div(npix, k.bn));
+    MfmaResult m = mfma_kernel(k, tiles, K, bytes, weight_bytes);
+    record(op, name, m.us, flops, bytes);
+    if (!m.sk.needs_fixup()) return;
+    const int64_t per = m.sk.total() / m.sk.G;
+    if (&k == &kConv64x128 && (m.sk.iters + per - 1) / per + 1 <= kMaxInKernelParts) return;
+    record(op, "conv_streamk_fixup", fixup_us(k, m.sk), 0.0, 0.0);
+}
+
 // ---------------------------------------------------------------------------
 // convolution: conv.hip conv_run's choices
 // ---------------------------------------------------------------------------
 constexpr double kRepackMinFlops = 1e9;
-constexpr int kMaxInKernelParts = 4;
 
 void conv(const char* op, Tensor* in, Tensor* w, Tensor* b, Tensor* res, Tensor* out, int kh, int kw, bool packed) {
     if (!in || !w || !out || !in->shape || !w->shape || !out->shape || in->ndim != 4 || out->ndim != 4) return;
@@ -257,10 +277,8 @@ void conv(const char* op, Tensor* in, Tensor* w, Tensor* b, Tensor* res, Tensor*
     } else {
         if (dma && ws_kernel(op, kh, kw, false, Co, npix, K, flops, bytes, nbytes(w))) return;
         const int tile = (K >= 512 && Co >= 128 && npix >= 1024) ? 2 : (K >= 512 && Co <= 64 && npix >= 4096) ? 1 : 0;
-        if (dma) {
-            k = tile == 2 ? &kConv128 : tile == 1 ? &kConv64x128 : &kConv64;
-            snprintf(name, sizeof name, "conv_igemm_%dx%d_k%dx%d_dma", k->bm, k->bn, kh, kw);
-        } else {
+        if (dma) return split_conv(op, kh, kw, false, Co, npix, K, flops, bytes, nbytes(w));
+        {
             k = tile == 2 ? &kGather128 : tile == 1 ? &kGather64x128 : &kGather64;
             const bool known = (kh == 1 && kw == 1) || (kh == 3 && kw == 3) || (kh == 7 && kw == 7);
             const char* vec = K % 4 == 0 ? "v4" : "s1";
@@ -273,9 +291,9 @@ void conv(const char* op, Tensor* in, Tensor* w, Tensor* b, Tensor* res, Tensor*
     MfmaResult m = mfma_kernel(*k, tiles, K, bytes, nbytes(w));
     record(op, name, m.us, flops, bytes);
     if (!m.sk.needs_fixup()) return;
-    // the 64x128 direct-to-LDS kernels finish a shared tile in the kernel
+    // the 64x128 direct-to-LDS stem finishes a shared tile in the kernel
     // when at most kMaxInKernelParts workgroups share it
-    const bool fin = (dma && !stem && k == &kConv64x128) || k == &kStem64x128;
+    const bool fin = k == &kStem64x128;
     const int64_t per = m.sk.total() / m.sk.G;
     // (its cost is inside the kernel's fitted efficiency)
     if (fin && (m.sk.iters + per - 1) / per + 1 <= kMaxInKernelParts) return;
@@ -348,6 +366,14 @@ void gemm(const char* op, int M, int N, int K, int batches, bool a_kc, bool b_kc
     static const char* kinds[4] = {"k4", "k1", "x4", "x1"};
     const int ak = a_kc ? (a4 ? 0 : 1) : (a4 ? 2 : 3), bk = b_kc ? (b4 ? 0 : 1) : (b4 ? 2 : 3);
     char name[64];
+    const bool fp32 = nnc::gemm_stays_fp32(ceil_div(M, 64) * ceil_div(N, 64) * batches, ceil_div(K, kBK), a4 && b4, kCUs);
+    if (!fp32) {
+        // gemm.hip's split kernels, priced as the fp32-MFMA tiles
+        const MfmaKind& k = a4 && b4 && big ? kGemm128 : kGemm64;
+        snprintf(name, sizeof name, "gemm_split_%dx%d_%s%s", k.bm, k.bn, a_kc ? "k" : "x", b_kc ? "k" : "x");
+        const int tiles = (int)(ceil_div(M, k.bm) * ceil_div(N, k.bn) * batches);
+        return record(op, name, mfma_kernel(k, tiles, K, bytes, b_bytes).us, flops, bytes);
+    }
     if (a4 && b4) {
         // direct-to-LDS: 128x128 or 64x64 tiles (one workgroup per CU over
         // 16 or more K slices); shared tiles of at most four partials are
@@ -561,7 +587,7 @@ void nnc_hip_conv_add_relu(Tensor* in, Tensor* w, Tensor* b, Tensor* res, Tensor
     (void)sh, (void)sw, (void)ph, (void)pw;
     conv("nnc_hip_conv_add_relu", in, w, b, res, out, kh, kw, false);
 }
-// conv.hip conv_proj_run: one direct-to-LDS kernel over K = 9*Ci + Cx
+// conv.hip conv_proj_run: one kernel over K = 9*Ci + Cx
 void nnc_hip_conv_proj(Tensor* in, Tensor* w, Tensor* b, Tensor* x, Tensor* out, int kh, int kw, int sh, int sw,
                        int ph, int pw, int psh, int psw, int act) {
     (void)kh, (void)kw, (void)sh, (void)sw, (void)ph, (void)pw, (void)psh, (void)psw, (void)act;
@@ -573,17 +599,7 @@ void nnc_hip_conv_proj(Tensor* in, Tensor* w, Tensor* b, Tensor* x, Tensor* out,
     const double flops = 2.0 * Co * (double)npix * K;
     const double bytes = nbytes(in) + nbytes(x) + nbytes(w) + nbytes(b) + nbytes(out);
     if (ws_kernel(op, 3, 3, true, Co, npix, K, flops, bytes, nbytes(w))) return;
-    const MfmaKind* k = (K >= 512 && Co >= 128 && npix >= 1024) ? &kConv128
-                        : (K >= 512 && Co <= 64 && npix >= 4096) ? &kConv64x128 : &kConv64;
-    char name[64];
-    snprintf(name, sizeof name, "conv_igemm_%dx%d_k3x3p_dma", k->bm, k->bn);
-    const int tiles = (int)(ceil_div(Co, k->bm) * ceil_div(npix, k->bn));
-    MfmaResult m = mfma_kernel(*k, tiles, K, bytes, nbytes(w));
-    record(op, name, m.us, flops, bytes);
-    if (!m.sk.needs_fixup()) return;
-    const int64_t per = m.sk.total() / m.sk.G;
-    if (k == &kConv64x128 && (m.sk.iters + per - 1) / per + 1 <= kMaxInKernelParts) return;
-    record(op, "conv_streamk_fixup", fixup_us(*k, m.sk), 0.0, 0.0);
+    split_conv(op, 3, 3, true, Co, npix, K, flops, bytes, nbytes(w));
 }
 void nnc_hip_conv_packed(Tensor* in, Tensor* w, Tensor* b, Tensor* res, Tensor* out, int kh, int kw, int sh, int sw,
                          int ph, int pw, int act) {

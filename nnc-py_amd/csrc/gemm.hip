@@ -1,14 +1,14 @@
 // Gemm, Gemm_nt and MatMul of the nnc ABI (runtime/x86/ops.c:1607-1886).
 //
-// Dense products run on the fp32 MFMA tile engine (mfma_tile.h), stream-K
-// scheduled over batches x tiles x K slices. Operands whose rows are 16-byte
-// aligned on both sides (k-contiguous or x-contiguous) go straight from
-// global memory into LDS (gemm_dma_k: 64x64 tiles with four LDS stages,
-// 128x128 tiles with two); shared tiles are finished inside the kernel by
-// the last workgroup to arrive, or by a fixup kernel when split further.
-// Other layouts (unaligned rows, K or M/N not a multiple of 4) stage through
-// registers (gemm_streamk_k, scalar loads where needed). Both sum a shared
-// tile's partials in fixed workgroup order. Products with one
+// Dense products run on split_tile.h's tiles (fp32 operands as f16 pieces on
+// the 16-bit matrix units), stream-K scheduled over batches x tiles x K
+// slices: gemm_split_k, rows of any alignment, tile shape and schedule by
+// plan_split's estimate. One round of 64x64 tiles over a few slices stays on
+// the fp32 matrix instruction (gemm_stays_fp32): gemm_dma_k where the rows
+// are 16-byte aligned (straight from global memory into LDS, four stages),
+// gemm_streamk_k otherwise. Shared tiles are finished inside the kernel by
+// the last workgroup to arrive, or by a fixup kernel when split further, the
+// partials summed in fixed workgroup order. Products with one
 // output row or column are HBM-bound and use dedicated kernels:
 //   gemv_xc_k  out[j] = sum_k a[k] * B[k][j]   (B row-major; float4 columns,
 //              K split across workgroups, deterministic partial reduction)
@@ -19,13 +19,13 @@
 // K split over its waves, summed in LDS).
 //
 // The reference accumulates Gemm in fp64 and MatMul with a Kahan fp32 sum;
-// here every product accumulates in fp32 (two-level in the register-staged
-// kernel), within the 1e-4 absolute / 1e-3 relative bar.
+// here every product accumulates in fp32 (two-level where rows are unaligned
+// and in 64x64 tiles), within the 1e-4 absolute / 1e-3 relative bar.
 //
 // DIVERGES: batched MatMul steps A by M*K and B by K*N per batch (numpy /
 // ONNX semantics). The reference steps by the batch count (ops.c:1687-1704),
 // which is only correct for a single batch.
-#include "mfma_tile.h"
+#include "split_tile.h"
 
 #include <stdlib.h>
 
@@ -49,6 +49,19 @@ struct GemmArgs {
     int* cnt;  // stream-K tile counters of the in-kernel finish, or null
     int out32;  // one batch of out (and C) below 2 GiB: whole tiles use 32-bit buffer offsets
 };
+
+// Tile `rem` of a batch: bands of kTileBand tile rows, each column by column,
+// so that 64 consecutive tiles (the workgroups of one XCD) share 8 row blocks
+// of A and 8 column blocks of B through its L2 rather than 2 column blocks
+// and every row block.
+static constexpr int kTileBand = 8;
+__device__ __forceinline__ void tile_pos(const GemmArgs& g, int rem, int& mt, int& nt) {
+    const int per_band = kTileBand * g.tiles_n;
+    const int band = rem / per_band, in = rem - band * per_band;
+    const int rows = min(kTileBand, g.tiles_m - band * kTileBand);
+    nt = in / rows;
+    mt = band * kTileBand + (in - nt * rows);
+}
 
 __device__ __forceinline__ float gemm_finish(const GemmArgs& g, int i, int j, float v) {
     float o = g.alpha * v;
@@ -143,7 +156,8 @@ __global__ void __launch_bounds__(256, 2) gemm_streamk_k(GemmArgs g, StreamK sk)
     Segment seg;
     while (walk.next(sk, seg)) {
         const int batch = seg.tile / per_batch, rem = seg.tile - batch * per_batch;
-        const int mt = rem % g.tiles_m, nt = rem / g.tiles_m;
+        int mt, nt;
+        tile_pos(g, rem, mt, nt);
         const int i0 = mt * T::BM, j0 = nt * T::BN;
         typename PA::type la;
         typename PB::type lb;
@@ -192,8 +206,10 @@ __global__ void __launch_bounds__(256) gemm_fixup_k(GemmArgs g, StreamK sk) {
     if (e4 >= T::BM * T::BN / 4) return;
     const int per_batch = g.tiles_m * g.tiles_n;
     const int batch = t / per_batch, rem = t - batch * per_batch;
-    const int i = (rem % g.tiles_m) * T::BM + (e4 * 4) / T::BN;
-    const int j = (rem / g.tiles_m) * T::BN + (e4 * 4) % T::BN;
+    int mt, nt;
+    tile_pos(g, rem, mt, nt);
+    const int i = mt * T::BM + (e4 * 4) / T::BN;
+    const int j = nt * T::BN + (e4 * 4) % T::BN;
     if (i >= g.M || j >= g.N) return;
     float4 v = reinterpret_cast<const float4*>(partial_slot<T>(g.ws, g0, first_slot))[e4];
     for (int w = g0 + 1; w <= g1; ++w) {
@@ -321,13 +337,15 @@ struct XcOperand {
 // gemm_fixup_k, so the result is the same to the bit), then alpha / beta * C
 // / relu. Each thread handles 4 consecutive columns of a tile row.
 template <class T>
-__device__ void gemm_finish_tile(const GemmArgs& g, int t, int g0, int g1, int first_slot) {
+__device__ __forceinline__ void gemm_finish_tile(const GemmArgs& g, int t, int g0, int g1, int first_slot) {
     constexpr int E = T::BM * T::BN / 1024;  // float4 per thread
     constexpr int CH = E < 4 ? E : 4;         // float4 in flight per partial (register budget)
     const __amdgpu_buffer_rsrc_t rws = make_rsrc(g.ws);
     const int per_batch = g.tiles_m * g.tiles_n;
     const int batch = t / per_batch, rem = t - batch * per_batch;
-    const int i0 = (rem % g.tiles_m) * T::BM, j0 = (rem / g.tiles_m) * T::BN;
+    int mt, nt;
+    tile_pos(g, rem, mt, nt);
+    const int i0 = mt * T::BM, j0 = nt * T::BN;
     const uint32_t first = slot_byte_offset<T>(g0, first_slot);
     for (int e0 = 0; e0 < E; e0 += CH) {
         f32x4 v[CH];
@@ -419,12 +437,12 @@ struct SliceCursor {
     Segment seg;
     int it;
     bool valid;
-    __device__ SliceCursor(const StreamK& sk, int wg) : walk(sk, wg) {
+    __device__ __forceinline__ SliceCursor(const StreamK& sk, int wg) : walk(sk, wg) {
         valid = walk.next(sk, seg);
         it = seg.kb;
     }
     // to the next slice; true if it starts a new segment
-    __device__ bool advance(const StreamK& sk) {
+    __device__ __forceinline__ bool advance(const StreamK& sk) {
         if (++it < seg.ke) return false;
         valid = walk.next(sk, seg);
         it = seg.kb;
@@ -457,7 +475,9 @@ __global__ void __launch_bounds__(T::THREADS, (GemmDma<T, NS>::MIN_WAVES)) gemm_
     ob.init_read((wave % T::WN) * T::WAVE_N, lane);
     auto set_tile = [&](int tile) {
         const int batch = tile / per_batch, rem = tile - batch * per_batch;
-        const int i0 = (rem % g.tiles_m) * T::BM, j0 = (rem / g.tiles_m) * T::BN;
+        int mt, nt;
+        tile_pos(g, rem, mt, nt);
+        const int i0 = mt * T::BM, j0 = nt * T::BN;
         oa.tile(g.A + batch * g.sa + OA::origin(i0, g.lda), g.lda, g.M - i0, wave, lane);
         ob.tile(g.B + batch * g.sb + OB::origin(j0, g.ldb), g.ldb, g.N - j0, wave, lane);
     };
@@ -483,7 +503,9 @@ __global__ void __launch_bounds__(T::THREADS, (GemmDma<T, NS>::MIN_WAVES)) gemm_
     int cs = 0, ls = NS - 1;  // stages being computed and loaded
     while (true) {
         const int batch = seg.tile / per_batch, rem = seg.tile - batch * per_batch;
-        const int i0 = (rem % g.tiles_m) * T::BM, j0 = (rem / g.tiles_m) * T::BN;
+        int mt, nt;
+        tile_pos(g, rem, mt, nt);
+        const int i0 = mt * T::BM, j0 = nt * T::BN;
         floatx16 sum[T::TM][T::TN];
 #pragma unroll
         for (int tm = 0; tm < T::TM; ++tm)
@@ -520,6 +542,107 @@ __global__ void __launch_bounds__(T::THREADS, (GemmDma<T, NS>::MIN_WAVES)) gemm_
     // the loads issued past the last slice (out of range: they write zeros to
     // LDS) land before the workgroup ends and its LDS is handed on
     wait_dma();
+}
+
+// ---------------------------------------------------------------------------
+// The tile engine's product on the 16-bit matrix units (split_tile.h).
+// Operand element (x, k) at base[x*ld + k] (KcSplit) or base[k*ld + x]
+// (XcSplit, 4 bytes per lane along x), rows of any alignment. Against the
+// fp32 matrix instruction: Gemm 4096^3 1013 -> 446 us, 2048^3 158 -> 74,
+// 1536^3 79 -> 48, 256x4096x4096 90 -> 43, 777x1001x1345 (unaligned) 36 -> 30.
+// What bounds 4096^3 (308 TFLOP/s of fp32 products, 925 of f16) is power: the
+// clock falls to 1.7 GHz on random operands, and on zeros the same launch
+// takes 297 us.
+// ---------------------------------------------------------------------------
+template <class T, int X, bool FULL>
+struct XcSplit : SplitStaged<T, X, X * 16 / T::THREADS> {
+    typedef SplitStaged<T, X, X * 16 / T::THREADS> S;
+    using S::koff;
+    using S::PER;
+    using S::v;
+    using S::x;
+    static constexpr bool BRANCH = false;
+    static __device__ int64_t origin(int x0, int64_t) { return x0; }
+    __amdgpu_buffer_rsrc_t r;
+    uint32_t vo, ld4;
+    __device__ __forceinline__ void init() {  // lanes along x; k uniform over a wave
+        x = threadIdx.x % X;
+        koff = __builtin_amdgcn_readfirstlane(threadIdx.x / X) * PER;
+    }
+    __device__ __forceinline__ void tile(const float* base, int64_t ld, int xlim) {
+        r = make_rsrc(base);
+        ld4 = (uint32_t)ld * 4u;
+        vo = keep_or_oob((uint32_t)x * 4u, x < xlim);
+    }
+    template <int Q>
+    __device__ __forceinline__ void load(int k0, int K, bool on) {
+        const uint32_t o = on ? vo : kOutOfRange;
+        const uint32_t s0 = (uint32_t)(k0 + koff) * ld4;
+#pragma unroll
+        for (int i = 0; i < PER; ++i)
+        {
+            const bool in = FULL || k0 + koff + i < K;  // (past K neither offset reaches the operand)
+            v[Q][i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+                r, (int)(in ? o : kOutOfRange), (int)(in ? s0 + (uint32_t)i * ld4 : 0u), 0));
+        }
+    }
+};
+
+template <class T, class OA, class OB>
+struct GemmSplit {
+    static constexpr bool LOADS_BRANCH = OA::BRANCH || OB::BRANCH;
+    const GemmArgs& g;
+    const StreamK& sk;
+    int wg, per_batch;
+    OA a;
+    OB b;
+    __device__ __forceinline__ GemmSplit(const GemmArgs& g_, const StreamK& sk_, int wg_)
+        : g(g_), sk(sk_), wg(wg_), per_batch(g_.tiles_m * g_.tiles_n) {
+        a.init();
+        b.init();
+    }
+    __device__ __forceinline__ void origin(int tile, int& batch, int& i0, int& j0) const {
+        batch = tile / per_batch;
+        const int rem = tile - batch * per_batch;
+        int mt, nt;
+        tile_pos(g, rem, mt, nt);
+        i0 = mt * T::BM;
+        j0 = nt * T::BN;
+    }
+    __device__ __forceinline__ void tile(int t) {
+        int batch, i0, j0;
+        origin(t, batch, i0, j0);
+        a.tile(g.A + batch * g.sa + OA::origin(i0, g.lda), g.lda, g.M - i0);
+        b.tile(g.B + batch * g.sb + OB::origin(j0, g.ldb), g.ldb, g.N - j0);
+    }
+    __device__ __forceinline__ void begin(int) {}
+    __device__ __forceinline__ void step() {}
+    template <int Q>
+    __device__ __forceinline__ void load_a(int it, int half, bool on) { a.template load<Q>(it * 32 + half * 16, g.K, on); }
+    template <int Q>
+    __device__ __forceinline__ void load_b(int it, int half, bool on) { b.template load<Q>(it * 32 + half * 16, g.K, on); }
+    __device__ __forceinline__ void out(const Segment& seg, const floatx16 (&sum)[T::TM][T::TN]) {
+        int batch, i0, j0;
+        origin(seg.tile, batch, i0, j0);
+        if (seg.slot < 0) {
+            // one batch of out below 2 GiB: gemm_run cuts larger ones
+            gemm_store_tile<T>(g, batch, i0, j0, sum);
+            return;
+        }
+        store_slot<T>(g.ws, wg, seg.slot, sum);
+        if (!g.cnt) return;  // gemm_fixup_k finishes the tile
+        int g0, g1, first_slot;
+        tile_partials(sk, seg.tile, g0, g1, first_slot);
+        if (finish_arrive(g.cnt + seg.tile, g1 - g0)) gemm_finish_tile<T>(g, seg.tile, g0, g1, first_slot);
+    }
+};
+
+template <class T, class OA, class OB>
+__global__ void __launch_bounds__(T::THREADS, 2) gemm_split_k(GemmArgs g, StreamK sk) {
+    extern __shared__ __align__(16) float lds[];
+    const int wg = xcd_remap(blockIdx.x, sk.G);
+    GemmSplit<T, OA, OB> p(g, sk, wg);
+    split_run<T>(p, sk, wg, reinterpret_cast<char*>(lds));
 }
 
 // out[j] partials: thread owns 4 consecutive columns (VEC) or 1.
@@ -780,6 +903,7 @@ __global__ void __launch_bounds__(64 * kSkinnyWaves) gemm_skinny_nt_k(GemmArgs g
 
 typedef Tile<128, 128, 32, 2, 2> GemmT128;
 typedef Tile<64, 64, 32, 2, 2> GemmT64;
+typedef Tile<128, 64, 32, 2, 2> GemmT12864;
 
 // Stream-K launch over batches x tiles x (K / BK) slice iterations.
 template <class T, int AK, int BKIND>
@@ -829,19 +953,14 @@ __global__ void __launch_bounds__(256) gemm_zero_counters_k(int* p, int n) {
 }
 
 // LDS stages of the direct-to-LDS kernel: 64x64 tiles have short slices
-// (16 MFMAs per wave) and keep three slices in flight; 128x128 tiles one
+// (16 MFMAs per wave) and keep three slices in flight
 template <class T>
 constexpr int dma_stages() {
-    return T::BM * T::BN < 128 * 128 ? 4 : 2;
+    return 4;
 }
 
-// Direct-to-LDS stream-K launch; OA / OB: KcOperand or XcOperand.
-// 64x64 tiles over 16 or more K slices run one workgroup per CU: whole
-// tiles then need no partials (Gemm 1024^3 on MI355X: 29.5 us against
-// 33.6 us with two workgroups per CU, each tile split in two and finished
-// in-kernel, and 33.5 us with the separate fixup kernel); over fewer slices
-// the second workgroup per CU hides the tile's load latency (1024x768x256:
-// 10.3 against 11.3 us).
+// Direct-to-LDS stream-K launch; OA / OB: KcOperand or XcOperand. At most one
+// round of 64x64 tiles over at most 8 slices (gemm_stays_fp32).
 template <class T, class OA, class OB>
 static void launch_gemm_dma(GemmArgs& g, int batches, const char* name, const char* kname) {
     constexpr int NS = dma_stages<T>();
@@ -861,8 +980,7 @@ static void launch_gemm_dma(GemmArgs& g, int batches, const char* name, const ch
     if ((int64_t)g.tiles_m * g.tiles_n * batches >= (1 << 30))
         return fail(NNC_HIP_EUNSUPP, name, "too many output tiles");
     const int iters = (int)ceil_div(g.K, T::BK);
-    const int use_slots = (T::BM * T::BN < 128 * 128 && iters >= 16) ? std::min(slots, cu_count()) : slots;
-    const StreamK sk = plan_streamk(g.tiles_m * g.tiles_n * batches, iters, use_slots, fixup_slices<T>());
+    const StreamK sk = plan_streamk(g.tiles_m * g.tiles_n * batches, iters, slots, fixup_slices<T>());
     if (sk.G < 1) return;
     const size_t ws_bytes = (size_t)sk.G * 2 * T::BM * T::BN * sizeof(float);
     g.ws = workspace(ws_bytes);
@@ -897,6 +1015,62 @@ static void dispatch_dma(GemmArgs& g, bool a_kc, bool b_kc, int batches, const c
     if (a_kc) return launch_gemm_dma_kinds<T, true, false>(g, batches, name);
     if (b_kc) return launch_gemm_dma_kinds<T, false, true>(g, batches, name);
     return launch_gemm_dma_kinds<T, false, false>(g, batches, name);
+}
+
+// Shared tiles of the split kernel with at most this many partials are
+// finished in it: a second launch costs more than the last workgroup's reads.
+static constexpr int kSplitInKernelParts = 8;
+
+template <class T, class OA, class OB>
+static void launch_gemm_split(GemmArgs& g, int batches, const StreamK& sk, const char* name, const char* kname) {
+    auto kernel = gemm_split_k<T, OA, OB>;
+    const size_t lds = (size_t)split_lds_bytes<T>();
+    // once per kernel, thread-safe (C++ static initialisation): the LDS limit
+    static const bool ready = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                  (int)lds) == hipSuccess;
+    if (!ready) return fail(NNC_HIP_EDEVICE, name, "hipFuncSetAttribute failed");
+    g.ws = nullptr;
+    g.cnt = nullptr;
+    if (sk.needs_fixup()) {
+        const size_t ws_bytes = (size_t)sk.G * 2 * T::BM * T::BN * sizeof(float);
+        g.ws = workspace(ws_bytes);
+        if (!g.ws) return partials_fail(name, ws_bytes);
+        if (split_parts(sk) <= kSplitInKernelParts) g.cnt = tile_counters((size_t)sk.sk_tiles);
+        if (g.cnt && ts().fixed)
+            launch("zero_tile_counters", gemm_zero_counters_k, dim3((unsigned)ceil_div(sk.sk_tiles, 256)), dim3(256), 0,
+                   g.cnt, (int)sk.sk_tiles);
+    }
+    set_work(2.0 * g.M * (double)g.N * g.K * batches, 0.0);
+    launch(kname, kernel, dim3(sk.G), dim3(T::THREADS), lds, g, sk);
+    if (sk.needs_fixup() && !g.cnt) {
+        set_work(0.0, 0.0);
+        launch("gemm_streamk_fixup", gemm_fixup_k<T>, dim3(T::BM * T::BN / 1024, sk.sk_tiles), dim3(256), 0, g, sk);
+    }
+}
+
+template <class T, bool A_KC, bool B_KC, bool FULL>
+static void launch_gemm_split_kinds(GemmArgs& g, int batches, const StreamK& sk, const char* name) {
+    typedef typename std::conditional<A_KC, KcSplit<T, T::BM, FULL>, XcSplit<T, T::BM, FULL>>::type OA;
+    typedef typename std::conditional<B_KC, KcSplit<T, T::BN, FULL>, XcSplit<T, T::BN, FULL>>::type OB;
+    char kname[64];
+    snprintf(kname, sizeof kname, "gemm_split_%dx%d_%s%s", T::BM, T::BN, A_KC ? "k" : "x", B_KC ? "k" : "x");
+    launch_gemm_split<T, OA, OB>(g, batches, sk, name, kname);
+}
+
+template <class T, bool FULL>
+static void dispatch_split_full(GemmArgs& g, bool a_kc, bool b_kc, int batches, const StreamK& sk, const char* name) {
+    if (a_kc && b_kc) return launch_gemm_split_kinds<T, true, true, FULL>(g, batches, sk, name);
+    if (a_kc) return launch_gemm_split_kinds<T, true, false, FULL>(g, batches, sk, name);
+    if (b_kc) return launch_gemm_split_kinds<T, false, true, FULL>(g, batches, sk, name);
+    return launch_gemm_split_kinds<T, false, false, FULL>(g, batches, sk, name);
+}
+
+template <class T>
+static void dispatch_split(GemmArgs& g, bool a_kc, bool b_kc, int batches, const StreamK& sk, const char* name) {
+    g.tiles_m = (int)ceil_div(g.M, T::BM);
+    g.tiles_n = (int)ceil_div(g.N, T::BN);
+    if (g.K % 32 == 0) return dispatch_split_full<T, true>(g, a_kc, b_kc, batches, sk, name);
+    return dispatch_split_full<T, false>(g, a_kc, b_kc, batches, sk, name);
 }
 
 template <int AK, int BKIND>
@@ -1239,19 +1413,42 @@ static void gemm_run(const GemmProblem& p, const char* name) {
     // a multiple of 4)
     const int akind = p.a_kc ? ((a_al && p.K % 4 == 0) ? kKC4 : kKC) : ((a_al && p.M % 4 == 0) ? kXC4 : kXC);
     const int bkind = p.b_kc ? ((b_al && p.K % 4 == 0) ? kKC4 : kKC) : ((b_al && p.N % 4 == 0) ? kXC4 : kXC);
-    const bool big = (int64_t)p.M * p.N * p.batches >= (int64_t)128 * 128 * 2 * cu_count() / 4 &&
-                     p.M >= 128 && p.N >= 128;
-    // 16-byte rows on both sides: direct-to-LDS staging
-    if ((akind == kKC4 || akind == kXC4) && (bkind == kKC4 || bkind == kXC4)) {
-        if (big) return dispatch_dma<GemmT128>(g, akind == kKC4, bkind == kKC4, p.batches, name);
-        return dispatch_dma<GemmT64>(g, akind == kKC4, bkind == kKC4, p.batches, name);
+    const bool aligned = (akind == kKC4 || akind == kXC4) && (bkind == kKC4 || bkind == kXC4);
+    const int64_t tiles64 = ceil_div(p.M, 64) * ceil_div(p.N, 64) * p.batches;
+    const int64_t iters = ceil_div(p.K, 32);
+    if (gemm_stays_fp32(tiles64, iters, aligned, cu_count())) {
+        if (aligned) return dispatch_dma<GemmT64>(g, akind == kKC4, bkind == kKC4, p.batches, name);
+        switch (akind) {
+            case kKC4: return dispatch_b_small<kKC4>(g, bkind, p.batches, name);
+            case kKC: return dispatch_b_small<kKC>(g, bkind, p.batches, name);
+            case kXC4: return dispatch_b_small<kXC4>(g, bkind, p.batches, name);
+            default: return dispatch_b_small<kXC>(g, bkind, p.batches, name);
+        }
     }
-    switch (akind) {
-        case kKC4: return dispatch_b_small<kKC4>(g, bkind, p.batches, name);
-        case kKC: return dispatch_b_small<kKC>(g, bkind, p.batches, name);
-        case kXC4: return dispatch_b_small<kXC4>(g, bkind, p.batches, name);
-        default: return dispatch_b_small<kXC>(g, bkind, p.batches, name);
+    if (!g.out32) {
+        // tiles store through 32-bit offsets: row ranges of less than 2 GiB
+        const int64_t rows = (((int64_t)1 << 31) - 1) / ((int64_t)p.N * 4);
+        if (rows < 1) return fail(NNC_HIP_EUNSUPP, name, "an output row spans 2 GiB or more");
+        for (int64_t i0 = 0; i0 < p.M; i0 += rows) {
+            GemmProblem q = p;
+            q.M = (int)std::min<int64_t>(rows, p.M - i0);
+            q.A = p.A + (p.a_kc ? i0 * p.lda : i0);
+            q.out = p.out + i0 * p.N;
+            if (p.c_mode == 2) q.C = p.C + i0 * p.N;
+            gemm_run(q, name);
+        }
+        return;
     }
+    if (tiles64 >= (1 << 30)) return fail(NNC_HIP_EUNSUPP, name, "too many output tiles");
+    // 64x64 and 128x64 tiles have registers for a second-level sum, which
+    // unaligned rows (formerly summed that way) keep; see split_tile.h
+    auto plan = [&](const SplitTileCost& c) {
+        return plan_split(c, ceil_div(p.M, c.bm) * ceil_div(p.N, c.bn) * p.batches, (int)iters, cu_count(), kGemmFinish);
+    };
+    const SplitPlan small = plan(kSplit64), big = plan(aligned ? kSplit128 : kSplit128x64);
+    if (small.us <= big.us) return dispatch_split<GemmT64>(g, p.a_kc, p.b_kc, p.batches, small.sk, name);
+    if (aligned) return dispatch_split<GemmT128>(g, p.a_kc, p.b_kc, p.batches, big.sk, name);
+    return dispatch_split<GemmT12864>(g, p.a_kc, p.b_kc, p.batches, big.sk, name);
 }
 
 static bool args_ok(const char* name, Tensor* a, Tensor* b, Tensor* out) {

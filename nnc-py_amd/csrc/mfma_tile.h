@@ -506,6 +506,24 @@ __device__ __forceinline__ float load_partial(__amdgpu_buffer_rsrc_t ws, uint32_
     return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ws, (int)byte_off, 0, kDeviceScope));
 }
 
+// A workgroup's partial tile to its slot, device scope.
+template <class T>
+__device__ __forceinline__ void store_slot(float* ws, int g, int which, const floatx16 (&sum)[T::TM][T::TN]) {
+    const __amdgpu_buffer_rsrc_t rws = make_rsrc(ws);
+    const uint32_t base = slot_byte_offset<T>(g, which);
+#pragma unroll
+    for (int tn = 0; tn < T::TN; ++tn)
+#pragma unroll
+        for (int tm = 0; tm < T::TM; ++tm)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                // copy the element first: this compiler's __builtin_bit_cast of
+                // an ext-vector element reads the wrong element
+                const float x = sum[tm][tn][r];
+                store_partial(rws, base + (uint32_t)(acc_row<T>(tm, r) * T::BN + acc_col<T>(tn)) * 4u, x);
+            }
+}
+
 // Four floats of a partial, loaded with device-scope coherence.
 __device__ __forceinline__ f32x4 load_partial4(__amdgpu_buffer_rsrc_t ws, uint32_t byte_off) {
     return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(ws, (int)byte_off, 0, kDeviceScope));

@@ -168,4 +168,106 @@ inline bool plan_gemm_ws(int64_t M, int64_t N, int64_t K, int64_t batches, WsPla
 // tiles, scaled by tile area for smaller tiles (shorter slices).
 constexpr int fixup_slices_for(int bm, int bn) { return (128 * 128) / (bm * bn); }
 
+// ---------------------------------------------------------------------------
+// Tile and schedule of the split kernels (split_tile.h). A tile shape's cost
+// per 32-k slice grows with the workgroups n that share a CU; the estimate of
+// a launch is its longest workgroup's slices at that price, plus finishing
+// the tiles where they are shared (SplitFinish; in the GEMM kernel its price
+// goes with the partials' bytes: 1024^3 split over 256 workgroups 22.2 us,
+// 2048^3 over 512 86 us against 73.6 whole). Prices measured on MI355X: 128x128 from Gemm 2048^3 (256
+// whole tiles, 73.6 us) and 4096^3 (two rounds of 512, 426 us); 64x64 from
+// 1024^3, 1536^3 and 2048^3 at 1 to 4 workgroups per CU; 64x256 from
+// ResNet-18's layer 1 at batch 12 and 32; 128x64 from 2048^3. What the
+// estimate decides, both sides measured: Gemm 2048x1024x256 64x64 12.3 us,
+// 128x128 15.8; 2048^3 102 and 73.6; 2000x2000x200 21.5 and 19.1; 3x3
+// convolutions at batch 32: 128 channels 28x28 as 128x128 tiles split 46.3 us,
+// whole 55.1; 256 channels 14x14 48 and 85; 1x1 256 -> 128 28x28 26.5 and 17.2;
+// layer 1 as 64x256 tiles whole 44.6, split 62.3, as 64x64 tiles 49.8 (batch
+// 12: 32.0, and 25.1 as 64x64). kConvFinish is below what a fixup launch
+// costs (about 12 us with its partials' traffic): at 196 tiles of 18 slices
+// (64 -> 128 channels, stride 2, batch 32) split and whole are 39 and 32 us,
+// and the launch table that the cost model shares has the fixup.
+// ---------------------------------------------------------------------------
+struct SplitTileCost {
+    int bm, bn, max_per_cu;
+    double us[4];   // per slice, at 1..max_per_cu workgroups per CU
+    double shared;  // more for tiles that are shared
+};
+constexpr SplitTileCost kSplit128 = {128, 128, 2, {1.02, 1.63, 0, 0}, 0};
+constexpr SplitTileCost kSplit64x256 = {64, 256, 2, {1.25, 1.90, 0, 0}, 20};
+constexpr SplitTileCost kSplit128x64 = {128, 64, 3, {0.80, 1.14, 1.71, 0}, 0};
+constexpr SplitTileCost kSplit64 = {64, 64, 4, {0.65, 0.77, 1.10, 1.48}, 0};
+
+// What finishing shared tiles adds (microseconds): per partial of a tile, per
+// MB of partials written.
+struct SplitFinish {
+    double base, per_part, per_mb;
+};
+constexpr SplitFinish kConvFinish = {2.5, 1.0, 0.0}, kGemmFinish = {3.0, 0.0, 0.35};
+
+struct SplitPlan {
+    StreamK sk;
+    double us;
+};
+
+// parts of a shared tile at most
+inline int64_t split_parts(const StreamK& sk) {
+    const int64_t per = sk.total() / sk.G;
+    return per > 0 ? (sk.iters + per - 1) / per + 1 : sk.iters;
+}
+
+inline double split_estimate(const SplitTileCost& c, const StreamK& sk, int cus, const SplitFinish& f) {
+    auto price = [&](int64_t groups) {
+        int64_t n = (groups + cus - 1) / cus;
+        return c.us[(n < 1 ? 1 : n > c.max_per_cu ? c.max_per_cu : n) - 1];
+    };
+    const int64_t whole = sk.tiles - sk.sk_tiles;
+    const int64_t full = whole / sk.G, rem = whole % sk.G;
+    double us = (double)full * sk.iters * price(sk.G) + (rem ? sk.iters * price(rem) : 0.0);
+    if (sk.sk_tiles) us += (double)((sk.total() + sk.G - 1) / sk.G) * price(sk.G);
+    if (sk.needs_fixup())
+        us += f.base + c.shared + f.per_part * (double)split_parts(sk) +
+              f.per_mb * ((double)sk.G + sk.sk_tiles) * c.bm * c.bn * 4e-6;
+    return us;
+}
+
+// The cheapest schedule of `tiles` tiles of `iters` slices on 1 to max_per_cu
+// workgroups per CU, tiles whole or shared.
+inline SplitPlan plan_split(const SplitTileCost& c, int64_t tiles, int iters, int cus, const SplitFinish& f) {
+    SplitPlan best{};
+    best.us = 1e30;
+    for (int n = 1; n <= c.max_per_cu; ++n)
+        for (int whole = 0; whole < 2; ++whole) {
+            const StreamK sk = plan_streamk((int)tiles, iters, n * cus, whole ? 1 << 20 : 0);
+            if (sk.G < 1) continue;
+            const double us = split_estimate(c, sk, cus, f);
+            if (us < best.us) best = SplitPlan{sk, us};
+        }
+    return best;
+}
+
+// Tile shape and schedule of a tap-major convolution (K a multiple of 32).
+struct ConvSplitPlan {
+    SplitTileCost tile;
+    StreamK sk;
+};
+inline ConvSplitPlan plan_conv_split(int64_t Co, int64_t Npix, int64_t K, int cus) {
+    auto plan = [&](const SplitTileCost& c) {
+        return plan_split(c, ((Co + c.bm - 1) / c.bm) * ((Npix + c.bn - 1) / c.bn), (int)(K / 32), cus, kConvFinish);
+    };
+    const SplitTileCost& large = Co <= 64 ? kSplit64x256 : kSplit128;
+    const SplitPlan a = plan(kSplit64), b = plan(large);
+    return a.us <= b.us ? ConvSplitPlan{kSplit64, a.sk} : ConvSplitPlan{large, b.sk};
+}
+
+// Products that stay on the fp32 matrix instruction: one round of 64x64
+// tiles over a few slices. The kernel's start, not its products, is what
+// takes the time there, and cutting the operands lengthens it
+// ([64,128,64] x [64,64,128] 6.9 us, split 7.0; unaligned [30,71,71] x [71,32]
+// 7.3 and 7.7; beyond: unaligned 1001x999x333 23.9 and 13.7, aligned
+// 1024x768x1024 27.9 and 22.7).
+inline bool gemm_stays_fp32(int64_t tiles64, int64_t iters, bool aligned, int cus) {
+    return tiles64 <= cus && iters <= (aligned ? 8 : 4);
+}
+
 }  // namespace nnc

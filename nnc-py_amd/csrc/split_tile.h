@@ -1,0 +1,421 @@
+// fp32 products on the 16-bit matrix units of gfx950, shared by implicit-GEMM
+// convolution and GEMM/MatMul.
+//
+// v_mfma_f32_32x32x2_f32 runs at 157 TFLOP/s, the f16 and bf16 instructions
+// at 16 times that, with fp32 accumulators. An fp32 operand is therefore cut
+// into 16-bit pieces whose products, all exact in fp32, add up to the
+// product of the operands:
+//
+//   SplitF16  x = h + m / 2048 with h = f16(x), m = f16(2048 (x - h)): 11 + 11
+//             bits and the remainder's sign. Three products (h h, h m, m h)
+//             per MFMA step; what is left out (m m and x's tail) is below
+//             2^-23 of each product. Holds where the operand row lies in
+//             f16's range (row_ok).
+//   SplitB16  x = h + m + l in bf16, h truncated: all 24 bits over fp32's
+//             whole exponent range. Six products (h h, h m, m h, m m, l h,
+//             h l); the rest is below 2^-23 of each product.
+//
+// The h h products go to one accumulator and the smaller ones to a second,
+// added once at the end: the large sum takes one rounding per 16 k (the
+// instruction adds a step's products before it rounds) instead of one per 2,
+// and the small ones cost it none. Tiles with registers to spare (at most two
+// blocks per wave) also move it to a second level every four slices. Measured against 64 bits (U(-1,1) and
+// relu'd normal operands, K 64 to 4608): relative error 0.4-0.45 of the
+// fp32 instruction's for either split, 1.15e-6 -> 0.41e-6 for Gemm 4096^3.
+//
+// A workgroup computes with SplitF16 and keeps, per thread, the largest |x|
+// of the operand row it stages. A row whose largest value is outside
+// [2^-12, 65504] (zero rows are exact either way) makes the workgroup
+// compute that segment again with SplitB16, and its later segments straight
+// away: values of any size, infinities included, get what the fp32
+// instruction gives, at a lower rate.
+//
+// The operands are cut once per workgroup, between global memory and LDS:
+// fp32 to registers two 16-k steps ahead, pieces to LDS one step ahead of
+// the MFMAs, the cutting's VALU work interleaved with the MFMAs
+// (split_order). Cutting them after the LDS read instead repeats it for each
+// wave that shares a row: 249 against 341 TFLOP/s for bf16 pieces in an
+// issue-rate probe (two waves per SIMD).
+#pragma once
+
+#include "mfma_tile.h"
+
+namespace nnc {
+
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef uint32_t u32v2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32v4 __attribute__((ext_vector_type(4)));
+
+struct SplitF16 {
+    static constexpr int PLANES = 2, PRODUCTS = 3;
+    static constexpr int OPS = 6;  // VALU operations per pair (with the row maximum)
+    typedef f16x8 Frag;
+    static __device__ __forceinline__ void cut(float x0, float x1, uint32_t (&p)[PLANES]) {
+        const f16x2 h = __builtin_convertvector(f32x2{x0, x1}, f16x2);
+        const _Float16 m0 = (_Float16)__builtin_fmaf((float)h[0], -2048.f, x0 * 2048.f);
+        const _Float16 m1 = (_Float16)__builtin_fmaf((float)h[1], -2048.f, x1 * 2048.f);
+        p[0] = __builtin_bit_cast(uint32_t, h);
+        p[1] = __builtin_bit_cast(uint32_t, f16x2{m0, m1});
+    }
+    static __device__ __forceinline__ floatx16 mma(Frag a, Frag b, floatx16 c) {
+        return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+    }
+    static __device__ __forceinline__ float sum(float hi, float lo) { return __builtin_fmaf(lo, 0x1p-11f, hi); }
+};
+
+struct SplitB16 {
+    static constexpr int PLANES = 3, PRODUCTS = 6;
+    static constexpr int OPS = 11;
+    typedef bf16x8 Frag;
+    static __device__ __forceinline__ uint32_t pack(float a, float b) {
+        return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2));
+    }
+    // h truncated: the largest floats stay finite (rounded, -FLT_MAX would be
+    // -inf); h + m + l == x for |x| >= 2^-109
+    static __device__ __forceinline__ void cut(float x0, float x1, uint32_t (&p)[PLANES]) {
+        const uint32_t a0 = __float_as_uint(x0) & 0xffff0000u, a1 = __float_as_uint(x1) & 0xffff0000u;
+        p[0] = __builtin_amdgcn_perm(a1, a0, 0x07060302u);
+        const float r0 = x0 - __uint_as_float(a0), r1 = x1 - __uint_as_float(a1);
+        p[1] = pack(r0, r1);
+        p[2] = pack(r0 - __uint_as_float(p[1] << 16), r1 - __uint_as_float(p[1] & 0xffff0000u));
+    }
+    static __device__ __forceinline__ floatx16 mma(Frag a, Frag b, floatx16 c) {
+        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+    }
+    // An infinite operand has h = x and NaN for m and l: hi is then what the
+    // fp32 products add up to (inf or NaN) and lo says nothing.
+    static __device__ __forceinline__ float sum(float hi, float lo) {
+        return __builtin_fabsf(hi) < __builtin_inff() ? hi + lo : hi;
+    }
+};
+
+// LDS image of one operand's 16-k step: plane p, k-half q (8 k each), row x
+// at p * PLANE + q * HALF + 16 x bytes: an MFMA lane's 8 k are one 16-byte
+// read, 32 lanes read 512 contiguous bytes. Halves are 64 bytes off a
+// multiple of 128 so that a store's eight lanes on four rows and both halves
+// hit all 32 banks.
+template <class Md, int X>
+struct SplitOperand {
+    static constexpr int HALF = X * 16 + 64, PLANE = 2 * HALF, BYTES = Md::PLANES * PLANE;
+};
+
+template <class Md, class T>
+struct SplitStage {
+    typedef SplitOperand<Md, T::BM> A;
+    typedef SplitOperand<Md, T::BN> B;
+    static constexpr int STAGE = A::BYTES + B::BYTES;  // bytes; two stages
+};
+
+template <class T>
+constexpr int split_lds_bytes() {
+    return 2 * SplitStage<SplitB16, T>::STAGE;
+}
+
+// One operand's staging registers: per thread and 16-k step, RUN consecutive
+// k of each of NG rows (x, x + X / NG, ...); two steps (sets Q) in flight.
+// The thread stages the same rows throughout a tile.
+template <class T, int X, int RUN_>
+struct SplitStaged {
+    static constexpr int PER = X * 16 / T::THREADS, RUN = RUN_, NG = PER / RUN;
+    static_assert(NG >= 1 && NG * RUN == PER && (RUN == 4 || RUN == 8 || RUN == 16), "k per thread");
+    int x, koff;
+    float v[2][PER];
+    // Per row the largest |x| staged since the last segment's end, and the
+    // same without the newest first half, which may belong to the next
+    // segment.
+    float mx[NG], mx_seg[NG];
+
+    __device__ __forceinline__ void reset_max() {
+#pragma unroll
+        for (int g = 0; g < NG; ++g) mx[g] = mx_seg[g] = 0.f;
+    }
+    // cuts set Q and stores it to the operand's image at S
+    template <class Md, int Q>
+    __device__ __forceinline__ void store(char* S) {
+        typedef SplitOperand<Md, X> O;
+#pragma unroll
+        for (int g = 0; g < NG; ++g) {
+            const float* u = v[Q] + g * RUN;
+            if (Md::PLANES == 2) {
+                if (Q == 0) mx_seg[g] = mx[g];
+#pragma unroll
+                for (int i = 0; i < RUN; i += 2)
+                    mx[g] = fmaxf(fmaxf(__builtin_fabsf(u[i]), __builtin_fabsf(u[i + 1])), mx[g]);
+                asm volatile("" : "+v"(mx[g]));  // here: sunk out of the block, it keeps copies of v alive
+            }
+            uint32_t w[RUN / 2][Md::PLANES];
+#pragma unroll
+            for (int i = 0; i < RUN / 2; ++i) Md::cut(u[2 * i], u[2 * i + 1], w[i]);
+#pragma unroll
+            for (int p = 0; p < Md::PLANES; ++p) {
+                char* d = S + p * O::PLANE + (koff >> 3) * O::HALF + (x + g * (X / NG)) * 16 + (koff & 4) * 2;
+                if constexpr (RUN == 4) {
+                    *reinterpret_cast<u32v2*>(d) = u32v2{w[0][p], w[1][p]};
+                } else {
+#pragma unroll
+                    for (int q = 0; q < RUN / 8; ++q)
+                        *reinterpret_cast<u32v4*>(d + q * O::HALF) =
+                            u32v4{w[4 * q][p], w[4 * q + 1][p], w[4 * q + 2][p], w[4 * q + 3][p]};
+                }
+            }
+        }
+    }
+    // Whether SplitF16 holds the thread's rows of the segment just computed:
+    // the representation error, at most 2^-23 |x| or 2^-36, is then below
+    // 2^-23 of a row's largest value. (The largest value is checked on all
+    // that was staged, the next segment's first half included.)
+    __device__ __forceinline__ bool rows_ok() const {
+        bool ok = true;
+#pragma unroll
+        for (int g = 0; g < NG; ++g) ok = ok && (mx_seg[g] == 0.f || mx_seg[g] >= 0x1p-12f) && mx[g] <= 65504.f;
+        return ok;
+    }
+};
+
+// An operand with rows contiguous in k: element (x, k) at base[x*ld + k], rows
+// of any alignment (buffer loads need 4-byte alignment only). Four lanes
+// load a row's 64 bytes of a step, so an instruction touches 16 whole
+// 64-byte pieces; with two lanes per row and 8 k per lane it touched 32
+// half-used ones, twice the L1 accesses (522 per 128x128 step against a step
+// of 384 MFMA cycles). FULL: K is a multiple of 32; otherwise the last steps
+// load their k < K 4 bytes at a time (16 bytes over a row's end would read
+// the next row, and past the matrix in its last).
+template <class T, int X, bool FULL>
+struct KcSplit : SplitStaged<T, X, 4> {
+    typedef SplitStaged<T, X, 4> S;
+    using S::koff;
+    using S::NG;
+    using S::v;
+    using S::x;
+    static constexpr bool BRANCH = !FULL;
+    static __device__ __forceinline__ int64_t origin(int x0, int64_t ld) { return (int64_t)x0 * ld; }
+    __amdgpu_buffer_rsrc_t r;
+    uint32_t vo[NG];  // byte offsets of this thread's rows at its first k, or kOutOfRange
+    __device__ __forceinline__ void init() {
+        x = threadIdx.x / 4;
+        koff = (threadIdx.x % 4) * 4;
+    }
+    __device__ __forceinline__ void tile(const float* base, int64_t ld, int xlim) {
+        r = make_rsrc(base);
+#pragma unroll
+        for (int g = 0; g < NG; ++g) {
+            const int row = x + g * (X / NG);
+            vo[g] = keep_or_oob((uint32_t)(row * (int)ld + koff) * 4u, row < xlim);
+        }
+    }
+    template <int Q>
+    __device__ __forceinline__ void load(int k0, int K, bool on) {
+#pragma unroll
+        for (int g = 0; g < NG; ++g) {
+            const uint32_t o = on ? vo[g] : kOutOfRange;
+            if (FULL || k0 + 16 <= K) {
+                const f32x4 q = __builtin_bit_cast(
+                    f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)o, (int)((uint32_t)k0 * 4u), 0));
+                v[Q][4 * g] = q[0], v[Q][4 * g + 1] = q[1], v[Q][4 * g + 2] = q[2], v[Q][4 * g + 3] = q[3];
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    v[Q][4 * g + i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+                        r, (int)(k0 + koff + i < K ? o + 4u * i : kOutOfRange), (int)((uint32_t)k0 * 4u), 0));
+            }
+        }
+    }
+};
+
+// A wave's MFMA operands of one step, read from a stage.
+template <class Md, class T>
+struct SplitFrags {
+    typedef SplitStage<Md, T> D;
+    typename Md::Frag a[Md::PLANES][T::TM], b[Md::PLANES][T::TN];
+    __device__ __forceinline__ void read(const char* S, int wave, int lane) {
+        const int wi = (wave / T::WN) * T::WAVE_M, wj = (wave % T::WN) * T::WAVE_N;
+        const int ra = (lane >> 5) * D::A::HALF + (wi + (lane & 31)) * 16;
+        const int rb = D::A::BYTES + (lane >> 5) * D::B::HALF + (wj + (lane & 31)) * 16;
+#pragma unroll
+        for (int p = 0; p < Md::PLANES; ++p) {
+#pragma unroll
+            for (int tm = 0; tm < T::TM; ++tm)
+                a[p][tm] = *reinterpret_cast<const typename Md::Frag*>(S + ra + p * D::A::PLANE + tm * 512);
+#pragma unroll
+            for (int tn = 0; tn < T::TN; ++tn)
+                b[p][tn] = *reinterpret_cast<const typename Md::Frag*>(S + rb + p * D::B::PLANE + tn * 512);
+        }
+    }
+    template <int P, int Q>
+    __device__ __forceinline__ void product(floatx16 (&c)[T::TM][T::TN]) const {
+#pragma unroll
+        for (int tm = 0; tm < T::TM; ++tm)
+#pragma unroll
+            for (int tn = 0; tn < T::TN; ++tn) c[tm][tn] = Md::mma(a[P][tm], b[Q][tn], c[tm][tn]);
+    }
+    __device__ __forceinline__ void mma(floatx16 (&hi)[T::TM][T::TN], floatx16 (&lo)[T::TM][T::TN]) const {
+        product<0, 0>(hi);
+        product<1, 0>(lo);
+        product<0, 1>(lo);
+        if constexpr (Md::PLANES == 3) {
+            product<1, 1>(lo);
+            product<2, 0>(lo);
+            product<0, 2>(lo);
+        }
+    }
+};
+
+// Instruction order of one step's block: its LDS reads, then every MFMA
+// followed by its share of the cutting (the compiler otherwise cuts first
+// and multiplies after: 177 against 190 TFLOP/s, Gemm_nt 4096^3 with bf16
+// pieces).
+template <class Md, class T, int PER>
+__device__ __forceinline__ void split_order() {
+    constexpr int M = Md::PRODUCTS * T::TM * T::TN;
+    constexpr int V = PER * Md::OPS / 2;  // PER: k per thread of both operands
+    __builtin_amdgcn_sched_group_barrier(0x100, Md::PLANES * (T::TM + T::TN), 0);
+#pragma unroll
+    for (int q = 0; q < M; ++q) {
+        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x2, (V + M - 1) / M, 0);
+    }
+}
+
+// This wave's LDS stores done, then the workgroup barrier; loads to
+// registers stay in flight across it.
+__device__ __forceinline__ void split_barrier() {
+    __builtin_amdgcn_sched_barrier(0);
+    dma_barrier<63>();
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+// base += hi; hi = 0
+template <class T>
+__device__ __forceinline__ void split_flush(floatx16 (&hi)[T::TM][T::TN], floatx16 (&base)[T::TM][T::TN]) {
+#pragma unroll
+    for (int tm = 0; tm < T::TM; ++tm)
+#pragma unroll
+        for (int tn = 0; tn < T::TN; ++tn)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const float x = hi[tm][tn][r], y = base[tm][tn][r];
+                base[tm][tn][r] = y + x;
+                hi[tm][tn][r] = 0.f;
+            }
+}
+
+// One pass of workgroup `wg` over its segments from `seg` on (`walk` just
+// past it). The operands run ahead across segment boundaries: a load cursor
+// walks the slices (32 k, two steps) one to one and a half ahead of the
+// MFMAs, so a new tile starts with its first step in LDS and its next two in
+// registers. False: SplitF16 does not hold `seg`; nothing of it was written.
+//
+// P: the product. `a`, `b`: its staged operands (SplitStaged); tile(t): the
+// loads' tile; load_a<Q>, load_b<Q>(slice, half, on): 16 k into set Q (zeros
+// when off); advance(new_tile): the loads' slice moves on by one; begin(it):
+// ... to `it` of the tile just set; out(seg, sum): a finished segment.
+template <class Md, class T, class P>
+__device__ __forceinline__ bool split_pass(P& p, const StreamK& sk, SegmentWalker& walk, Segment& seg, char* lds) {
+    typedef SplitStage<Md, T> D;
+    constexpr int PER = decltype(p.a)::PER + decltype(p.b)::PER;
+    constexpr bool TWO_LEVEL = T::TM * T::TN <= 2;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    SegmentWalker lw = walk;  // load cursor: segment ls, slice lit
+    Segment ls = seg;
+    int lit = seg.kb;
+    bool on = true;
+    auto next_slice = [&]() {
+        if (!on) return;
+        if (++lit < ls.ke) {
+            p.step();
+        } else {
+            on = lw.next(sk, ls);
+            lit = ls.kb;
+            if (on) {
+                p.tile(ls.tile);
+                p.begin(lit);
+            }
+        }
+    };
+    p.a.reset_max();
+    p.b.reset_max();
+    p.tile(ls.tile);
+    p.begin(lit);
+    p.template load_a<0>(lit, 0, true);
+    p.template load_b<0>(lit, 0, true);
+    p.template load_a<1>(lit, 1, true);
+    p.template load_b<1>(lit, 1, true);
+    p.a.template store<Md, 0>(lds);
+    p.b.template store<Md, 0>(lds + D::A::BYTES);
+    next_slice();
+    p.template load_a<0>(lit, 0, on);
+    p.template load_b<0>(lit, 0, on);
+    split_barrier();
+    while (true) {
+        floatx16 hi[T::TM][T::TN], lo[T::TM][T::TN], base[T::TM][T::TN];
+#pragma unroll
+        for (int tm = 0; tm < T::TM; ++tm)
+#pragma unroll
+            for (int tn = 0; tn < T::TN; ++tn)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) hi[tm][tn][r] = lo[tm][tn][r] = base[tm][tn][r] = 0.f;
+        for (int it = seg.kb; it < seg.ke; ++it) {
+            if (TWO_LEVEL && ((it - seg.kb) & 3) == 3) split_flush<T>(hi, base);
+            SplitFrags<Md, T> f;
+            // first half out of stage 0; the second half's pieces to stage 1
+            f.read(lds, wave, lane);
+            p.a.template store<Md, 1>(lds + D::STAGE);
+            if (!P::LOADS_BRANCH) p.template load_a<1>(lit, 1, on);
+            p.b.template store<Md, 1>(lds + D::STAGE + D::A::BYTES);
+            if (!P::LOADS_BRANCH) p.template load_b<1>(lit, 1, on);
+            f.mma(hi, lo);
+            split_order<Md, T, PER>();
+            if (P::LOADS_BRANCH) {
+                p.template load_a<1>(lit, 1, on);
+                p.template load_b<1>(lit, 1, on);
+            }
+            split_barrier();
+            // second half out of stage 1; the next slice's first to stage 0
+            next_slice();
+            f.read(lds + D::STAGE, wave, lane);
+            p.a.template store<Md, 0>(lds);
+            if (!P::LOADS_BRANCH) p.template load_a<0>(lit, 0, on);
+            p.b.template store<Md, 0>(lds + D::A::BYTES);
+            if (!P::LOADS_BRANCH) p.template load_b<0>(lit, 0, on);
+            f.mma(hi, lo);
+            split_order<Md, T, PER>();
+            if (P::LOADS_BRANCH) {
+                p.template load_a<0>(lit, 0, on);
+                p.template load_b<0>(lit, 0, on);
+            }
+            split_barrier();
+        }
+        if (TWO_LEVEL) split_flush<T>(hi, base);
+        if (Md::PLANES == 2) {
+            if (__builtin_amdgcn_readfirstlane(__syncthreads_or(!(p.a.rows_ok() && p.b.rows_ok())))) return false;
+            p.a.reset_max();
+            p.b.reset_max();
+        }
+#pragma unroll
+        for (int tm = 0; tm < T::TM; ++tm)
+#pragma unroll
+            for (int tn = 0; tn < T::TN; ++tn)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const float x = TWO_LEVEL ? base[tm][tn][r] : hi[tm][tn][r], y = lo[tm][tn][r];
+                    hi[tm][tn][r] = Md::sum(x, y);
+                }
+        p.out(seg, hi);
+        if (!walk.next(sk, seg)) return true;
+    }
+}
+
+template <class T, class P>
+__device__ __forceinline__ void split_run(P& p, const StreamK& sk, int wg, char* lds) {
+    SegmentWalker walk(sk, wg);
+    Segment seg;
+    if (!walk.next(sk, seg)) return;
+    if (!split_pass<SplitF16, T>(p, sk, walk, seg, lds)) split_pass<SplitB16, T>(p, sk, walk, seg, lds);
+}
+
+}  // namespace nnc
