@@ -320,8 +320,11 @@ __device__ void conv_finish_tile(const ConvArgs& a, int t, int g0, int g1, int f
 // interleaved with stores made the compiler wait for each element's load -
 // and, counting in order, for every earlier store). Out-of-range rows and
 // pixels get an out-of-range buffer offset: loads read 0, stores are
-// dropped. Needs output (and residual) below 2 GiB.
-template <class T>
+// dropped. Needs output (and residual) below 2 GiB. RES: whether there is a
+// residual, or -1 to ask (the split kernels, which have one copy of their
+// epilogue; in the others the selects cost more than a second copy: 1x1
+// 72 -> 108 channels, 32x30, batch 28: 19.4 us, as two copies 14.2).
+template <class T, int RES = -1>
 __device__ __forceinline__ void store_tile(const ConvArgs& a, int i0, int j0, const floatx16 (&sum)[T::TM][T::TN]) {
     const int hw = a.Ho * a.Wo;
     const __amdgpu_buffer_rsrc_t rb = make_rsrc(a.bias), rr = make_rsrc(a.res), ro = make_rsrc(a.out);
@@ -334,7 +337,7 @@ __device__ __forceinline__ void store_tile(const ConvArgs& a, int i0, int j0, co
     }
     const int co0 = i0 + acc_row<T>(0, 0);  // this lane's first row; row (tm, r) adds a wave-uniform step
     const int act = a.act;
-    const bool has_res = a.res != nullptr;
+    const bool has_res = RES < 0 ? a.res != nullptr : RES != 0;
 #pragma unroll
     for (int tm = 0; tm < T::TM; ++tm) {
         float bv[16];
@@ -354,21 +357,23 @@ __device__ __forceinline__ void store_tile(const ConvArgs& a, int i0, int j0, co
                     rv[tn][r] = load_f32(rr, ok ? (pbase[tn] + (uint32_t)(co * hw)) * 4u : kOutOfRange);
                 }
         }
-        // relu as a select per element; sigmoid (a call per element) behind
-        // one branch per block
-#pragma unroll
-        for (int tn = 0; tn < T::TN; ++tn)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                float v = sum[tm][tn][r] + bv[r];
-                v = has_res ? v + rv[tn][r] : v;
-                rv[tn][r] = act == kActRelu && !(v > 0.0f) ? 0.0f : v;
-            }
-        if (act == kActSigmoid) {
+        if constexpr (RES < 0) {
+            // relu as a select per element; sigmoid (a call per element)
+            // behind one branch per block
 #pragma unroll
             for (int tn = 0; tn < T::TN; ++tn)
 #pragma unroll
-                for (int r = 0; r < 16; ++r) rv[tn][r] = activate(rv[tn][r], kActSigmoid);
+                for (int r = 0; r < 16; ++r) {
+                    float v = sum[tm][tn][r] + bv[r];
+                    v = has_res ? v + rv[tn][r] : v;
+                    rv[tn][r] = act == kActRelu && !(v > 0.0f) ? 0.0f : v;
+                }
+            if (act == kActSigmoid) {
+#pragma unroll
+                for (int tn = 0; tn < T::TN; ++tn)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) rv[tn][r] = activate(rv[tn][r], kActSigmoid);
+            }
         }
 #pragma unroll
         for (int tn = 0; tn < T::TN; ++tn)
@@ -376,7 +381,12 @@ __device__ __forceinline__ void store_tile(const ConvArgs& a, int i0, int j0, co
             for (int r = 0; r < 16; ++r) {
                 const int co = co0 + tm * 32 + 8 * (r >> 2) + (r & 3);
                 const bool ok = pbase[tn] != kOutOfRange && co < a.Co;
-                const float v = rv[tn][r];
+                float v = rv[tn][r];
+                if constexpr (RES >= 0) {
+                    v = sum[tm][tn][r] + bv[r];
+                    if (RES) v += rv[tn][r];
+                    v = activate(v, act);
+                }
                 __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), ro,
                                                       (int)(ok ? (pbase[tn] + (uint32_t)(co * hw)) * 4u : kOutOfRange),
                                                       0, 0);
@@ -392,7 +402,10 @@ __device__ __forceinline__ void conv_segment_out(const ConvArgs& a, const Stream
                                                  int i0, int j0, const floatx16 (&sum)[T::TM][T::TN]) {
     const int hw = a.Ho * a.Wo;
     if (BATCHED && seg.slot < 0 && a.out32) {
-        store_tile<T>(a, i0, j0, sum);
+        if (a.res)
+            store_tile<T, 1>(a, i0, j0, sum);
+        else
+            store_tile<T, 0>(a, i0, j0, sum);
         return;
     }
     if (seg.slot < 0) {
@@ -882,16 +895,17 @@ __global__ void __launch_bounds__(T::THREADS, 2) conv_split_k(ConvArgs a, Stream
 // 4608): `conv_ws_k`. A workgroup owns one 32 x 32 output tile (32 channels
 // x 32 pixels) over a contiguous range of K slices, and its four waves split
 // that range among themselves - wave w takes the range's slices w, w + 4,
-// ... - each computing the whole tile into its own v_mfma_f32_32x32x2_f32
-// accumulator; the four sums are added through LDS in wave order. Operands
+// ... - each computing the whole tile (split_wave_product: f16 pieces on
+// the 16-bit instruction from two slices a wave up; ResNet-18 at batch 1
+// 190.6 -> 181.2 us); the four sums are added through LDS in wave order. Operands
 // go straight from global memory into the MFMA operand registers, with no
 // LDS staging and no barrier in the main loop: per slice (one tap and 32
 // channels of the tap-major weights, or 32 channels of the folded 1x1
 // projection) lane half h of a wave takes the slice's k = 16h .. 16h + 15,
 // so lane (row i, half h) loads A[i][16h ..] as four 16-byte loads and lane
 // (pixel j, half h) gathers B[16h + c][j] for c < 16 (one input channel
-// each, 0 outside the image), and MFMA step c multiplies those pairs. All
-// of a wave's slices (at most NS) are loaded before its first MFMA.
+// each, 0 outside the image). All of a wave's slices (at most NS) are loaded
+// before its first MFMA.
 //
 // A tile with more K than one workgroup should take is split over S <= 16
 // workgroups (contiguous slice ranges): each stores its 4 KB partial with
@@ -905,6 +919,41 @@ __global__ void __launch_bounds__(T::THREADS, 2) conv_split_k(ConvArgs a, Stream
 // One 16-byte partial, stored with device-scope coherence.
 __device__ __forceinline__ void store_partial4(__amdgpu_buffer_rsrc_t ws, uint32_t byte_off, f32x4 v) {
     __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), ws, (int)byte_off, 0, kDeviceScope);
+}
+
+// The tile of a workgroup out of its waves' sums `acc`.
+__device__ __forceinline__ void conv_ws_finish(const ConvArgs& a, int S, int t, int part, int i0, int j0,
+                                               const floatx16& acc, float (*red)[32 * 32]) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, h = lane >> 5, l32 = lane & 31;
+    // the four waves' sums in wave order; thread t then holds 4 consecutive
+    // pixels (columns 4 (t % 8) ..) of tile row t / 8
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const float x = acc[r];  // (element copied first: see store_tile)
+        red[wave][(8 * (r >> 2) + 4 * h + (r & 3)) * 32 + l32] = x;
+    }
+    __syncthreads();
+    const int row = threadIdx.x >> 3, c4 = (threadIdx.x & 7) * 4;
+    f32x4 v = *reinterpret_cast<const f32x4*>(&red[0][row * 32 + c4]);
+#pragma unroll
+    for (int w = 1; w < 4; ++w) v += *reinterpret_cast<const f32x4*>(&red[w][row * 32 + c4]);
+    const int oco = i0 + row, op0 = j0 + c4;
+    if (S > 1) {
+        const __amdgpu_buffer_rsrc_t rws = make_rsrc(a.ws);
+        const uint32_t slot = (uint32_t)t * (uint32_t)S * 4096u + threadIdx.x * 16u;
+        store_partial4(rws, slot + (uint32_t)part * 4096u, v);
+        if (!finish_arrive(a.cnt + t, S - 1)) return;  // uniform
+        f32x4 p[kWsMaxSplit];
+#pragma unroll
+        for (int q = 0; q < kWsMaxSplit; ++q)
+            p[q] = load_partial4(rws, q < S && q != part ? slot + (uint32_t)q * 4096u : kOutOfRange);
+        f32x4 sum = part == 0 ? v : p[0];
+#pragma unroll
+        for (int q = 1; q < kWsMaxSplit; ++q)
+            if (q < S) sum += q == part ? v : p[q];
+        v = sum;
+    }
+    if (oco < a.Co && op0 < a.Npix) fixup_store(a, oco, op0, make_float4(v.x, v.y, v.z, v.w));
 }
 
 template <int NS, bool PROJ>
@@ -946,15 +995,16 @@ __global__ void __launch_bounds__(256, 2) conv_ws_k(ConvArgs a, int S, int iters
         xvo = n * a.pci * pHW + oh * a.psh * a.pW + ow * a.psw + 16 * h * pHW;
     }
 
-    f32x4 av[NS][4];
-    float bv[NS][16];
+    float av[NS][16], bv[NS][16];
 #pragma unroll
     for (int q = 0; q < NS; ++q) {
         const int sl = kb + wave + 4 * q;  // wave-uniform
         const bool on = sl < ke;
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
-            av[q][u] = load_f32x4(rw, on ? arow + (uint32_t)sl * 128u + 16u * u : kOutOfRange);
+        for (int u = 0; u < 4; ++u) {
+            const f32x4 v = load_f32x4(rw, on ? arow + (uint32_t)sl * 128u + 16u * u : kOutOfRange);
+            av[q][4 * u] = v[0], av[q][4 * u + 1] = v[1], av[q][4 * u + 2] = v[2], av[q][4 * u + 3] = v[3];
+        }
         const int tap = sl / CB, cb = sl - tap * CB;
         const int r = tap / a.kw, cc = tap - r * a.kw;
         bool in = on && ((mask >> (tap & 31)) & 1u);
@@ -976,46 +1026,80 @@ __global__ void __launch_bounds__(256, 2) conv_ws_k(ConvArgs a, int S, int iters
     }
     // every load above is issued before the first MFMA below
     __builtin_amdgcn_sched_barrier(0);
-    floatx16 acc;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
     // a wave with fewer slices multiplies zeros in its last one (straight-line
     // code: a branch around it made the compiler sink that slice's loads
     // into it, one round trip per load); its workgroup waits for the waves
     // with NS slices anyway
-#pragma unroll
-    for (int q = 0; q < NS; ++q)
-#pragma unroll
-        for (int c = 0; c < 16; ++c) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av[q][c >> 2][c & 3], bv[q][c], acc, 0, 0, 0);
-    // the four waves' sums in wave order; thread t then holds 4 consecutive
-    // pixels (columns 4 (t % 8) ..) of tile row t / 8
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const float x = acc[r];  // (element copied first: see store_tile)
-        red[wave][(8 * (r >> 2) + 4 * h + (r & 3)) * 32 + l32] = x;
+    const floatx16 acc = split_wave_product<NS>(av, bv);
+    conv_ws_finish(a, S, t, part, i0, j0, acc, red);
+}
+
+// The same for weights as stored ([Co][Ci][kh][kw], any kernel size, any
+// channel counts): `conv_wss_k`. k = ci * taps + tap has no order that a
+// gather could step through in wide strides, so the workgroup first writes
+// where its k's lie to LDS (byte offset from the pixel's tap (0, 0) of
+// channel 0, and the tap), and a lane reads its 16 k's entries of a slice
+// back as broadcasts. AVEC: K % 4 == 0.
+// Few output pixels and a long contraction are latency-bound in the tile
+// kernel (64 x 64 stream-K tiles staged through LDS, then a fixup launch):
+// 39 -> 239 channels 3x3 on 10x8, batch 5, 12.9 -> 8.7 us; 23 -> 370 3x3
+// stride 2 on 9x12, batch 2, 12.6 -> 6.0; LeNet-5 at batch 3 36.6 -> 29.7.
+template <int NS, bool AVEC>
+__global__ void __launch_bounds__(256, 2) conv_wss_k(ConvArgs a, int S, int iters) {
+    __shared__ __align__(16) float red[4][32 * 32];
+    __shared__ __align__(16) int2 where[4 * NS * 32];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int t = blockIdx.x / S, part = blockIdx.x - t * S;
+    const int mt = t % a.tiles_m, nt = t / a.tiles_m;
+    const int i0 = mt * 32, j0 = nt * 32;
+    const int kb = (int)((int64_t)part * iters / S), ke = (int)((int64_t)(part + 1) * iters / S);
+    const int h = lane >> 5, l32 = lane & 31;
+    const int HW = a.H * a.W, taps = a.kh * a.kw;
+    // past K (and past the range): tap 63, which no pixel's mask holds
+    for (int e = threadIdx.x; e < 4 * NS * 32; e += 256) {
+        const int k = kb * 32 + e;
+        const int ci = k / taps, tap = k - ci * taps, r = tap / a.kw;
+        const bool on = k < a.K && k < ke * 32;
+        where[e] = make_int2(on ? (ci * HW + r * a.W + (tap - r * a.kw)) * 4 : 0, on ? tap : 63);
     }
-    __syncthreads();
-    const int row = threadIdx.x >> 3, c4 = (threadIdx.x & 7) * 4;
-    f32x4 v = *reinterpret_cast<const f32x4*>(&red[0][row * 32 + c4]);
+    const int px = j0 + l32;
+    const bool valid = px < a.Npix;
+    const int hw = a.Ho * a.Wo;
+    const int pq = valid ? px : 0;
+    const int n = pq / hw, rem = pq - n * hw;
+    const int oh = rem / a.Wo, ow = rem - oh * a.Wo;
+    const int h0 = oh * a.sh - a.ph, w0 = ow * a.sw - a.pw;
+    uint64_t mask = 0;
+    for (int r = 0; r < a.kh; ++r)
+        for (int c = 0; c < a.kw; ++c) {
+            const bool in = valid && (unsigned)(h0 + r) < (unsigned)a.H && (unsigned)(w0 + c) < (unsigned)a.W;
+            mask |= (uint64_t)in << (r * a.kw + c);
+        }
+    const uint32_t bpo = (uint32_t)(n * a.Ci * HW + h0 * a.W + w0) * 4u;  // tap (0, 0), channel 0
+    __syncthreads();  // (waits for loads too: none is under way)
+    const __amdgpu_buffer_rsrc_t rw = make_rsrc(a.w), rin = make_rsrc(a.in);
+    const int co = i0 + l32;
+    float av[NS][16], bv[NS][16];
 #pragma unroll
-    for (int w = 1; w < 4; ++w) v += *reinterpret_cast<const f32x4*>(&red[w][row * 32 + c4]);
-    const int oco = i0 + row, op0 = j0 + c4;
-    if (S > 1) {
-        const __amdgpu_buffer_rsrc_t rws = make_rsrc(a.ws);
-        const uint32_t slot = (uint32_t)t * (uint32_t)S * 4096u + threadIdx.x * 16u;
-        store_partial4(rws, slot + (uint32_t)part * 4096u, v);
-        if (!finish_arrive(a.cnt + t, S - 1)) return;  // uniform
-        f32x4 p[kWsMaxSplit];
-#pragma unroll
-        for (int q = 0; q < kWsMaxSplit; ++q)
-            p[q] = load_partial4(rws, q < S && q != part ? slot + (uint32_t)q * 4096u : kOutOfRange);
-        f32x4 sum = part == 0 ? v : p[0];
-#pragma unroll
-        for (int q = 1; q < kWsMaxSplit; ++q)
-            if (q < S) sum += q == part ? v : p[q];
-        v = sum;
+    for (int q = 0; q < NS; ++q) {
+        const int sl = kb + wave + 4 * q;  // wave-uniform
+        const int k0 = sl * 32 + 16 * h;
+        const bool on = sl < ke && co < a.Co;
+        ws_row<!AVEC>(rw, (uint32_t)(co * a.ldw) * 4u, k0, a.K, on, av[q]);
     }
-    if (oco < a.Co && op0 < a.Npix) fixup_store(a, oco, op0, make_float4(v.x, v.y, v.z, v.w));
+#pragma unroll
+    for (int q = 0; q < NS; ++q) {
+        const int e = (wave + 4 * q) * 32 + 16 * h;
+#pragma unroll
+        for (int c = 0; c < 16; ++c) {
+            const int2 w = where[e + c];
+            bv[q][c] = load_f32(rin, (mask >> w.y) & 1 ? bpo + (uint32_t)w.x : kOutOfRange);
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    const floatx16 acc = split_wave_product<NS>(av, bv);
+    conv_ws_finish(a, S, t, part, i0, j0, acc, red);
 }
 
 // ---------------------------------------------------------------------------
@@ -1491,9 +1575,14 @@ static void conv_split(ConvArgs& a, const char* entry) {
     launch_conv_split<ConvT128, KH, KW, PROJ>(a, p.sk, entry);
 }
 
-template <int NS, bool PROJ>
+enum WsKind { kWsTaps, kWsProj, kWsStored, kWsStoredVec };
+
+template <int NS, int KIND>
 static void launch_ws_ns(const ConvArgs& a, int S, int iters, unsigned grid, const char* name) {
-    launch(name, conv_ws_k<NS, PROJ>, dim3(grid), dim3(256), 0, a, S, iters);
+    if constexpr (KIND == kWsTaps || KIND == kWsProj)
+        launch(name, conv_ws_k<NS, KIND == kWsProj>, dim3(grid), dim3(256), 0, a, S, iters);
+    else
+        launch(name, conv_wss_k<NS, KIND == kWsStoredVec>, dim3(grid), dim3(256), 0, a, S, iters);
 }
 
 // conv_ws_k where plan_ws (plan.h) takes the convolution. Needs tap-major
@@ -1502,10 +1591,10 @@ static void launch_ws_ns(const ConvArgs& a, int S, int iters, unsigned grid, con
 // at most 32 taps: checked by the callers. Returns false (nothing launched)
 // where plan_ws declines or the split's scratch cannot be had (capture
 // before growth); the caller then takes its usual path.
-template <bool PROJ>
+template <int KIND>
 static bool launch_conv_ws(ConvArgs& a, const char* entry) {
     WsPlan wp;
-    if (!plan_ws(a.Co, a.Npix, a.K, wp)) return false;
+    if (!(KIND >= kWsStored ? plan_ws_stored(a.Co, a.Npix, a.K, wp) : plan_ws(a.Co, a.Npix, a.K, wp))) return false;
     const int64_t tiles = wp.tiles;
     const int iters = wp.iters, S = wp.S, NS = wp.NS;
     a.tiles_m = (int)ceil_div(a.Co, 32);
@@ -1521,16 +1610,19 @@ static bool launch_conv_ws(ConvArgs& a, const char* entry) {
                    (int)tiles);
     }
     char name[64];
-    snprintf(name, sizeof name, "conv_ws_32x32_k%dx%d%s", a.kh, a.kw, PROJ ? "p" : "");
+    if (KIND >= kWsStored)
+        snprintf(name, sizeof name, "conv_igemm_32x32_k%dx%d", a.kh, a.kw);
+    else
+        snprintf(name, sizeof name, "conv_ws_32x32_k%dx%d%s", a.kh, a.kw, KIND == kWsProj ? "p" : "");
     set_work(2.0 * a.Co * (double)a.Npix * a.K, 0.0);
     const unsigned grid = (unsigned)(tiles * S);
     switch (NS) {
-        case 1: launch_ws_ns<1, PROJ>(a, S, iters, grid, name); break;
-        case 2: launch_ws_ns<2, PROJ>(a, S, iters, grid, name); break;
-        case 3: launch_ws_ns<3, PROJ>(a, S, iters, grid, name); break;
-        case 4: launch_ws_ns<4, PROJ>(a, S, iters, grid, name); break;
-        case 5: launch_ws_ns<5, PROJ>(a, S, iters, grid, name); break;
-        default: launch_ws_ns<6, PROJ>(a, S, iters, grid, name); break;
+        case 1: launch_ws_ns<1, KIND>(a, S, iters, grid, name); break;
+        case 2: launch_ws_ns<2, KIND>(a, S, iters, grid, name); break;
+        case 3: launch_ws_ns<3, KIND>(a, S, iters, grid, name); break;
+        case 4: launch_ws_ns<4, KIND>(a, S, iters, grid, name); break;
+        case 5: launch_ws_ns<5, KIND>(a, S, iters, grid, name); break;
+        default: launch_ws_ns<6, KIND>(a, S, iters, grid, name); break;
     }
     (void)entry;
     return true;
@@ -1913,8 +2005,12 @@ static void launch_conv_stem(ConvArgs& a, const char* entry) {
 // 1x1 or 3x3, weights 16-byte aligned; checked by the caller.
 template <class T>
 static void launch_conv(ConvArgs& a, bool avec, bool dma, const char* entry) {
-    if (dma && launch_conv_ws<false>(a, entry)) return;
+    if (dma && launch_conv_ws<kWsTaps>(a, entry)) return;
     if (dma) return a.kh == 3 ? conv_split<3, 3, false>(a, entry) : conv_split<1, 1, false>(a, entry);
+    // short ones: 32 x 32 tiles (the tap mask holds 63 taps)
+    if (a.K > 0 && a.kh * a.kw < 64 &&
+        (a.K % 4 == 0 ? launch_conv_ws<kWsStoredVec>(a, entry) : launch_conv_ws<kWsStored>(a, entry)))
+        return;
     a.tiles_m = (int)ceil_div(a.Co, T::BM);
     a.tiles_n = (int)ceil_div(a.Npix, T::BN);
 #define NNC_CONV_KS(KH, KW)                                                 \
@@ -2227,7 +2323,7 @@ static void conv_proj_run(Tensor* in, Tensor* w, Tensor* b, Tensor* x, Tensor* o
     a.vec_out = aligned16(a.out);
     a.out32 = (int64_t)a.N * a.Co * a.Ho * a.Wo * 4 < ((int64_t)1 << 31);
     if (a.N == 0 || a.Co == 0 || a.Ho <= 0 || a.Wo <= 0) return;
-    if (launch_conv_ws<true>(a, name)) return;
+    if (launch_conv_ws<kWsProj>(a, name)) return;
     conv_split<3, 3, true>(a, name);
 }
 

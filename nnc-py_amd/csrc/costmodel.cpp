@@ -203,12 +203,14 @@ double fixup_us(const MfmaKind& k, const nnc::StreamK& sk) {
 
 // conv.hip conv_ws_k: each workgroup's waves run NS slices side by side;
 // a split tile adds the finish
-bool ws_kernel(const char* op, int kh, int kw, bool proj, int64_t Co, int64_t npix, int64_t K, double flops,
+// (`kind`: "p" with a projection, "s" conv_wss_k, else "")
+bool ws_kernel(const char* op, int kh, int kw, const char* kind, int64_t Co, int64_t npix, int64_t K, double flops,
                double bytes, double weight_bytes) {
     nnc::WsPlan p;
-    if (!nnc::plan_ws(Co, npix, K, p)) return false;
+    if (!(*kind == 's' ? nnc::plan_ws_stored(Co, npix, K, p) : nnc::plan_ws(Co, npix, K, p))) return false;
     char name[64];
-    snprintf(name, sizeof name, "conv_ws_32x32_k%dx%d%s", kh, kw, proj ? "p" : "");
+    if (*kind == 's') snprintf(name, sizeof name, "conv_igemm_32x32_k%dx%d", kh, kw);
+    else snprintf(name, sizeof name, "conv_ws_32x32_k%dx%d%s", kh, kw, kind);
     const int r = (int)ceil_div(p.tiles * p.S, kCUs);  // workgroups sharing a CU
     double us = kLaunchUs + r * p.NS * kWsSliceUs + kColdUsPerMB * weight_bytes * 1e-6;
     if (p.S > 1) us += kWsFinishUs + kWsFinishUsPerPart * p.S;
@@ -275,7 +277,7 @@ void conv(const char* op, Tensor* in, Tensor* w, Tensor* b, Tensor* res, Tensor*
         k = (Co <= 64 && npix >= 65536) ? &kStem64x128 : &kStem64;
         snprintf(name, sizeof name, "conv_igemm_%dx%d_k7x7c3_dma", k->bm, k->bn);
     } else {
-        if (dma && ws_kernel(op, kh, kw, false, Co, npix, K, flops, bytes, nbytes(w))) return;
+        if ((dma || kh * kw < 64) && ws_kernel(op, kh, kw, dma ? "" : "s", Co, npix, K, flops, bytes, nbytes(w))) return;
         const int tile = (K >= 512 && Co >= 128 && npix >= 1024) ? 2 : (K >= 512 && Co <= 64 && npix >= 4096) ? 1 : 0;
         if (dma) return split_conv(op, kh, kw, false, Co, npix, K, flops, bytes, nbytes(w));
         {
@@ -347,12 +349,12 @@ void gemm(const char* op, int M, int N, int K, int batches, bool a_kc, bool b_kc
         return;
     }
     {
-        // gemm.hip gemm_ws_k (plan_gemm_ws): k-contiguous operands need K % 4
-        // == 0 (16-byte rows), x-contiguous ones take any layout
+        // gemm.hip gemm_ws_k (plan_gemm_ws)
         nnc::WsPlan p;
-        if ((!a_kc || K % 4 == 0) && (!b_kc || K % 4 == 0) && nnc::plan_gemm_ws(M, N, K, batches, p)) {
+        if (nnc::plan_gemm_ws(M, N, K, batches, K % 4 == 0 || !(a_kc || b_kc), p)) {
             char name[48];
-            snprintf(name, sizeof name, "gemm_ws_32x32_%s%s", a_kc ? "k4" : "x1", b_kc ? "k4" : "x1");
+            const char* k = K % 4 == 0 ? "k4" : "k1";
+            snprintf(name, sizeof name, "gemm_ws_32x32_%s%s", a_kc ? k : "x1", b_kc ? k : "x1");
             const int r = (int)ceil_div(p.tiles * p.S, kCUs);  // workgroups sharing a CU
             double us = kLaunchUs + r * p.NS * kWsSliceUs + kColdUsPerMB * b_bytes * 1e-6;
             if (p.S > 1) us += kWsFinishUs + kWsFinishUsPerPart * p.S;
@@ -598,7 +600,7 @@ void nnc_hip_conv_proj(Tensor* in, Tensor* w, Tensor* b, Tensor* x, Tensor* out,
     if (N == 0 || Co == 0 || npix == 0) return;
     const double flops = 2.0 * Co * (double)npix * K;
     const double bytes = nbytes(in) + nbytes(x) + nbytes(w) + nbytes(b) + nbytes(out);
-    if (ws_kernel(op, 3, 3, true, Co, npix, K, flops, bytes, nbytes(w))) return;
+    if (ws_kernel(op, 3, 3, "p", Co, npix, K, flops, bytes, nbytes(w))) return;
     split_conv(op, 3, 3, true, Co, npix, K, flops, bytes, nbytes(w));
 }
 void nnc_hip_conv_packed(Tensor* in, Tensor* w, Tensor* b, Tensor* res, Tensor* out, int kh, int kw, int sh, int sw,

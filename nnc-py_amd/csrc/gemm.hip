@@ -1092,7 +1092,7 @@ static void dispatch_b_small(GemmArgs& g, int bkind, int batches, const char* na
 // Short GEMMs: gemm_ws_k, the GEMM form of conv.hip's conv_ws_k. A
 // workgroup owns one 32 x 32 output tile of one batch over a contiguous
 // range of K slices; its four waves split the range (wave w takes slices w,
-// w + 4, ...), each computing the whole tile with v_mfma_f32_32x32x2_f32, and
+// w + 4, ...), each computing the whole tile (split_wave_product), and
 // the four sums are added through LDS in wave order. Operands go straight
 // into the MFMA operand registers: lane half h takes k = 16h .. 16h + 15 of
 // each 32-wide slice, so a k-contiguous operand row is four 16-byte loads
@@ -1104,10 +1104,12 @@ static void dispatch_b_small(GemmArgs& g, int bkind, int batches, const char* na
 // gemm_finish.
 // ---------------------------------------------------------------------------
 typedef unsigned int gws_u32x4 __attribute__((ext_vector_type(4)));
+// an operand's loads: k-contiguous rows on 16-byte boundaries with K % 4 == 0,
+// k-contiguous rows anywhere, x-contiguous
+enum GwsLoad { kGwsK4, kGwsK1, kGwsX };
 
-template <int NS, bool A_KC, bool B_KC>
-__global__ void __launch_bounds__(256, 2) gemm_ws_k(GemmArgs g, int S, int iters, int tiles) {
-    __shared__ __align__(16) float red[4][32 * 32];
+template <int NS, GwsLoad LA, GwsLoad LB>
+__device__ __forceinline__ void gemm_ws_tile(const GemmArgs& g, int S, int iters, int tiles, float (*red)[32 * 32]) {
     const int lane = threadIdx.x & 63, h = lane >> 5, l32 = lane & 31;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int part = blockIdx.x % S, rest = blockIdx.x / S;
@@ -1148,13 +1150,8 @@ __global__ void __launch_bounds__(256, 2) gemm_ws_k(GemmArgs g, int S, int iters
         const int sl = kb + wave + 4 * q;  // wave-uniform
         const bool on = sl < ke;
         const int k0 = sl * 32 + 16 * h;
-        if constexpr (A_KC) {
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const bool ok = on && iok && k0 + 4 * u < g.K;
-                const f32x4 v = load_f32x4(ra, ok ? (uint32_t)(i * lda + k0 + 4 * u) * 4u : kOutOfRange);
-                av[q][4 * u] = v[0], av[q][4 * u + 1] = v[1], av[q][4 * u + 2] = v[2], av[q][4 * u + 3] = v[3];
-            }
+        if constexpr (LA != kGwsX) {
+            ws_row<LA == kGwsK1>(ra, (uint32_t)(i * lda) * 4u, k0, g.K, on && iok, av[q]);
         } else {
 #pragma unroll
             for (int c = 0; c < 16; ++c) {
@@ -1162,13 +1159,8 @@ __global__ void __launch_bounds__(256, 2) gemm_ws_k(GemmArgs g, int S, int iters
                 av[q][c] = load_f32(ra, ok ? (uint32_t)((k0 + c) * lda + i) * 4u : kOutOfRange);
             }
         }
-        if constexpr (B_KC) {
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const bool ok = on && jok && k0 + 4 * u < g.K;
-                const f32x4 v = load_f32x4(rb, ok ? (uint32_t)(j * ldb + k0 + 4 * u) * 4u : kOutOfRange);
-                bv[q][4 * u] = v[0], bv[q][4 * u + 1] = v[1], bv[q][4 * u + 2] = v[2], bv[q][4 * u + 3] = v[3];
-            }
+        if constexpr (LB != kGwsX) {
+            ws_row<LB == kGwsK1>(rb, (uint32_t)(j * ldb) * 4u, k0, g.K, on && jok, bv[q]);
         } else {
 #pragma unroll
             for (int c = 0; c < 16; ++c) {
@@ -1180,13 +1172,7 @@ __global__ void __launch_bounds__(256, 2) gemm_ws_k(GemmArgs g, int S, int iters
     // every load above is issued before the first MFMA (a wave with fewer
     // slices multiplies zeros in its last one: straight-line code)
     __builtin_amdgcn_sched_barrier(0);
-    floatx16 acc;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
-#pragma unroll
-    for (int q = 0; q < NS; ++q)
-#pragma unroll
-        for (int c = 0; c < 16; ++c) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av[q][c], bv[q][c], acc, 0, 0, 0);
+    const floatx16 acc = split_wave_product<NS>(av, bv);
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
         const float x = acc[r];  // (element copied first: see store_tile)
@@ -1232,18 +1218,42 @@ __global__ void __launch_bounds__(256, 2) gemm_ws_k(GemmArgs g, int S, int iters
 }
 
 template <int NS, bool A_KC, bool B_KC>
-static void launch_gws_ns(const GemmArgs& g, int S, int iters, int tiles, unsigned grid, const char* kname) {
-    launch(kname, gemm_ws_k<NS, A_KC, B_KC>, dim3(grid), dim3(256), 0, g, S, iters, tiles);
+__global__ void __launch_bounds__(256, 2) gemm_ws_k(GemmArgs g, int S, int iters, int tiles) {
+    __shared__ __align__(16) float red[4][32 * 32];
+    gemm_ws_tile<NS, A_KC ? kGwsK4 : kGwsX, B_KC ? kGwsK4 : kGwsX>(g, S, iters, tiles, red);
 }
 
-template <bool A_KC, bool B_KC>
-static void launch_gws(const GemmArgs& g, int NS, int S, int iters, int tiles, unsigned grid, const char* kname) {
-    switch (NS) {
-        case 1: return launch_gws_ns<1, A_KC, B_KC>(g, S, iters, tiles, grid, kname);
-        case 2: return launch_gws_ns<2, A_KC, B_KC>(g, S, iters, tiles, grid, kname);
-        case 3: return launch_gws_ns<3, A_KC, B_KC>(g, S, iters, tiles, grid, kname);
-        default: return launch_gws_ns<4, A_KC, B_KC>(g, S, iters, tiles, grid, kname);  // NS <= kGwsMaxSlices
+// with k-contiguous rows off 16-byte boundaries on at least one side
+template <int NS, GwsLoad LA, GwsLoad LB>
+__global__ void __launch_bounds__(256, 2) gemm_wsu_k(GemmArgs g, int S, int iters, int tiles) {
+    __shared__ __align__(16) float red[4][32 * 32];
+    gemm_ws_tile<NS, LA, LB>(g, S, iters, tiles, red);
+}
+
+template <int NS, GwsLoad LA, GwsLoad LB>
+static void launch_gws_ns(const GemmArgs& g, int S, int iters, int tiles, unsigned grid, const char* kname) {
+    if constexpr (LA == kGwsK1 || LB == kGwsK1)
+        launch(kname, gemm_wsu_k<NS, LA, LB>, dim3(grid), dim3(256), 0, g, S, iters, tiles);
+    else
+        launch(kname, gemm_ws_k<NS, LA == kGwsK4, LB == kGwsK4>, dim3(grid), dim3(256), 0, g, S, iters, tiles);
+}
+
+template <GwsLoad LA, GwsLoad LB>
+static void launch_gws(const GemmArgs& g, const WsPlan& p, int tiles, const char* kname) {
+    const unsigned grid = (unsigned)(p.tiles * p.S);
+    switch (p.NS) {
+        case 1: return launch_gws_ns<1, LA, LB>(g, p.S, p.iters, tiles, grid, kname);
+        case 2: return launch_gws_ns<2, LA, LB>(g, p.S, p.iters, tiles, grid, kname);
+        case 3: return launch_gws_ns<3, LA, LB>(g, p.S, p.iters, tiles, grid, kname);
+        default: return launch_gws_ns<4, LA, LB>(g, p.S, p.iters, tiles, grid, kname);  // NS <= kGwsMaxSlices
     }
+}
+
+template <GwsLoad LA>
+static void dispatch_gws(const GemmArgs& g, GwsLoad b, const WsPlan& p, int tiles, const char* kname) {
+    if (b == kGwsK4) return launch_gws<LA, kGwsK4>(g, p, tiles, kname);
+    if (b == kGwsK1) return launch_gws<LA, kGwsK1>(g, p, tiles, kname);
+    return launch_gws<LA, kGwsX>(g, p, tiles, kname);
 }
 
 // Describe operands as: A element (i, k) = A[i*lda + k] if a_kc else A[k*lda + i];
@@ -1361,17 +1371,19 @@ static void gemm_run(const GemmProblem& p, const char* name) {
         else launch("gemm_skinny_nt_32", gemm_skinny_nt_k<2>, grid, block, 0, g);
         return;
     }
-    // short products: gemm_ws_k, where plan_gemm_ws takes them and each
-    // operand is either k-contiguous with 16-byte rows (and K % 4 == 0) or
-    // x-contiguous, one batch of each below 2 GiB (32-bit buffer offsets)
+    // short products: gemm_ws_k, where plan_gemm_ws takes them, one batch of
+    // each operand below 2 GiB (32-bit buffer offsets). Rows off 16-byte
+    // boundaries too: against 64 x 64 tiles and their fixup launch
+    // [225,3771] x [71,3771]^T 23.1 -> 9.6 us, [7,835] x [835,103] 13.5 -> 8.1.
     {
         WsPlan wp;
-        const bool a_kc4 = p.a_kc && aligned16(p.A) && p.lda % 4 == 0 && p.sa % 4 == 0 && p.K % 4 == 0;
-        const bool b_kc4 = p.b_kc && aligned16(p.B) && p.ldb % 4 == 0 && p.sb % 4 == 0 && p.K % 4 == 0;
+        const bool a_kc4 = aligned16(p.A) && p.lda % 4 == 0 && p.sa % 4 == 0 && p.K % 4 == 0;
+        const bool b_kc4 = aligned16(p.B) && p.ldb % 4 == 0 && p.sb % 4 == 0 && p.K % 4 == 0;
+        const GwsLoad la = !p.a_kc ? kGwsX : a_kc4 ? kGwsK4 : kGwsK1, lb = !p.b_kc ? kGwsX : b_kc4 ? kGwsK4 : kGwsK1;
         const int64_t a_elems = p.a_kc ? (int64_t)p.M * p.lda : (int64_t)p.K * p.lda;
         const int64_t b_elems = p.b_kc ? (int64_t)p.N * p.ldb : (int64_t)p.K * p.ldb;
-        if ((a_kc4 || !p.a_kc) && (b_kc4 || !p.b_kc) && a_elems * 4 < ((int64_t)1 << 31) &&
-            b_elems * 4 < ((int64_t)1 << 31) && plan_gemm_ws(p.M, p.N, p.K, p.batches, wp)) {
+        if (a_elems * 4 < ((int64_t)1 << 31) &&
+            b_elems * 4 < ((int64_t)1 << 31) && plan_gemm_ws(p.M, p.N, p.K, p.batches, la != kGwsK1 && lb != kGwsK1, wp)) {
             g.tiles_m = (int)ceil_div(p.M, 32);
             g.tiles_n = (int)ceil_div(p.N, 32);
             const int tiles = g.tiles_m * g.tiles_n;
@@ -1386,13 +1398,12 @@ static void gemm_run(const GemmProblem& p, const char* name) {
             }
             if (ok) {
                 char kname[48];
-                snprintf(kname, sizeof kname, "gemm_ws_32x32_%s%s", p.a_kc ? "k4" : "x1", p.b_kc ? "k4" : "x1");
+                static const char* const kinds[] = {"k4", "k1", "x1"};
+                snprintf(kname, sizeof kname, "gemm_ws_32x32_%s%s", kinds[la], kinds[lb]);
                 set_work(2.0 * p.M * (double)p.N * p.K * p.batches, 0.0);
-                const unsigned grid = (unsigned)(wp.tiles * wp.S);
-                if (p.a_kc && p.b_kc) launch_gws<true, true>(g, wp.NS, wp.S, wp.iters, tiles, grid, kname);
-                else if (p.a_kc) launch_gws<true, false>(g, wp.NS, wp.S, wp.iters, tiles, grid, kname);
-                else if (p.b_kc) launch_gws<false, true>(g, wp.NS, wp.S, wp.iters, tiles, grid, kname);
-                else launch_gws<false, false>(g, wp.NS, wp.S, wp.iters, tiles, grid, kname);
+                if (la == kGwsK4) dispatch_gws<kGwsK4>(g, lb, wp, tiles, kname);
+                else if (la == kGwsK1) dispatch_gws<kGwsK1>(g, lb, wp, tiles, kname);
+                else dispatch_gws<kGwsX>(g, lb, wp, tiles, kname);
                 return;
             }
             g.ws = nullptr;

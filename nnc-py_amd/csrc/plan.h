@@ -116,14 +116,13 @@ struct WsPlan {
     int S, NS;
 };
 
-// false: conv_ws_k does not take this convolution (K a multiple of 32 and
-// the tap-major layout are the caller's to check)
-inline bool plan_ws(int64_t Co, int64_t Npix, int64_t K, WsPlan& p) {
-    if (K <= 0 || K % 32 != 0 || Co <= 0 || Npix <= 0) return false;
+// false: no 32 x 32 tiles for this convolution
+inline bool plan_ws_slices(int64_t Co, int64_t Npix, int64_t K, WsPlan& p) {
+    if (K <= 0 || Co <= 0 || Npix <= 0) return false;
     if (((Co + 63) / 64) * ((Npix + 63) / 64) >= kWsMaxTiles64 || 2.0 * Co * (double)Npix * K > kWsMaxFlops)
         return false;
     p.tiles = ((Co + 31) / 32) * ((Npix + 31) / 32);
-    p.iters = (int)(K / 32);
+    p.iters = (int)((K + 31) / 32);
     int S = 1;
     while (S < kWsMaxSplit && (p.iters + S - 1) / S > 4 * kWsMaxSlices) S *= 2;
     if (S > 1)
@@ -135,6 +134,14 @@ inline bool plan_ws(int64_t Co, int64_t Npix, int64_t K, WsPlan& p) {
     return true;
 }
 
+// conv_ws_k (the tap-major layout is the caller's to check)
+inline bool plan_ws(int64_t Co, int64_t Npix, int64_t K, WsPlan& p) {
+    return K % 32 == 0 && plan_ws_slices(Co, Npix, K, p);
+}
+
+// conv_wss_k
+inline bool plan_ws_stored(int64_t Co, int64_t Npix, int64_t K, WsPlan& p) { return plan_ws_slices(Co, Npix, K, p); }
+
 // Short GEMMs (gemm.hip gemm_ws_k, the GEMM form of conv_ws_k): products of
 // at most kGwsMaxFlops (a transformer encoder's projections and FFN2 at
 // batch 8, sequence 128), on 32 x 32 tiles of every batch with the same
@@ -145,10 +152,14 @@ inline bool plan_ws(int64_t Co, int64_t Npix, int64_t K, WsPlan& p) {
 // 1024x768x256 11.0 vs 11.5, 1024x256x1024 (split in two) 15.1 vs 16.1;
 // the tile kernel ahead at 1024 workgroups (1024x1024x256: 12.2-12.8 vs
 // 11.3-11.5 us) and with six slices per wave (768^3: 28.1 vs 22.4 us).
+// `rows16`: every k-contiguous row is on a 16-byte boundary. Others load up
+// to three more values per slice and stay on 64 x 64 tiles where many tiles
+// have one slice per wave ([36,183,51] x [36,51,120] 6.2 vs 7.3 here;
+// [59,3582] x [61,3582]^T 20.5 vs 8.5 here).
 constexpr double kGwsMaxFlops = 1e9;
 constexpr int kGwsMaxSlices = 4, kGwsMaxGroups = 1024;
 
-inline bool plan_gemm_ws(int64_t M, int64_t N, int64_t K, int64_t batches, WsPlan& p) {
+inline bool plan_gemm_ws(int64_t M, int64_t N, int64_t K, int64_t batches, bool rows16, WsPlan& p) {
     if (M <= 0 || N <= 0 || K <= 0 || batches <= 0) return false;
     if (2.0 * M * (double)N * K * batches > kGwsMaxFlops) return false;
     p.tiles = ((M + 31) / 32) * ((N + 31) / 32) * batches;
@@ -159,6 +170,7 @@ inline bool plan_gemm_ws(int64_t M, int64_t N, int64_t K, int64_t batches, WsPla
         while (S < kWsMaxSplit && p.tiles * 2 * S <= kWsGroups && p.iters / (2 * S) >= 8) S *= 2;
     const int per = (p.iters + S - 1) / S;
     if (per > 4 * kGwsMaxSlices || p.tiles * S >= kGwsMaxGroups) return false;
+    if (!rows16 && per <= 4 && p.tiles * S > kWsGroups) return false;
     p.S = S;
     p.NS = (per + 3) / 4;
     return true;
@@ -265,9 +277,10 @@ inline ConvSplitPlan plan_conv_split(int64_t Co, int64_t Npix, int64_t K, int cu
 // takes the time there, and cutting the operands lengthens it
 // ([64,128,64] x [64,64,128] 6.9 us, split 7.0; unaligned [30,71,71] x [71,32]
 // 7.3 and 7.7; beyond: unaligned 1001x999x333 23.9 and 13.7, aligned
-// 1024x768x1024 27.9 and 22.7).
+// 1024x768x1024 27.9 and 22.7). Over one or two slices a few rounds more do
+// ([24,247,25] x [24,25,242] 6.4 and 7.9; 1799x1057x45 8.1 and 9.2).
 inline bool gemm_stays_fp32(int64_t tiles64, int64_t iters, bool aligned, int cus) {
-    return tiles64 <= cus && iters <= (aligned ? 8 : 4);
+    return tiles64 <= cus ? iters <= (aligned ? 8 : 4) : iters <= 2 && tiles64 <= 4 * cus;
 }
 
 }  // namespace nnc
