@@ -124,14 +124,19 @@ struct SplitStaged {
     static_assert(NG >= 1 && NG * RUN == PER && (RUN == 4 || RUN == 8 || RUN == 16), "k per thread");
     int x, koff;
     float v[2][PER];
-    // Per row the largest |x| staged since the last segment's end, and the
-    // same without the newest first half, which may belong to the next
-    // segment.
-    float mx[NG], mx_seg[NG];
+    // Per row the largest |x| of the segment and of what is staged past it,
+    // the same without the newest first half, which may belong to the next
+    // segment, and that half's alone.
+    float mx[NG], mx_seg[NG], mx_half[NG];
 
     __device__ __forceinline__ void reset_max() {
 #pragma unroll
-        for (int g = 0; g < NG; ++g) mx[g] = mx_seg[g] = 0.f;
+        for (int g = 0; g < NG; ++g) mx[g] = mx_seg[g] = mx_half[g] = 0.f;
+    }
+    // to the next segment, whose first half is staged already
+    __device__ __forceinline__ void next_max() {
+#pragma unroll
+        for (int g = 0; g < NG; ++g) mx[g] = mx_half[g], mx_seg[g] = 0.f;
     }
     // cuts set Q and stores it to the operand's image at S
     template <class Md, int Q>
@@ -141,11 +146,13 @@ struct SplitStaged {
         for (int g = 0; g < NG; ++g) {
             const float* u = v[Q] + g * RUN;
             if (Md::PLANES == 2) {
-                if (Q == 0) mx_seg[g] = mx[g];
+                float m = Q == 0 ? 0.f : mx[g];
 #pragma unroll
                 for (int i = 0; i < RUN; i += 2)
-                    mx[g] = fmaxf(fmaxf(__builtin_fabsf(u[i]), __builtin_fabsf(u[i + 1])), mx[g]);
-                asm volatile("" : "+v"(mx[g]));  // here: sunk out of the block, it keeps copies of v alive
+                    m = fmaxf(fmaxf(__builtin_fabsf(u[i]), __builtin_fabsf(u[i + 1])), m);
+                asm volatile("" : "+v"(m));  // here: sunk out of the block, it keeps copies of v alive
+                if (Q == 0) mx_seg[g] = mx[g], mx_half[g] = m, m = fmaxf(m, mx[g]);
+                mx[g] = m;
             }
             uint32_t w[RUN / 2][Md::PLANES];
 #pragma unroll
@@ -393,8 +400,8 @@ __device__ __forceinline__ bool split_pass(P& p, const StreamK& sk, SegmentWalke
         if (TWO_LEVEL) split_flush<T>(hi, base);
         if (Md::PLANES == 2) {
             if (__builtin_amdgcn_readfirstlane(__syncthreads_or(!(p.a.rows_ok() && p.b.rows_ok())))) return false;
-            p.a.reset_max();
-            p.b.reset_max();
+            p.a.next_max();
+            p.b.next_max();
         }
 #pragma unroll
         for (int tm = 0; tm < T::TM; ++tm)
