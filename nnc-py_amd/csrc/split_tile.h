@@ -1,42 +1,47 @@
 // fp32 products on the 16-bit matrix units of gfx950, shared by implicit-GEMM
 // convolution and GEMM/MatMul.
 //
-// v_mfma_f32_32x32x2_f32 runs at 157 TFLOP/s, the f16 and bf16 instructions
-// at 16 times that, with fp32 accumulators. An fp32 operand is therefore cut
-// into 16-bit pieces whose products, all exact in fp32, add up to the
-// product of the operands:
+// v_mfma_f32_32x32x2_f32 runs at 157 TFLOP/s, the bf16 instructions at 16
+// times that, with fp32 accumulators. An fp32 operand is therefore cut into
+// three bf16 pieces of 8 bits each, which hold all 24 of its bits (a known
+// way to have fp32 products from 16-bit units; SplitB16):
 //
-//   SplitF16  x = h + m / 2048 with h = f16(x), m = f16(2048 (x - h)): 11 + 11
-//             bits and the remainder's sign. Three products (h h, h m, m h)
-//             per MFMA step; what is left out (m m and x's tail) is below
-//             2^-23 of each product. Holds where the operand row lies in
-//             f16's range (row_ok).
-//   SplitB16  x = h + m + l in bf16, h truncated: all 24 bits over fp32's
-//             whole exponent range. Six products (h h, h m, m h, m m, l h,
-//             h l); the rest is below 2^-23 of each product.
+//   x 2^24 = h + m + l   h = bf16(x 2^24), m = bf16(rest), l = the rest
+//
+// with |m| <= 2^-8 |h| and |l| <= 2^-17 |h| up to a rounding. Six products
+// (h h, h m, m h, m m, l h, h l), each exact in fp32, add up to the product
+// of the operands but for m l + l m + l l, at most 2^-24 of it: what the fp32
+// instruction rounds off a product. The factor 2^24 on either operand, taken
+// out of the sum at the end, keeps the smallest fp32 values' pieces among
+// normal numbers, so the pieces are the operand at any size: whatever scales
+// meet inside a row, each term has fp32's precision by itself, and products
+// with one nonzero term (selections, whole numbers of 16 bits or less) are
+// exact.
+//
+// What the factor takes away is at the other end: |x| from 2^104, sums from
+// 2^80, infinities and NaN. Each of them makes a sum of the tile infinite or
+// NaN, so a workgroup looks at its segment's finished sums (no test of the
+// operands in the loop) and, if one is not finite, computes that segment
+// again with the fp32 instruction out of the same LDS image (WholeF32), and
+// its later segments straight away. Such tiles take about the time that the
+// fp32 instruction needs, plus the segment thrown away; outputs beside the
+// large value in a tile then have the fp32 instruction's rounding.
 //
 // The h h products go to one accumulator and the smaller ones to a second,
 // added once at the end: the large sum takes one rounding per 16 k (the
 // instruction adds a step's products before it rounds) instead of one per 2,
 // and the small ones cost it none. Tiles with registers to spare (at most two
-// blocks per wave) also move it to a second level every four slices. Measured against 64 bits (U(-1,1) and
-// relu'd normal operands, K 64 to 4608): relative error 0.4-0.45 of the
-// fp32 instruction's for either split, 1.15e-6 -> 0.41e-6 for Gemm 4096^3.
-//
-// A workgroup computes with SplitF16 and keeps, per thread, the largest |x|
-// of the operand row it stages. A row whose largest value is outside
-// [2^-12, 65504] (zero rows are exact either way) makes the workgroup
-// compute that segment again with SplitB16, and its later segments straight
-// away: values of any size, infinities included, get what the fp32
-// instruction gives, at a lower rate.
+// blocks per wave) also move it to a second level every four slices.
 //
 // The operands are cut once per workgroup, between global memory and LDS:
 // fp32 to registers two 16-k steps ahead, pieces to LDS one step ahead of
 // the MFMAs, the cutting's VALU work interleaved with the MFMAs
 // (split_order). Cutting them after the LDS read instead repeats it for each
-// wave that shares a row: 249 against 341 TFLOP/s for bf16 pieces in an
-// issue-rate probe (two waves per SIMD).
+// wave that shares a row: 249 against 341 TFLOP/s in an issue-rate probe (two
+// waves per SIMD).
 #pragma once
+
+#include <type_traits>
 
 #include "mfma_tile.h"
 
@@ -69,28 +74,37 @@ struct SplitF16 {
 
 struct SplitB16 {
     static constexpr int PLANES = 3, PRODUCTS = 6;
-    static constexpr int OPS = 11;
+    static constexpr int OPS = 13;  // VALU operations per pair
+    static constexpr bool CHECKED = true;
     typedef bf16x8 Frag;
     static __device__ __forceinline__ uint32_t pack(float a, float b) {
         return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2));
     }
-    // h truncated: the largest floats stay finite (rounded, -FLT_MAX would be
-    // -inf); h + m + l == x for |x| >= 2^-109
     static __device__ __forceinline__ void cut(float x0, float x1, uint32_t (&p)[PLANES]) {
-        const uint32_t a0 = __float_as_uint(x0) & 0xffff0000u, a1 = __float_as_uint(x1) & 0xffff0000u;
-        p[0] = __builtin_amdgcn_perm(a1, a0, 0x07060302u);
-        const float r0 = x0 - __uint_as_float(a0), r1 = x1 - __uint_as_float(a1);
+        const float s0 = x0 * 0x1p24f, s1 = x1 * 0x1p24f;
+        p[0] = pack(s0, s1);
+        const float r0 = s0 - __uint_as_float(p[0] << 16), r1 = s1 - __uint_as_float(p[0] & 0xffff0000u);
         p[1] = pack(r0, r1);
         p[2] = pack(r0 - __uint_as_float(p[1] << 16), r1 - __uint_as_float(p[1] & 0xffff0000u));
     }
     static __device__ __forceinline__ floatx16 mma(Frag a, Frag b, floatx16 c) {
         return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
     }
-    // An infinite operand has h = x and NaN for m and l: hi is then what the
-    // fp32 products add up to (inf or NaN) and lo says nothing.
-    static __device__ __forceinline__ float sum(float hi, float lo) {
-        return __builtin_fabsf(hi) < __builtin_inff() ? hi + lo : hi;
+    // the sum, and whether the pieces hold it
+    static __device__ __forceinline__ float sum(float hi, float lo, bool& ok) {
+        const float s = hi + lo;
+        ok &= __builtin_fabsf(s) < __builtin_inff();
+        return s * 0x1p-48f;
     }
+};
+
+// The operands whole, for the fp32 instruction: plane p of a 16-k step's half
+// holds k 4p .. 4p + 3 of its eight.
+struct WholeF32 {
+    static constexpr int PLANES = 2, PRODUCTS = 8;
+    static constexpr bool CHECKED = false;
+    typedef f32x4 Frag;
+    static __device__ __forceinline__ float sum(float hi, float, bool&) { return hi; }
 };
 
 // LDS image of one operand's 16-k step: plane p, k-half q (8 k each), row x
@@ -124,20 +138,7 @@ struct SplitStaged {
     static_assert(NG >= 1 && NG * RUN == PER && (RUN == 4 || RUN == 8 || RUN == 16), "k per thread");
     int x, koff;
     float v[2][PER];
-    // Per row the largest |x| of the segment and of what is staged past it,
-    // the same without the newest first half, which may belong to the next
-    // segment, and that half's alone.
-    float mx[NG], mx_seg[NG], mx_half[NG];
 
-    __device__ __forceinline__ void reset_max() {
-#pragma unroll
-        for (int g = 0; g < NG; ++g) mx[g] = mx_seg[g] = mx_half[g] = 0.f;
-    }
-    // to the next segment, whose first half is staged already
-    __device__ __forceinline__ void next_max() {
-#pragma unroll
-        for (int g = 0; g < NG; ++g) mx[g] = mx_half[g], mx_seg[g] = 0.f;
-    }
     // cuts set Q and stores it to the operand's image at S
     template <class Md, int Q>
     __device__ __forceinline__ void store(char* S) {
@@ -145,41 +146,31 @@ struct SplitStaged {
 #pragma unroll
         for (int g = 0; g < NG; ++g) {
             const float* u = v[Q] + g * RUN;
-            if (Md::PLANES == 2) {
-                float m = Q == 0 ? 0.f : mx[g];
+            if constexpr (std::is_same<Md, WholeF32>::value) {
 #pragma unroll
-                for (int i = 0; i < RUN; i += 2)
-                    m = fmaxf(fmaxf(__builtin_fabsf(u[i]), __builtin_fabsf(u[i + 1])), m);
-                asm volatile("" : "+v"(m));  // here: sunk out of the block, it keeps copies of v alive
-                if (Q == 0) mx_seg[g] = mx[g], mx_half[g] = m, m = fmaxf(m, mx[g]);
-                mx[g] = m;
-            }
-            uint32_t w[RUN / 2][Md::PLANES];
+                for (int i = 0; i < RUN; i += 4) {
+                    const int k = koff + i;
+                    *reinterpret_cast<f32x4*>(S + ((k >> 2) & 1) * O::PLANE + (k >> 3) * O::HALF + (x + g * (X / NG)) * 16) =
+                        f32x4{u[i], u[i + 1], u[i + 2], u[i + 3]};
+                }
+            } else {
+                uint32_t w[RUN / 2][Md::PLANES];
 #pragma unroll
-            for (int i = 0; i < RUN / 2; ++i) Md::cut(u[2 * i], u[2 * i + 1], w[i]);
+                for (int i = 0; i < RUN / 2; ++i) Md::cut(u[2 * i], u[2 * i + 1], w[i]);
 #pragma unroll
-            for (int p = 0; p < Md::PLANES; ++p) {
-                char* d = S + p * O::PLANE + (koff >> 3) * O::HALF + (x + g * (X / NG)) * 16 + (koff & 4) * 2;
-                if constexpr (RUN == 4) {
-                    *reinterpret_cast<u32v2*>(d) = u32v2{w[0][p], w[1][p]};
-                } else {
+                for (int p = 0; p < Md::PLANES; ++p) {
+                    char* d = S + p * O::PLANE + (koff >> 3) * O::HALF + (x + g * (X / NG)) * 16 + (koff & 4) * 2;
+                    if constexpr (RUN == 4) {
+                        *reinterpret_cast<u32v2*>(d) = u32v2{w[0][p], w[1][p]};
+                    } else {
 #pragma unroll
-                    for (int q = 0; q < RUN / 8; ++q)
-                        *reinterpret_cast<u32v4*>(d + q * O::HALF) =
-                            u32v4{w[4 * q][p], w[4 * q + 1][p], w[4 * q + 2][p], w[4 * q + 3][p]};
+                        for (int q = 0; q < RUN / 8; ++q)
+                            *reinterpret_cast<u32v4*>(d + q * O::HALF) =
+                                u32v4{w[4 * q][p], w[4 * q + 1][p], w[4 * q + 2][p], w[4 * q + 3][p]};
+                    }
                 }
             }
         }
-    }
-    // Whether SplitF16 holds the thread's rows of the segment just computed:
-    // the representation error, at most 2^-23 |x| or 2^-36, is then below
-    // 2^-23 of a row's largest value. (The largest value is checked on all
-    // that was staged, the next segment's first half included.)
-    __device__ __forceinline__ bool rows_ok() const {
-        bool ok = true;
-#pragma unroll
-        for (int g = 0; g < NG; ++g) ok = ok && (mx_seg[g] == 0.f || mx_seg[g] >= 0x1p-12f) && mx[g] <= 65504.f;
-        return ok;
     }
 };
 
@@ -260,10 +251,22 @@ struct SplitFrags {
             for (int tn = 0; tn < T::TN; ++tn) c[tm][tn] = Md::mma(a[P][tm], b[Q][tn], c[tm][tn]);
     }
     __device__ __forceinline__ void mma(floatx16 (&hi)[T::TM][T::TN], floatx16 (&lo)[T::TM][T::TN]) const {
-        product<0, 0>(hi);
-        product<1, 0>(lo);
-        product<0, 1>(lo);
-        if constexpr (Md::PLANES == 3) {
+        if constexpr (std::is_same<Md, WholeF32>::value) {
+#pragma unroll
+            for (int p = 0; p < 2; ++p)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int tm = 0; tm < T::TM; ++tm)
+#pragma unroll
+                        for (int tn = 0; tn < T::TN; ++tn) {
+                            const float x = a[p][tm][e], y = b[p][tn][e];
+                            hi[tm][tn] = __builtin_amdgcn_mfma_f32_32x32x2f32(x, y, hi[tm][tn], 0, 0, 0);
+                        }
+        } else {
+            product<0, 0>(hi);
+            product<1, 0>(lo);
+            product<0, 1>(lo);
             product<1, 1>(lo);
             product<2, 0>(lo);
             product<0, 2>(lo);
@@ -277,13 +280,15 @@ struct SplitFrags {
 // pieces).
 template <class Md, class T, int PER>
 __device__ __forceinline__ void split_order() {
-    constexpr int M = Md::PRODUCTS * T::TM * T::TN;
-    constexpr int V = PER * Md::OPS / 2;  // PER: k per thread of both operands
-    __builtin_amdgcn_sched_group_barrier(0x100, Md::PLANES * (T::TM + T::TN), 0);
+    if constexpr (Md::CHECKED) {
+        constexpr int M = Md::PRODUCTS * T::TM * T::TN;
+        constexpr int V = PER * Md::OPS / 2;  // PER: k per thread of both operands
+        __builtin_amdgcn_sched_group_barrier(0x100, Md::PLANES * (T::TM + T::TN), 0);
 #pragma unroll
-    for (int q = 0; q < M; ++q) {
-        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x2, (V + M - 1) / M, 0);
+        for (int q = 0; q < M; ++q) {
+            __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x2, (V + M - 1) / M, 0);
+        }
     }
 }
 
@@ -314,7 +319,7 @@ __device__ __forceinline__ void split_flush(floatx16 (&hi)[T::TM][T::TN], floatx
 // past it). The operands run ahead across segment boundaries: a load cursor
 // walks the slices (32 k, two steps) one to one and a half ahead of the
 // MFMAs, so a new tile starts with its first step in LDS and its next two in
-// registers. False: SplitF16 does not hold `seg`; nothing of it was written.
+// registers. False: a sum of `seg` is not finite; nothing of it was written.
 //
 // P: the product. `a`, `b`: its staged operands (SplitStaged); tile(t): the
 // loads' tile; load_a<Q>, load_b<Q>(slice, half, on): 16 k into set Q (zeros
@@ -344,8 +349,6 @@ __device__ __forceinline__ bool split_pass(P& p, const StreamK& sk, SegmentWalke
             }
         }
     };
-    p.a.reset_max();
-    p.b.reset_max();
     p.tile(ls.tile);
     p.begin(lit);
     p.template load_a<0>(lit, 0, true);
@@ -398,11 +401,7 @@ __device__ __forceinline__ bool split_pass(P& p, const StreamK& sk, SegmentWalke
             split_barrier();
         }
         if (TWO_LEVEL) split_flush<T>(hi, base);
-        if (Md::PLANES == 2) {
-            if (__builtin_amdgcn_readfirstlane(__syncthreads_or(!(p.a.rows_ok() && p.b.rows_ok())))) return false;
-            p.a.next_max();
-            p.b.next_max();
-        }
+        bool ok = true;
 #pragma unroll
         for (int tm = 0; tm < T::TM; ++tm)
 #pragma unroll
@@ -410,8 +409,9 @@ __device__ __forceinline__ bool split_pass(P& p, const StreamK& sk, SegmentWalke
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
                     const float x = TWO_LEVEL ? base[tm][tn][r] : hi[tm][tn][r], y = lo[tm][tn][r];
-                    hi[tm][tn][r] = Md::sum(x, y);
+                    hi[tm][tn][r] = Md::sum(x, y, ok);
                 }
+        if (Md::CHECKED && __builtin_amdgcn_readfirstlane(__syncthreads_or(!ok))) return false;
         p.out(seg, hi);
         if (!walk.next(sk, seg)) return true;
     }
@@ -422,7 +422,7 @@ __device__ __forceinline__ void split_run(P& p, const StreamK& sk, int wg, char*
     SegmentWalker walk(sk, wg);
     Segment seg;
     if (!walk.next(sk, seg)) return;
-    if (!split_pass<SplitF16, T>(p, sk, walk, seg, lds)) split_pass<SplitB16, T>(p, sk, walk, seg, lds);
+    if (!split_pass<SplitB16, T>(p, sk, walk, seg, lds)) split_pass<WholeF32, T>(p, sk, walk, seg, lds);
 }
 
 // 16 consecutive k from k0 of a k-contiguous row at byte offset `row`, zeros

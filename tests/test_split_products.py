@@ -1,11 +1,11 @@
 """Convolutions and products on the 16-bit matrix units (csrc/split_tile.h).
 
 Sizes at the edges of tiles, 16-k steps and 32-k slices, and values outside
-the range of the two-piece split, where a workgroup computes its segment
-again with three pieces. The reference is the float64 product; each output
-may be off by the representation and accumulation error of the split, at most
-2^-21 of the sum of its terms' magnitudes (2^-23 per operand piece left out,
-one fp32 rounding per 16 terms), with K <= 4096.
+the range of the pieces, where a workgroup computes its segment again with
+the fp32 instruction. The reference is the float64 product; each output may
+be off by 2^-21 of the sum of its terms' magnitudes: 2^-24 of each term that
+the pieces leave out, one fp32 rounding per 16 terms (per 2 with the fp32
+instruction), K <= 4096, on random signs.
 """
 
 from __future__ import annotations

@@ -1,9 +1,12 @@
 """Products and convolutions over the whole range of fp32 values.
 
-Whatever a kernel does about operands outside a range, it has to do in every
-tile that a workgroup takes. Each output may be off by 2^-21 of the sum of its
-terms' magnitudes (roundings of at most 4096 terms and what 16-bit pieces
-leave out of each).
+An fp32 product rounds each term once: a small element beside a large one
+keeps its 24 bits, and a product with one nonzero term is that term. Kernels
+that cut their operands into 16-bit pieces have to do the same, whatever
+scales meet inside a row, in any tile that a workgroup takes. Each output may
+be off by 2^-21 of the sum of its terms' magnitudes (roundings of at most
+4096 terms and what the pieces leave out of each); selections and products of
+whole numbers below 2^24 are exact.
 """
 
 from __future__ import annotations
@@ -14,6 +17,9 @@ import pytest
 from test_split_products import _check, _conv, _gemm
 
 pytestmark = pytest.mark.gpu
+
+# (m, n, k, nt): 128x128, 128x64 (unaligned) and 64x64 tiles
+PRODUCTS = [(1500, 1100, 640, True), (1500, 1100, 640, False), (1999, 2001, 333, True), (700, 900, 544, False)]
 
 
 def _uniform(rng, *shape):
@@ -46,3 +52,90 @@ def test_later_pixels_of_a_workgroup(scale, hip, abi):
     x[32:, 16:] = 0
     w = rng.standard_normal((64, 1, 1, 32)).astype(np.float32)
     _check(*_conv(hip, abi, x, w, 1, 0), f"scale {scale}")
+
+
+def _mixed(rng, which, m, n, k):
+    """Elements of very different size within a row; what the large ones
+    meet is zero, so that the small ones make the result."""
+    a, b = _uniform(rng, m, k), _uniform(rng, k, n)
+    big = np.arange(k) % 4 == 0
+    a_small, b_size = {"2^-30": (2.0 ** -30, 3e4), "2^-60": (2.0 ** -60, 3e4), "2^-100": (2.0 ** -100, 2.0 ** 80),
+                       "denormal": (2.0 ** -130, 2.0 ** 90), "plain": (2.0 ** -40, 1.0)}[which]
+    a[:, ~big] *= np.float32(a_small)
+    b[big] = 0
+    b[~big] *= np.float32(b_size)
+    return a, b
+
+
+@pytest.mark.parametrize("which", ["2^-30", "2^-60", "2^-100", "denormal", "plain"])
+@pytest.mark.parametrize("m,n,k,nt", PRODUCTS)
+def test_small_beside_large(m, n, k, nt, which, hip, abi):
+    print(f"case gemm {m}x{n}x{k} nt={nt} small beside large {which}", flush=True)
+    a, b = _mixed(np.random.default_rng(m + k), which, m, n, k)
+    _check(_gemm(hip, abi, a, b, nt), a, b, which)
+
+
+def _spread(rng, shape, lo, hi):
+    """fp32 values with all 24 bits, exponents of [lo, hi]."""
+    x = rng.integers(1 << 23, 1 << 24, shape).astype(np.float32) * rng.choice([-1, 1], shape).astype(np.float32)
+    return np.ldexp(x, (rng.integers(lo, hi + 1, shape) - 23)).astype(np.float32)
+
+
+EXPONENTS = {"one": (0, 0), "f16": (-12, 15), "small": (-126, -90), "usual": (-126, 100), "all": (-126, 127)}
+
+
+@pytest.mark.parametrize("which", sorted(EXPONENTS))
+@pytest.mark.parametrize("m,n,k,nt", PRODUCTS)
+def test_selection_is_exact(m, n, k, nt, which, hip, abi):
+    """Rows of a permutation: the product's rows are the other operand's."""
+    print(f"case gemm {m}x{n}x{k} nt={nt} selection of {which}", flush=True)
+    rng = np.random.default_rng(m + k)
+    pick = rng.integers(0, k, m)
+    a = np.zeros((m, k), np.float32)
+    a[np.arange(m), pick] = 1
+    b = _spread(rng, (k, n), *EXPONENTS[which])
+    assert np.array_equal(_gemm(hip, abi, a, b, nt), b[pick])
+
+
+@pytest.mark.parametrize("m,n,k,nt", PRODUCTS)
+def test_whole_numbers_are_exact(m, n, k, nt, hip, abi):
+    """One product of two 12-bit numbers per output, sums of some others."""
+    print(f"case gemm {m}x{n}x{k} nt={nt} whole numbers", flush=True)
+    rng = np.random.default_rng(m)
+    a = np.zeros((m, k), np.float32)
+    a[np.arange(m), rng.integers(0, k, m)] = rng.integers(2048, 4096, m)
+    b = rng.integers(-4095, 4096, (k, n)).astype(np.float32)
+    assert np.array_equal(_gemm(hip, abi, a, b, nt), (a.astype(np.float64) @ b).astype(np.float32))
+    a = rng.integers(-100, 101, (m, k)).astype(np.float32) * (np.arange(k) < 300)
+    b = rng.integers(-500, 501, (k, n)).astype(np.float32)
+    assert np.array_equal(_gemm(hip, abi, a, b, nt), (a.astype(np.float64) @ b).astype(np.float32))
+
+
+# (n, ci, h, w, co, k): tiles of 128x128 and 64x256 (whole, shared)
+CONVS = [(16, 256, 28, 27, 128, 1), (32, 64, 56, 56, 64, 3), (8, 256, 14, 14, 256, 3)]
+
+
+@pytest.mark.parametrize("which", sorted(EXPONENTS))
+@pytest.mark.parametrize("shape", CONVS, ids=[str(s) for s in CONVS])
+def test_selection_by_a_convolution(shape, which, hip, abi):
+    n, ci, h, w, co, k = shape
+    print(f"case conv {shape} selection of {which}", flush=True)
+    rng = np.random.default_rng(ci + h)
+    x = _spread(rng, (n, ci, h, w), *EXPONENTS[which])
+    pick = rng.integers(0, ci, co)
+    v = np.zeros((co, k, k, ci), np.float32)
+    v[np.arange(co), k // 2, k // 2, pick] = 1
+    got, _, _ = _conv(hip, abi, x, v, 1, k // 2)
+    assert np.array_equal(got.reshape(co, n, h, w).transpose(1, 0, 2, 3), x[:, pick])
+
+
+@pytest.mark.parametrize("which", ["2^-30", "2^-60", "2^-100", "denormal", "plain"])
+@pytest.mark.parametrize("shape", CONVS, ids=[str(s) for s in CONVS])
+def test_small_beside_large_channels(shape, which, hip, abi):
+    n, ci, h, w, co, k = shape
+    print(f"case conv {shape} small beside large {which}", flush=True)
+    rng = np.random.default_rng(ci + h)
+    a, b = _mixed(rng, which, 1, 1, ci)
+    x = (_uniform(rng, n, ci, h, w) * np.abs(a.reshape(1, ci, 1, 1))).astype(np.float32)
+    v = (_uniform(rng, co, k, k, ci) * np.abs(b.reshape(ci))).astype(np.float32)
+    _check(*_conv(hip, abi, x, v, 1, k // 2), f"{shape} {which}")
