@@ -894,11 +894,10 @@ __global__ void __launch_bounds__(T::THREADS, 2) conv_split_k(ConvArgs a, Stream
 // 4608): `conv_ws_k`. A workgroup owns one 32 x 32 output tile (32 channels
 // x 32 pixels) over a contiguous range of K slices, and its four waves split
 // that range among themselves - wave w takes the range's slices w, w + 4,
-// ... - each computing the whole tile (split_wave_product: f16 pieces on
-// the 16-bit instruction from two slices a wave up; ResNet-18 at batch 1
-// 190.6 -> 181.2 us); the four sums are added through LDS in wave order. Operands
-// go straight from global memory into the MFMA operand registers, with no
-// LDS staging and no barrier in the main loop: per slice (one tap and 32
+// ... - each computing the whole tile (wave_product_as); the four sums are
+// added through LDS in wave order. Operands go straight from global memory
+// into the MFMA operand registers, with no LDS staging and no barrier in the
+// main loop: per slice (one tap and 32
 // channels of the tap-major weights, or 32 channels of the folded 1x1
 // projection) lane half h of a wave takes the slice's k = 16h .. 16h + 15,
 // so lane (row i, half h) loads A[i][16h ..] as four 16-byte loads and lane
@@ -949,13 +948,16 @@ __device__ __forceinline__ void conv_ws_finish(const ConvArgs& a, int S, int t, 
         f32x4 sum = part == 0 ? v : p[0];
 #pragma unroll
         for (int q = 1; q < kWsMaxSplit; ++q)
-            if (q < S) sum += q == part ? v : p[q];
+            if (q < S) {
+                sum += q == part ? v : p[q];
+                asm volatile("");  // stays a branch: as selects, every tile waits for and runs through all 16
+            }
         v = sum;
     }
     if (oco < a.Co && op0 < a.Npix) fixup_store(a, oco, op0, make_float4(v.x, v.y, v.z, v.w));
 }
 
-template <int NS, bool PROJ>
+template <int NS, bool PROJ, bool PIECES>
 __global__ void __launch_bounds__(256, 2) conv_ws_k(ConvArgs a, int S, int iters) {
     __shared__ __align__(16) float red[4][32 * 32];
     const int lane = threadIdx.x & 63;
@@ -1029,7 +1031,7 @@ __global__ void __launch_bounds__(256, 2) conv_ws_k(ConvArgs a, int S, int iters
     // code: a branch around it made the compiler sink that slice's loads
     // into it, one round trip per load); its workgroup waits for the waves
     // with NS slices anyway
-    const floatx16 acc = split_wave_product<NS>(av, bv);
+    const floatx16 acc = wave_product_as<NS, PIECES>(av, bv);
     conv_ws_finish(a, S, t, part, i0, j0, acc, red);
 }
 
@@ -1043,7 +1045,7 @@ __global__ void __launch_bounds__(256, 2) conv_ws_k(ConvArgs a, int S, int iters
 // kernel (64 x 64 stream-K tiles staged through LDS, then a fixup launch):
 // 39 -> 239 channels 3x3 on 10x8, batch 5, 12.9 -> 8.7 us; 23 -> 370 3x3
 // stride 2 on 9x12, batch 2, 12.6 -> 6.0; LeNet-5 at batch 3 36.6 -> 29.7.
-template <int NS, bool AVEC>
+template <int NS, bool AVEC, bool PIECES>
 __global__ void __launch_bounds__(256, 2) conv_wss_k(ConvArgs a, int S, int iters) {
     __shared__ __align__(16) float red[4][32 * 32];
     __shared__ __align__(16) int2 where[4 * NS * 32];
@@ -1097,7 +1099,7 @@ __global__ void __launch_bounds__(256, 2) conv_wss_k(ConvArgs a, int S, int iter
         }
     }
     __builtin_amdgcn_sched_barrier(0);
-    const floatx16 acc = split_wave_product<NS>(av, bv);
+    const floatx16 acc = wave_product_as<NS, PIECES>(av, bv);
     conv_ws_finish(a, S, t, part, i0, j0, acc, red);
 }
 
@@ -1576,12 +1578,19 @@ static void conv_split(ConvArgs& a, const char* entry) {
 
 enum WsKind { kWsTaps, kWsProj, kWsStored, kWsStoredVec };
 
-template <int NS, int KIND>
-static void launch_ws_ns(const ConvArgs& a, int S, int iters, unsigned grid, const char* name) {
+template <int NS, int KIND, bool PIECES>
+static void launch_ws_as(const ConvArgs& a, int S, int iters, unsigned grid, const char* name) {
     if constexpr (KIND == kWsTaps || KIND == kWsProj)
-        launch(name, conv_ws_k<NS, KIND == kWsProj>, dim3(grid), dim3(256), 0, a, S, iters);
+        launch(name, conv_ws_k<NS, KIND == kWsProj, PIECES>, dim3(grid), dim3(256), 0, a, S, iters);
     else
-        launch(name, conv_wss_k<NS, KIND == kWsStoredVec>, dim3(grid), dim3(256), 0, a, S, iters);
+        launch(name, conv_wss_k<NS, KIND == kWsStoredVec, PIECES>, dim3(grid), dim3(256), 0, a, S, iters);
+}
+
+template <int NS, int KIND>
+static void launch_ws_ns(const ConvArgs& a, const WsPlan& p, unsigned grid, const char* name) {
+    if constexpr (NS >= kWsPieceSlices)
+        if (p.pieces) return launch_ws_as<NS, KIND, true>(a, p.S, p.iters, grid, name);
+    launch_ws_as<NS, KIND, false>(a, p.S, p.iters, grid, name);
 }
 
 // conv_ws_k where plan_ws (plan.h) takes the convolution. Needs tap-major
@@ -1595,7 +1604,7 @@ static bool launch_conv_ws(ConvArgs& a, const char* entry) {
     WsPlan wp;
     if (!(KIND >= kWsStored ? plan_ws_stored(a.Co, a.Npix, a.K, wp) : plan_ws(a.Co, a.Npix, a.K, wp))) return false;
     const int64_t tiles = wp.tiles;
-    const int iters = wp.iters, S = wp.S, NS = wp.NS;
+    const int S = wp.S;
     a.tiles_m = (int)ceil_div(a.Co, 32);
     a.tiles_n = (int)ceil_div(a.Npix, 32);
     a.ws = nullptr;
@@ -1615,13 +1624,13 @@ static bool launch_conv_ws(ConvArgs& a, const char* entry) {
         snprintf(name, sizeof name, "conv_ws_32x32_k%dx%d%s", a.kh, a.kw, KIND == kWsProj ? "p" : "");
     set_work(2.0 * a.Co * (double)a.Npix * a.K, 0.0);
     const unsigned grid = (unsigned)(tiles * S);
-    switch (NS) {
-        case 1: launch_ws_ns<1, KIND>(a, S, iters, grid, name); break;
-        case 2: launch_ws_ns<2, KIND>(a, S, iters, grid, name); break;
-        case 3: launch_ws_ns<3, KIND>(a, S, iters, grid, name); break;
-        case 4: launch_ws_ns<4, KIND>(a, S, iters, grid, name); break;
-        case 5: launch_ws_ns<5, KIND>(a, S, iters, grid, name); break;
-        default: launch_ws_ns<6, KIND>(a, S, iters, grid, name); break;
+    switch (wp.NS) {
+        case 1: launch_ws_ns<1, KIND>(a, wp, grid, name); break;
+        case 2: launch_ws_ns<2, KIND>(a, wp, grid, name); break;
+        case 3: launch_ws_ns<3, KIND>(a, wp, grid, name); break;
+        case 4: launch_ws_ns<4, KIND>(a, wp, grid, name); break;
+        case 5: launch_ws_ns<5, KIND>(a, wp, grid, name); break;
+        default: launch_ws_ns<6, KIND>(a, wp, grid, name); break;
     }
     (void)entry;
     return true;

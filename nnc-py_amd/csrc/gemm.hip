@@ -1089,7 +1089,7 @@ static void dispatch_b_small(GemmArgs& g, int bkind, int batches, const char* na
 // Short GEMMs: gemm_ws_k, the GEMM form of conv.hip's conv_ws_k. A
 // workgroup owns one 32 x 32 output tile of one batch over a contiguous
 // range of K slices; its four waves split the range (wave w takes slices w,
-// w + 4, ...), each computing the whole tile (split_wave_product), and
+// w + 4, ...), each computing the whole tile (wave_product), and
 // the four sums are added through LDS in wave order. Operands go straight
 // into the MFMA operand registers: lane half h takes k = 16h .. 16h + 15 of
 // each 32-wide slice, so a k-contiguous operand row is four 16-byte loads
@@ -1150,26 +1150,28 @@ __device__ __forceinline__ void gemm_ws_tile(const GemmArgs& g, int S, int iters
         if constexpr (LA != kGwsX) {
             ws_row<LA == kGwsK1>(ra, (uint32_t)(i * lda) * 4u, k0, g.K, on && iok, av[q]);
         } else {
+            const int k_end = (on & iok) ? g.K : 0;
 #pragma unroll
             for (int c = 0; c < 16; ++c) {
-                const bool ok = on && iok && k0 + c < g.K;
-                av[q][c] = load_f32(ra, ok ? (uint32_t)((k0 + c) * lda + i) * 4u : kOutOfRange);
+                const uint32_t o = (uint32_t)((k0 + c) * lda + i) * 4u;
+                av[q][c] = load_f32(ra, k0 + c < k_end ? o : kOutOfRange);
             }
         }
         if constexpr (LB != kGwsX) {
             ws_row<LB == kGwsK1>(rb, (uint32_t)(j * ldb) * 4u, k0, g.K, on && jok, bv[q]);
         } else {
+            const int k_end = (on & jok) ? g.K : 0;
 #pragma unroll
             for (int c = 0; c < 16; ++c) {
-                const bool ok = on && jok && k0 + c < g.K;
-                bv[q][c] = load_f32(rb, ok ? (uint32_t)((k0 + c) * ldb + j) * 4u : kOutOfRange);
+                const uint32_t o = (uint32_t)((k0 + c) * ldb + j) * 4u;
+                bv[q][c] = load_f32(rb, k0 + c < k_end ? o : kOutOfRange);
             }
         }
     }
     // every load above is issued before the first MFMA (a wave with fewer
     // slices multiplies zeros in its last one: straight-line code)
     __builtin_amdgcn_sched_barrier(0);
-    const floatx16 acc = split_wave_product<NS>(av, bv);
+    const floatx16 acc = wave_product<NS>(av, bv);
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
         const float x = acc[r];  // (element copied first: see store_tile)
@@ -1192,7 +1194,10 @@ __device__ __forceinline__ void gemm_ws_tile(const GemmArgs& g, int S, int iters
         f32x4 sum = part == 0 ? v : p[0];
 #pragma unroll
         for (int q = 1; q < kWsMaxSplit; ++q)
-            if (q < S) sum += q == part ? v : p[q];
+            if (q < S) {
+                sum += q == part ? v : p[q];
+                asm volatile("");  // stays a branch: as selects, every tile runs through all 16 (see conv_ws_finish)
+            }
         v = sum;
     }
     if (oi >= g.M) return;

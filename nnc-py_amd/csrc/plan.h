@@ -103,8 +103,14 @@ inline StreamK plan_streamk(int tiles, int iters, int slots, int fixup_slices) {
 // workgroup stays whole, and a split one is split further while the grid
 // stays within kWsGroups workgroups (one per CU) and each keeps at least 8
 // slices.
+// pieces: the waves multiply bf16 pieces (split_tile.h) where workgroups share
+// CUs and have four or more slices a wave, so that the fp32 instruction, of
+// 64 cycles for 2 k, is what they share: weights as stored, 23 slices on 276
+// tiles 18.2 -> 15.0 us, 21 on 312 17.5 -> 14.2, 18 on 318 14.5 -> 14.0. A
+// workgroup alone on its CU only waits for the cutting: 18 slices on 198
+// tiles 10.4 -> 10.7, 8 on 214 5.6 -> 6.1, ResNet-18 at batch 1 191 -> 197.
 // ---------------------------------------------------------------------------
-constexpr int kWsMaxSlices = 6;
+constexpr int kWsMaxSlices = 6, kWsPieceSlices = 4;
 constexpr int kWsMaxSplit = 16;
 constexpr int kWsMaxTiles64 = 256;
 constexpr double kWsMaxFlops = 5e8;
@@ -114,6 +120,7 @@ struct WsPlan {
     int64_t tiles;  // 32 x 32 tiles
     int iters;      // slices of 32 k
     int S, NS;
+    bool pieces;
 };
 
 // false: no 32 x 32 tiles for this convolution
@@ -131,6 +138,7 @@ inline bool plan_ws_slices(int64_t Co, int64_t Npix, int64_t K, WsPlan& p) {
     if (per > 4 * kWsMaxSlices) return false;
     p.S = S;
     p.NS = (per + 3) / 4;
+    p.pieces = p.tiles * S > kWsGroups && p.NS >= kWsPieceSlices;
     return true;
 }
 
@@ -139,8 +147,15 @@ inline bool plan_ws(int64_t Co, int64_t Npix, int64_t K, WsPlan& p) {
     return K % 32 == 0 && plan_ws_slices(Co, Npix, K, p);
 }
 
-// conv_wss_k
-inline bool plan_ws_stored(int64_t Co, int64_t Npix, int64_t K, WsPlan& p) { return plan_ws_slices(Co, Npix, K, p); }
+// conv_wss_k. Each of its workgroups first writes the table of its k's, so
+// rounds of many short ones go to the 64 x 64 tiles: tiles more than 256
+// times the smaller of the slices and three (one slice on 540 tiles 5.9 us
+// here, 5.3 there; two on 630 6.9 and 6.4, on 402 5.4 and 6.2; six on 792 12.3
+// and 10.8, on 582 11.3 and 14.5).
+inline bool plan_ws_stored(int64_t Co, int64_t Npix, int64_t K, WsPlan& p) {
+    if (!plan_ws_slices(Co, Npix, K, p)) return false;
+    return p.S > 1 || (p.tiles + kWsGroups - 1) / kWsGroups <= (p.iters < 3 ? p.iters : 3);
+}
 
 // Short GEMMs (gemm.hip gemm_ws_k, the GEMM form of conv_ws_k): products of
 // at most kGwsMaxFlops (a transformer encoder's projections and FFN2 at
@@ -173,6 +188,7 @@ inline bool plan_gemm_ws(int64_t M, int64_t N, int64_t K, int64_t batches, bool 
     if (!rows16 && per <= 4 && p.tiles * S > kWsGroups) return false;
     p.S = S;
     p.NS = (per + 3) / 4;
+    p.pieces = false;
     return true;
 }
 

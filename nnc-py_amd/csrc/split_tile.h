@@ -435,14 +435,18 @@ __device__ __forceinline__ void ws_row(__amdgpu_buffer_rsrc_t r, uint32_t row, i
     const int kt = TAIL ? K & ~3 : K;
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-        const f32x4 x = load_f32x4(r, on && k0 + 4 * u < kt ? row + (uint32_t)(k0 + 4 * u) * 4u : kOutOfRange);
+        const uint32_t o = row + (uint32_t)(k0 + 4 * u) * 4u;
+        const f32x4 x = load_f32x4(r, (on & (k0 + 4 * u < kt)) ? o : kOutOfRange);
         v[4 * u] = x[0], v[4 * u + 1] = x[1], v[4 * u + 2] = x[2], v[4 * u + 3] = x[3];
     }
     if constexpr (TAIL) {
-        const bool here = on && kt >= k0 && kt < k0 + 16;
+        const bool here = on & (kt >= k0) & (kt < k0 + 16);
         float t[3];
 #pragma unroll
-        for (int e = 0; e < 3; ++e) t[e] = load_f32(r, here && kt + e < K ? row + (uint32_t)(kt + e) * 4u : kOutOfRange);
+        for (int e = 0; e < 3; ++e) {
+            const uint32_t o = row + (uint32_t)(kt + e) * 4u;
+            t[e] = load_f32(r, (here & (kt + e < K)) ? o : kOutOfRange);
+        }
 #pragma unroll
         for (int u = 0; u < 4; ++u)
 #pragma unroll
@@ -452,65 +456,64 @@ __device__ __forceinline__ void ws_row(__amdgpu_buffer_rsrc_t r, uint32_t row, i
 
 // A wave's 32 x 32 product of operands that it holds whole in registers (the
 // short convolutions and GEMMs): lane (row l % 32, half l / 32) has NS slices
-// of 16 consecutive k of its row of either operand, so one slice is two f16
-// steps of 8 k per half, six 8-pass instructions in place of sixteen 16-pass
-// ones. The split products run as the operands arrive, the rows' maxima
-// beside them (checked ahead of the first product they waited for the last
-// load: 1043x64x672 7.9 -> 8.2 us); where a row does not hold, the wave goes
-// over its registers again with the fp32 instruction. One slice stays on
-// that: 32 k are too few roundings for the pieces to be closer to 64 bits
-// (1x1 64 -> 122 channels 8.5e-8 against 1.0e-7), and no slower.
+// of 16 consecutive k of its row of either operand, one fp32 instruction per
+// k of each half.
 template <int NS>
-__device__ __forceinline__ floatx16 split_wave_product(const float (&a)[NS][16], const float (&b)[NS][16]) {
-    floatx16 hi;
+__device__ __forceinline__ floatx16 wave_product(const float (&a)[NS][16], const float (&b)[NS][16]) {
+    floatx16 acc;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) hi[r] = 0.f;
-    if constexpr (NS > 1) {
-        float ma = 0.f, mb = 0.f;
-        floatx16 lo;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) lo[r] = 0.f;
-#pragma unroll
-        for (int q = 0; q < NS; ++q)
-#pragma unroll
-            for (int s = 0; s < 16; s += 8) {
-                uint32_t pa[4][2], pb[4][2];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const float a0 = a[q][s + 2 * i], a1 = a[q][s + 2 * i + 1];
-                    const float b0 = b[q][s + 2 * i], b1 = b[q][s + 2 * i + 1];
-                    SplitF16::cut(a0, a1, pa[i]);
-                    SplitF16::cut(b0, b1, pb[i]);
-                    ma = fmaxf(fmaxf(__builtin_fabsf(a0), __builtin_fabsf(a1)), ma);
-                    mb = fmaxf(fmaxf(__builtin_fabsf(b0), __builtin_fabsf(b1)), mb);
-                }
-                f16x8 fa[2], fb[2];
-#pragma unroll
-                for (int p = 0; p < 2; ++p) {
-                    fa[p] = __builtin_bit_cast(f16x8, u32v4{pa[0][p], pa[1][p], pa[2][p], pa[3][p]});
-                    fb[p] = __builtin_bit_cast(f16x8, u32v4{pb[0][p], pb[1][p], pb[2][p], pb[3][p]});
-                }
-                hi = SplitF16::mma(fa[0], fb[0], hi);
-                lo = SplitF16::mma(fa[1], fb[0], lo);
-                lo = SplitF16::mma(fa[0], fb[1], lo);
-            }
-        const bool ok = (ma == 0.f || ma >= 0x1p-12f) && ma <= 65504.f && (mb == 0.f || mb >= 0x1p-12f) && mb <= 65504.f;
-        if (__all(ok)) {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const float x = hi[r], y = lo[r];
-                hi[r] = SplitF16::sum(x, y);
-            }
-            return hi;
-        }
-#pragma unroll
-        for (int r = 0; r < 16; ++r) hi[r] = 0.f;
-    }
+    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
 #pragma unroll
     for (int q = 0; q < NS; ++q)
 #pragma unroll
-        for (int c = 0; c < 16; ++c) hi = __builtin_amdgcn_mfma_f32_32x32x2f32(a[q][c], b[q][c], hi, 0, 0, 0);
-    return hi;
+        for (int c = 0; c < 16; ++c) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[q][c], b[q][c], acc, 0, 0, 0);
+    return acc;
+}
+
+// The same in bf16 pieces, twelve 8-pass instructions a slice in place of
+// sixteen 16-pass ones and 208 VALU operations beside them. A wave with a sum
+// that is not finite goes over its registers again with the fp32 instruction.
+template <int NS>
+__device__ __forceinline__ floatx16 wave_product_pieces(const float (&a)[NS][16], const float (&b)[NS][16]) {
+    floatx16 hi, lo;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) hi[r] = lo[r] = 0.f;
+#pragma unroll
+    for (int q = 0; q < NS; ++q)
+#pragma unroll
+        for (int s = 0; s < 16; s += 8) {
+            uint32_t pa[4][3], pb[4][3];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                SplitB16::cut(a[q][s + 2 * i], a[q][s + 2 * i + 1], pa[i]);
+                SplitB16::cut(b[q][s + 2 * i], b[q][s + 2 * i + 1], pb[i]);
+            }
+            bf16x8 fa[3], fb[3];
+#pragma unroll
+            for (int p = 0; p < 3; ++p) {
+                fa[p] = __builtin_bit_cast(bf16x8, u32v4{pa[0][p], pa[1][p], pa[2][p], pa[3][p]});
+                fb[p] = __builtin_bit_cast(bf16x8, u32v4{pb[0][p], pb[1][p], pb[2][p], pb[3][p]});
+            }
+            hi = SplitB16::mma(fa[0], fb[0], hi);
+            lo = SplitB16::mma(fa[1], fb[0], lo);
+            lo = SplitB16::mma(fa[0], fb[1], lo);
+            lo = SplitB16::mma(fa[1], fb[1], lo);
+            lo = SplitB16::mma(fa[2], fb[0], lo);
+            lo = SplitB16::mma(fa[0], fb[2], lo);
+        }
+    bool ok = true;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const float x = hi[r], y = lo[r];
+        hi[r] = SplitB16::sum(x, y, ok);
+    }
+    return __all(ok) ? hi : wave_product<NS>(a, b);
+}
+
+template <int NS, bool PIECES>
+__device__ __forceinline__ floatx16 wave_product_as(const float (&a)[NS][16], const float (&b)[NS][16]) {
+    if constexpr (PIECES) return wave_product_pieces<NS>(a, b);
+    else return wave_product<NS>(a, b);
 }
 
 }  // namespace nnc

@@ -1,10 +1,9 @@
 """Short convolutions and products on 32 x 32 tiles held in registers
 (conv_ws_k, conv_wss_k, gemm_ws_k, gemm_wsu_k): weights as stored, rows off
 16-byte boundaries, K that ends inside a 16-byte load, a tile's K split over
-workgroups, and values outside the two-piece split's range, where a wave
-takes the fp32 instruction. The reference is the float64 result; an output
-may be off by 2^-21 of the sum of its terms' magnitudes (the split leaves out
-2^-23 of each term per piece, one rounding per 16 terms, K <= 4096).
+workgroups, and operands of any size. The reference is the float64 result; an
+output may be off by 2^-21 of the sum of its terms' magnitudes (one rounding
+per 2 terms of random signs, K <= 4096).
 """
 
 from __future__ import annotations

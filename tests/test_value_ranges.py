@@ -14,12 +14,14 @@ from __future__ import annotations
 import numpy as np
 import pytest
 
-from test_split_products import _check, _conv, _gemm
+from test_split_products import _call, _check, _conv, _gemm
 
 pytestmark = pytest.mark.gpu
 
-# (m, n, k, nt): 128x128, 128x64 (unaligned) and 64x64 tiles
-PRODUCTS = [(1500, 1100, 640, True), (1500, 1100, 640, False), (1999, 2001, 333, True), (700, 900, 544, False)]
+# (m, n, k, nt): 128x128, 128x64 (unaligned) and 64x64 tiles, and short
+# products on 32x32 tiles (aligned, unaligned)
+PRODUCTS = [(1500, 1100, 640, True), (1500, 1100, 640, False), (1999, 2001, 333, True), (700, 900, 544, False),
+            (64, 352, 1120, True), (129, 300, 263, True)]
 
 
 def _uniform(rng, *shape):
@@ -111,8 +113,10 @@ def test_whole_numbers_are_exact(m, n, k, nt, hip, abi):
     assert np.array_equal(_gemm(hip, abi, a, b, nt), (a.astype(np.float64) @ b).astype(np.float32))
 
 
-# (n, ci, h, w, co, k): tiles of 128x128 and 64x256 (whole, shared)
-CONVS = [(16, 256, 28, 27, 128, 1), (32, 64, 56, 56, 64, 3), (8, 256, 14, 14, 256, 3)]
+# (n, ci, h, w, co, k): tiles of 128x128 and 64x256 (whole, shared); short, in
+# pieces (five slices a wave on 392 tiles) and with the fp32 instruction
+CONVS = [(16, 256, 28, 27, 128, 1), (32, 64, 56, 56, 64, 3), (8, 256, 14, 14, 256, 3), (2, 64, 56, 56, 64, 3),
+         (1, 64, 14, 14, 64, 3), (1, 96, 9, 11, 40, 1)]
 
 
 @pytest.mark.parametrize("which", sorted(EXPONENTS))
@@ -139,3 +143,38 @@ def test_small_beside_large_channels(shape, which, hip, abi):
     x = (_uniform(rng, n, ci, h, w) * np.abs(a.reshape(1, ci, 1, 1))).astype(np.float32)
     v = (_uniform(rng, co, k, k, ci) * np.abs(b.reshape(ci))).astype(np.float32)
     _check(*_conv(hip, abi, x, v, 1, k // 2), f"{shape} {which}")
+
+
+# (n, ci, h, w, co): with the fp32 instruction, and in pieces (six slices a
+# wave on 352 tiles, K % 4 == 3 and 0)
+@pytest.mark.parametrize("which", ["2^-30", "plain", "one", "whole", "large", "inf", "nan"])
+@pytest.mark.parametrize("shape", [(1, 83, 9, 11, 40), (3, 83, 30, 31, 100), (3, 84, 30, 31, 100)], ids=str)
+def test_stored_weights(shape, which, hip, abi):
+    """The short kernel of weights as stored."""
+    n, ci, h, w, co = shape
+    print(f"case stored conv {shape} {which}", flush=True)
+    rng = np.random.default_rng(4)
+    x, v = _uniform(rng, n, ci, h, w), _uniform(rng, co, ci, 3, 3)
+    pick = rng.integers(0, ci, co)
+    if which in ("one", "whole"):
+        x = _spread(rng, x.shape, 0, 0) if which == "one" else rng.integers(-4095, 4096, x.shape).astype(np.float32)
+        v[:] = 0
+        v[np.arange(co), pick, 1, 1] = 1 if which == "one" else 4095
+    elif which == "large":
+        x *= np.float32(1e32)
+    elif which == "inf":
+        x[0, 5, 4, 6] = np.inf
+    elif which == "nan":
+        v[7, 80, 0, 2] = np.nan
+    else:
+        a, b = _mixed(rng, which, 1, 1, ci)
+        x *= np.abs(a.reshape(1, ci, 1, 1))
+        v *= np.abs(b.reshape(1, ci, 1, 1))
+    got = _call(abi, lambda i, u, o, *s: hip.nnc_conv(i, u, None, o, *s), [x, v], (3, 3, 1, 1, 1, 1), (n, co, h, w))
+    if which in ("one", "whole"):
+        assert np.array_equal(got, x[:, pick] * v[np.arange(co), pick, 1, 1].reshape(1, co, 1, 1))
+        return
+    xp = np.pad(x, ((0, 0), (0, 0), (1, 1), (1, 1)))
+    cols = np.stack([xp[:, :, r:r + h, q:q + w] for r in range(3) for q in range(3)], 2)
+    cols = cols.transpose(1, 2, 0, 3, 4).reshape(ci * 9, n * h * w)
+    _check(got.transpose(1, 0, 2, 3).reshape(co, -1), v.reshape(co, -1), cols, which)
