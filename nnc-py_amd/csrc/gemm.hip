@@ -50,17 +50,25 @@ struct GemmArgs {
     int out32;  // one batch of out (and C) below 2 GiB: whole tiles use 32-bit buffer offsets
 };
 
-// Tile `rem` of a batch: bands of kTileBand tile rows, each column by column,
-// so that 64 consecutive tiles (the workgroups of one XCD) share 8 row blocks
-// of A and 8 column blocks of B through its L2 rather than 2 column blocks
-// and every row block.
+// Tile `rem` of a batch, column by column. BAND (the split kernels, several
+// rounds of tiles): bands of kTileBand tile rows, each column by column, so
+// that 64 consecutive tiles (the workgroups of one XCD) share 8 row blocks of
+// A and 8 column blocks of B through its L2 rather than 2 column blocks and
+// every row block. Its second division costs the one-round kernels 0.07 us
+// ([64,128,64] x [64,64,128] 6.45 and 6.52) for nothing.
 static constexpr int kTileBand = 8;
+template <bool BAND>
 __device__ __forceinline__ void tile_pos(const GemmArgs& g, int rem, int& mt, int& nt) {
-    const int per_band = kTileBand * g.tiles_n;
-    const int band = rem / per_band, in = rem - band * per_band;
-    const int rows = min(kTileBand, g.tiles_m - band * kTileBand);
-    nt = in / rows;
-    mt = band * kTileBand + (in - nt * rows);
+    if constexpr (BAND) {
+        const int per_band = kTileBand * g.tiles_n;
+        const int band = rem / per_band, in = rem - band * per_band;
+        const int rows = min(kTileBand, g.tiles_m - band * kTileBand);
+        nt = in / rows;
+        mt = band * kTileBand + (in - nt * rows);
+    } else {
+        mt = rem % g.tiles_m;
+        nt = rem / g.tiles_m;
+    }
 }
 
 __device__ __forceinline__ float gemm_finish(const GemmArgs& g, int i, int j, float v) {
@@ -157,7 +165,7 @@ __global__ void __launch_bounds__(256, 2) gemm_streamk_k(GemmArgs g, StreamK sk)
     while (walk.next(sk, seg)) {
         const int batch = seg.tile / per_batch, rem = seg.tile - batch * per_batch;
         int mt, nt;
-        tile_pos(g, rem, mt, nt);
+        tile_pos<false>(g, rem, mt, nt);
         const int i0 = mt * T::BM, j0 = nt * T::BN;
         typename PA::type la;
         typename PB::type lb;
@@ -197,7 +205,7 @@ __global__ void __launch_bounds__(256, 2) gemm_streamk_k(GemmArgs g, StreamK sk)
 // (256 float4 of the BM x BN tile): shared tiles sum their partials in
 // workgroup order and apply alpha / beta * C / relu. Each thread handles 4
 // consecutive columns of a tile row.
-template <class T>
+template <class T, bool BAND>
 __global__ void __launch_bounds__(256) gemm_fixup_k(GemmArgs g, StreamK sk) {
     const int t = blockIdx.y;
     int g0, g1, first_slot;
@@ -207,7 +215,7 @@ __global__ void __launch_bounds__(256) gemm_fixup_k(GemmArgs g, StreamK sk) {
     const int per_batch = g.tiles_m * g.tiles_n;
     const int batch = t / per_batch, rem = t - batch * per_batch;
     int mt, nt;
-    tile_pos(g, rem, mt, nt);
+    tile_pos<BAND>(g, rem, mt, nt);
     const int i = mt * T::BM + (e4 * 4) / T::BN;
     const int j = nt * T::BN + (e4 * 4) % T::BN;
     if (i >= g.M || j >= g.N) return;
@@ -336,7 +344,7 @@ struct XcOperand {
 // last: partials summed in workgroup order g0..g1 (the order of
 // gemm_fixup_k, so the result is the same to the bit), then alpha / beta * C
 // / relu. Each thread handles 4 consecutive columns of a tile row.
-template <class T>
+template <class T, bool BAND>
 __device__ __forceinline__ void gemm_finish_tile(const GemmArgs& g, int t, int g0, int g1, int first_slot) {
     constexpr int E = T::BM * T::BN / 1024;  // float4 per thread
     constexpr int CH = E < 4 ? E : 4;         // float4 in flight per partial (register budget)
@@ -344,7 +352,7 @@ __device__ __forceinline__ void gemm_finish_tile(const GemmArgs& g, int t, int g
     const int per_batch = g.tiles_m * g.tiles_n;
     const int batch = t / per_batch, rem = t - batch * per_batch;
     int mt, nt;
-    tile_pos(g, rem, mt, nt);
+    tile_pos<BAND>(g, rem, mt, nt);
     const int i0 = mt * T::BM, j0 = nt * T::BN;
     const uint32_t first = slot_byte_offset<T>(g0, first_slot);
     for (int e0 = 0; e0 < E; e0 += CH) {
@@ -426,7 +434,7 @@ __device__ __forceinline__ void gemm_segment_out(const GemmArgs& g, const Stream
                 }
         int g0, g1, first_slot;
         tile_partials(sk, seg.tile, g0, g1, first_slot);
-        if (finish_arrive(g.cnt + seg.tile, g1 - g0)) gemm_finish_tile<T>(g, seg.tile, g0, g1, first_slot);
+        if (finish_arrive(g.cnt + seg.tile, g1 - g0)) gemm_finish_tile<T, false>(g, seg.tile, g0, g1, first_slot);
     }
 }
 
@@ -476,7 +484,7 @@ __global__ void __launch_bounds__(T::THREADS, (GemmDma<T, NS>::MIN_WAVES)) gemm_
     auto set_tile = [&](int tile) {
         const int batch = tile / per_batch, rem = tile - batch * per_batch;
         int mt, nt;
-        tile_pos(g, rem, mt, nt);
+        tile_pos<false>(g, rem, mt, nt);
         const int i0 = mt * T::BM, j0 = nt * T::BN;
         oa.tile(g.A + batch * g.sa + OA::origin(i0, g.lda), g.lda, g.M - i0, wave, lane);
         ob.tile(g.B + batch * g.sb + OB::origin(j0, g.ldb), g.ldb, g.N - j0, wave, lane);
@@ -504,7 +512,7 @@ __global__ void __launch_bounds__(T::THREADS, (GemmDma<T, NS>::MIN_WAVES)) gemm_
     while (true) {
         const int batch = seg.tile / per_batch, rem = seg.tile - batch * per_batch;
         int mt, nt;
-        tile_pos(g, rem, mt, nt);
+        tile_pos<false>(g, rem, mt, nt);
         const int i0 = mt * T::BM, j0 = nt * T::BN;
         floatx16 sum[T::TM][T::TN];
 #pragma unroll
@@ -602,7 +610,7 @@ struct GemmSplit {
         batch = tile / per_batch;
         const int rem = tile - batch * per_batch;
         int mt, nt;
-        tile_pos(g, rem, mt, nt);
+        tile_pos<true>(g, rem, mt, nt);
         i0 = mt * T::BM;
         j0 = nt * T::BN;
     }
@@ -630,7 +638,7 @@ struct GemmSplit {
         if (!g.cnt) return;  // gemm_fixup_k finishes the tile
         int g0, g1, first_slot;
         tile_partials(sk, seg.tile, g0, g1, first_slot);
-        if (finish_arrive(g.cnt + seg.tile, g1 - g0)) gemm_finish_tile<T>(g, seg.tile, g0, g1, first_slot);
+        if (finish_arrive(g.cnt + seg.tile, g1 - g0)) gemm_finish_tile<T, true>(g, seg.tile, g0, g1, first_slot);
     }
 };
 
@@ -933,7 +941,7 @@ static void launch_mfma(GemmArgs& g, int batches, const char* name) {
     launch(kname, kernel, dim3(sk.G), dim3(256), lds, g, sk);
     if (sk.needs_fixup()) {
         set_work(0.0, 0.0);
-        launch("gemm_streamk_fixup", gemm_fixup_k<T>, dim3(T::BM * T::BN / 1024, sk.sk_tiles), dim3(256), 0, g, sk);
+        launch("gemm_streamk_fixup", gemm_fixup_k<T, false>, dim3(T::BM * T::BN / 1024, sk.sk_tiles), dim3(256), 0, g, sk);
     }
 }
 
@@ -949,18 +957,15 @@ __global__ void __launch_bounds__(256) gemm_zero_counters_k(int* p, int n) {
     if (i < n) p[i] = 0;
 }
 
-// LDS stages of the direct-to-LDS kernel: 64x64 tiles have short slices
+// LDS stages of the direct-to-LDS kernel: its 64x64 tiles have short slices
 // (16 MFMAs per wave) and keep three slices in flight
-template <class T>
-constexpr int dma_stages() {
-    return 4;
-}
+static constexpr int kDmaStages = 4;
 
 // Direct-to-LDS stream-K launch; OA / OB: KcOperand or XcOperand. At most one
 // round of 64x64 tiles over at most 8 slices (gemm_stays_fp32).
 template <class T, class OA, class OB>
 static void launch_gemm_dma(GemmArgs& g, int batches, const char* name, const char* kname) {
-    constexpr int NS = dma_stages<T>();
+    constexpr int NS = kDmaStages;
     auto kernel = gemm_dma_k<T, NS, OA, OB, true>;
     const size_t lds = (size_t)GemmDma<T, NS>::LDS_FLOATS * sizeof(float);
     // once per kernel, thread-safe (C++ static initialisation): the LDS limit
@@ -992,7 +997,7 @@ static void launch_gemm_dma(GemmArgs& g, int batches, const char* name, const ch
     launch(kname, kernel, dim3(sk.G), dim3(T::THREADS), lds, g, sk);
     if (sk.needs_fixup() && !g.cnt) {
         set_work(0.0, 0.0);
-        launch("gemm_streamk_fixup", gemm_fixup_k<T>, dim3(T::BM * T::BN / 1024, sk.sk_tiles), dim3(256), 0, g, sk);
+        launch("gemm_streamk_fixup", gemm_fixup_k<T, false>, dim3(T::BM * T::BN / 1024, sk.sk_tiles), dim3(256), 0, g, sk);
     }
 }
 
@@ -1041,7 +1046,7 @@ static void launch_gemm_split(GemmArgs& g, int batches, const StreamK& sk, const
     launch(kname, kernel, dim3(sk.G), dim3(T::THREADS), lds, g, sk);
     if (sk.needs_fixup() && !g.cnt) {
         set_work(0.0, 0.0);
-        launch("gemm_streamk_fixup", gemm_fixup_k<T>, dim3(T::BM * T::BN / 1024, sk.sk_tiles), dim3(256), 0, g, sk);
+        launch("gemm_streamk_fixup", gemm_fixup_k<T, true>, dim3(T::BM * T::BN / 1024, sk.sk_tiles), dim3(256), 0, g, sk);
     }
 }
 
