@@ -1541,30 +1541,39 @@ static void launch_conv_split(ConvArgs& a, const StreamK& sk, const char* entry)
 
 // A tap-major convolution on split_tile.h's tiles (plan_conv_split). Their
 // epilogue stores through 32-bit offsets: an output of 2 GiB or more goes in
-// ranges of images, a single image's in ranges of channels.
+// ranges of images, a single image's in ranges of channels, a single plane's
+// in ranges of rows, a single row's in ranges of pixels.
 template <int KH, int KW, bool PROJ>
 static void conv_split(ConvArgs& a, const char* entry) {
     if (!a.out32) {
         const int64_t hw = (int64_t)a.Ho * a.Wo, most = (((int64_t)1 << 31) - 1) / 4;
-        const bool images = a.N > 1;
-        const int64_t unit = images ? a.Co * hw : hw, total = images ? a.N : a.Co;
-        if (!images && hw > most) return fail(NNC_HIP_EUNSUPP, entry, "an output plane spans 2 GiB or more");
-        const int64_t per = std::max<int64_t>(1, most / unit);
+        const int level = a.N > 1 ? 0 : a.Co > 1 ? 1 : a.Ho > 1 ? 2 : 3;
+        const int64_t units[] = {a.Co * hw, hw, a.Wo, 1}, totals[] = {a.N, a.Co, a.Ho, a.Wo};
+        const int64_t unit = units[level], total = totals[level], per = std::max<int64_t>(1, most / unit);
         for (int64_t u = 0; u < total; u += per) {
             ConvArgs c = a;
             const int64_t n = std::min(per, total - u);
             c.out = a.out + u * unit;
             if (a.res) c.res = a.res + u * unit;
-            if (images) {
+            c.vec_out = aligned16(c.out) && (!c.res || aligned16(c.res));
+            if (level == 0) {
                 c.N = (int)n;
-                c.Npix = (int)(n * hw);
                 c.in = a.in + u * a.Ci * a.H * a.W;
                 if (PROJ) c.pin = a.pin + u * a.pci * a.pH * a.pW;
-            } else {
+            } else if (level == 1) {
                 c.Co = (int)n;
                 c.w = a.w + u * a.ldw;
                 if (a.bias) c.bias = a.bias + u;
+            } else if (level == 2) {
+                c.Ho = (int)n;
+                c.ph = (int)(a.ph - u * a.sh);
+                if (PROJ) c.pin = a.pin + u * a.psh * a.pW;
+            } else {
+                c.Wo = (int)n;
+                c.pw = (int)(a.pw - u * a.sw);
+                if (PROJ) c.pin = a.pin + u * a.psw;
             }
+            c.Npix = c.N * c.Ho * c.Wo;
             c.out32 = n * unit <= most;
             conv_split<KH, KW, PROJ>(c, entry);
         }

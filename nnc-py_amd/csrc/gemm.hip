@@ -1434,7 +1434,9 @@ static void gemm_run(const GemmProblem& p, const char* name) {
     const bool aligned = (akind == kKC4 || akind == kXC4) && (bkind == kKC4 || bkind == kXC4);
     const int64_t tiles64 = ceil_div(p.M, 64) * ceil_div(p.N, 64) * p.batches;
     const int64_t iters = ceil_div(p.K, 32);
-    if (gemm_stays_fp32(tiles64, iters, aligned, cu_count())) {
+    // (an output row of 2 GiB or more: tiles that store through 64-bit addresses)
+    const bool row64 = (int64_t)p.N * 4 >= ((int64_t)1 << 31);
+    if (row64 || gemm_stays_fp32(tiles64, iters, aligned, cu_count())) {
         if (aligned) return dispatch_dma<GemmT64>(g, akind == kKC4, bkind == kKC4, p.batches, name);
         switch (akind) {
             case kKC4: return dispatch_b_small<kKC4>(g, bkind, p.batches, name);
@@ -1446,7 +1448,6 @@ static void gemm_run(const GemmProblem& p, const char* name) {
     if (!g.out32) {
         // tiles store through 32-bit offsets: row ranges of less than 2 GiB
         const int64_t rows = (((int64_t)1 << 31) - 1) / ((int64_t)p.N * 4);
-        if (rows < 1) return fail(NNC_HIP_EUNSUPP, name, "an output row spans 2 GiB or more");
         for (int64_t i0 = 0; i0 < p.M; i0 += rows) {
             GemmProblem q = p;
             q.M = (int)std::min<int64_t>(rows, p.M - i0);

@@ -178,3 +178,33 @@ def test_stored_weights(shape, which, hip, abi):
     cols = np.stack([xp[:, :, r:r + h, q:q + w] for r in range(3) for q in range(3)], 2)
     cols = cols.transpose(1, 2, 0, 3, 4).reshape(ci * 9, n * h * w)
     _check(got.transpose(1, 0, 2, 3).reshape(co, -1), v.reshape(co, -1), cols, which)
+
+
+# ---------------------------------------------------------------------------
+# extents past 32-bit byte offsets
+# ---------------------------------------------------------------------------
+def test_output_row_of_2_gib(hip, abi):
+    m, n = 2, (1 << 29) + 72
+    print(f"case gemm_nt {m}x{n}x1", flush=True)
+    a = np.array([[3], [-5]], np.float32)
+    b = (np.arange(n, dtype=np.int64) % 8191).astype(np.float32).reshape(n, 1)
+    got = _call(abi, lambda x, y, o, *s: hip.nnc_gemm_nt(x, y, None, o, *s), [a, b], (1.0, 0.0), (m, n))
+    assert np.array_equal(got[0], 3 * b[:, 0]) and np.array_equal(got[1], -5 * b[:, 0])
+
+
+@pytest.mark.parametrize("k", [1, 3])
+def test_output_plane_of_2_gib(k, hip, abi):
+    """A plane that reaches far past its image: the bias there."""
+    side = 23171
+    print(f"case conv {k}x{k} plane {side}", flush=True)
+    rng = np.random.default_rng(k)
+    x, v = _uniform(rng, 1, 32, 5, 5), _uniform(rng, 1, k, k, 32)
+    bias = np.array([0.5], np.float32)
+    got = _call(abi, lambda i, w, b, o, *s: hip.nnc_hip_conv_packed(i, w, b, None, o, *s), [x, v, bias],
+                (k, k, 1, 1, 0, 0, 0), (1, 1, side, side))[0, 0]
+    xp = np.pad(x.astype(np.float64), ((0, 0), (0, 0), (0, k), (0, k)))
+    want = sum(np.einsum("c,chw->hw", v[0, r, q].astype(np.float64), xp[0, :, r:r + 5, q:q + 5])
+               for r in range(k) for q in range(k)) + 0.5
+    assert np.max(np.abs(got[:5, :5] - want)) < 1e-4
+    got[:5, :5] = 0.5
+    assert np.all(got == np.float32(0.5))
