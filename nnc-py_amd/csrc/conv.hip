@@ -1678,7 +1678,7 @@ static constexpr int kStemK = 147, kStemSteps = 37;  // 3 * 7 * 7, rounded up to
 
 // LDS requested per workgroup: at most two workgroups per CU, so that a
 // grid of 2 per CU puts exactly two on every CU (tiles spread evenly)
-static constexpr int kStemLdsBytes = 60 * 1024;
+static constexpr int kStemLdsBytes = 56 * 1024;
 
 template <int BPR>
 struct StemShape {
@@ -1686,8 +1686,7 @@ struct StemShape {
     static constexpr int CP = 7 * LW, BUF = 3 * CP;              // channel pitch, one window
     static constexpr int CHUNKS = W / 4;                         // 16-byte pieces per input row
     static_assert(CHUNKS <= 64, "one load instruction per input row");
-    static constexpr int PLANE = BUF * 2, PIECES = 2 * BUF * 4, FLAG = PIECES + 2 * PLANE;  // byte offsets, f16 pieces
-    static_assert(FLAG + 4 <= kStemLdsBytes, "two windows and their pieces in the requested LDS");
+    static_assert(2 * BUF * 4 <= kStemLdsBytes, "two windows in the requested LDS");
 };
 
 // one tile's window: rows (ci, ky) of input row 2 oy - 3 + ky, wave w
@@ -1704,123 +1703,6 @@ __device__ __forceinline__ void stem_window(const StemArgs& a, __amdgpu_buffer_r
         const uint32_t voff =
             in_img ? (uint32_t)(((n * 3 + ci) * a.H + iy) * a.W) * 4u + (uint32_t)lane * 16u : kOutOfRange;
         if (lane < S::CHUNKS) dma_load16(rin, buf + ci * S::CP + ky * S::LW + 4, voff, 0);
-    }
-}
-
-// The products of a row on the 16-bit matrix units (SplitF16 of
-// split_tile.h): the window is cut into two f16 planes once per row, for all
-// four waves and every tap, and v_mfma_f32_16x16x32_f16 reads its 8 k per lane
-// out of them: k group g = ci * 7 + ky, the eight columns from 2 ox on, i.e.
-// kx = -1 .. 6 with a zero weight for kx = -1 (21 groups in 6 steps of 4). Out
-// of the window as fp32, one v_mfma_f32_16x16x4_f32 per 4 k, the products of a
-// row took 8300 cycles of each SIMD, now 2000: 92 -> 70 us at batch 32.
-// Pixels are scaled by 2^8 first, so that f16's range starts at 2^-20 for
-// them: a row whose window has a value above 255.8, or a pair of neighbours
-// that is not zero but below 2^-20, infinities or NaN goes to the fp32
-// instruction, and so does everything where the weights are outside f16's
-// range.
-struct StemWeights {
-    f16x8 w[2][6];  // [piece][step]: this lane's channel, group 4 step + lane / 16
-    bool ok;
-};
-
-// (call with the whole workgroup: has a barrier)
-__device__ __forceinline__ void stem_weights(const StemArgs& a, __amdgpu_buffer_rsrc_t rw, int co, int kq, StemWeights& W) {
-    float mx = 0.f;
-    bool fin = true;
-#pragma unroll
-    for (int s = 0; s < 6; ++s) {
-        const int g = 4 * s + kq, ci = g / 7, ky = g - ci * 7;
-        float v[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const bool in = g < 21 && e > 0;
-            v[e] = load_f32(rw, in ? (uint32_t)(co * a.ldw + (ky * 7 + e - 1) * 3 + ci) * 4u : kOutOfRange);
-            fin = fin && __builtin_fabsf(v[e]) <= 65504.f;
-            mx = fmaxf(mx, __builtin_fabsf(v[e]));
-        }
-        uint32_t p[4][2];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) SplitF16::cut(v[2 * e], v[2 * e + 1], p[e]);
-#pragma unroll
-        for (int q = 0; q < 2; ++q) W.w[q][s] = __builtin_bit_cast(f16x8, u32v4{p[0][q], p[1][q], p[2][q], p[3][q]});
-    }
-    W.ok = !__syncthreads_or(!(fin && (mx == 0.f || mx >= 0x1p-12f)));
-}
-
-// Cuts the window at `win` into the pieces; true (for the whole workgroup) if
-// they hold it. `row`: the workgroup's row count, from 1.
-template <int BPR>
-__device__ __forceinline__ bool stem_cut(char* lds, const float* win, int row) {
-    typedef StemShape<BPR> S;
-    bool ok = true;
-    for (int e = threadIdx.x; e < S::BUF / 4; e += 256) {
-        const f32x4 x = *reinterpret_cast<const f32x4*>(win + 4 * e) * 256.f;
-        const float x0 = x[0], x1 = x[1], x2 = x[2], x3 = x[3];
-        const float m0 = fmaxf(__builtin_fabsf(x0), __builtin_fabsf(x1)), m1 = fmaxf(__builtin_fabsf(x2), __builtin_fabsf(x3));
-        ok = ok && (m0 == 0.f || m0 >= 0x1p-12f) && (m1 == 0.f || m1 >= 0x1p-12f);
-        ok = ok && __builtin_fabsf(x0) <= 65504.f && __builtin_fabsf(x1) <= 65504.f && __builtin_fabsf(x2) <= 65504.f &&
-             __builtin_fabsf(x3) <= 65504.f;
-        uint32_t p[2][2];
-        SplitF16::cut(x0, x1, p[0]);
-        SplitF16::cut(x2, x3, p[1]);
-#pragma unroll
-        for (int q = 0; q < 2; ++q)
-            *reinterpret_cast<u32v2*>(lds + S::PIECES + q * S::PLANE + 8 * e) = u32v2{p[0][q], p[1][q]};
-    }
-    int* flag = reinterpret_cast<int*>(lds + S::FLAG);
-    if (!ok) *flag = row;
-    dma_barrier<63>();  // (the next window's loads stay in flight)
-    return __builtin_amdgcn_readfirstlane(*flag) != row;
-}
-
-// One output row's products, lane (channel, 4 pixels 16 b + 4 kq ..).
-template <int BPR>
-__device__ __forceinline__ void stem_row(const StemArgs& a, __amdgpu_buffer_rsrc_t rw, const char* lds, const float* win,
-                                         const StemWeights& W, bool split, int co, int j, int kq, f32x4 (&acc)[BPR]) {
-    typedef StemShape<BPR> S;
-#pragma unroll
-    for (int b = 0; b < BPR; ++b) acc[b] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (split) {
-        f32x4 lo[BPR];
-#pragma unroll
-        for (int b = 0; b < BPR; ++b) lo[b] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int s = 0; s < 6; ++s) {
-            // groups past 20 have zero weights: any finite columns do
-            const int g = s < 5 ? 4 * s + kq : 20;
-            const char* at = lds + S::PIECES + (g * S::LW + 2 * j) * 2;
-#pragma unroll
-            for (int b = 0; b < BPR; ++b) {
-                f16x8 x[2];
-#pragma unroll
-                for (int q = 0; q < 2; ++q) {
-                    const uint32_t* d = reinterpret_cast<const uint32_t*>(at + q * S::PLANE + 64 * b);
-                    x[q] = __builtin_bit_cast(f16x8, u32v4{d[0], d[1], d[2], d[3]});
-                }
-                acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x[0], W.w[0][s], acc[b], 0, 0, 0);
-                lo[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x[1], W.w[0][s], lo[b], 0, 0, 0);
-                lo[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x[0], W.w[1][s], lo[b], 0, 0, 0);
-            }
-        }
-#pragma unroll
-        for (int b = 0; b < BPR; ++b)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const float x = acc[b][r], y = lo[b][r];
-                acc[b][r] = SplitF16::sum(x, y) * 0x1p-8f;
-            }
-        return;
-    }
-#pragma unroll 1
-    for (int s = 0; s < kStemSteps; ++s) {
-        const int k = 4 * s + kq;
-        const int tap = k / 3, ci = k - tap * 3, ky = tap / 7, kx = tap - ky * 7;
-        const float w = load_f32(rw, (uint32_t)(co * a.ldw + k) * 4u);
-        const float* x = win + (k < kStemK ? ci * S::CP + ky * S::LW + kx + 1 + 2 * j : 0);
-#pragma unroll
-        for (int b = 0; b < BPR; ++b)
-            acc[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(k < kStemK ? x[32 * b] : 0.f, w, acc[b], 0, 0, 0);
     }
 }
 
@@ -1847,17 +1729,49 @@ __global__ void __launch_bounds__(256, 2) __attribute__((amdgpu_waves_per_eu(2, 
     const int co_a = 16 * wave + j;  // also this lane's output channel
     const __amdgpu_buffer_rsrc_t rw =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.w), (short)0, a.Co * a.ldw * 4, 0x00020000);
-    StemWeights W;
-    if (threadIdx.x == 0) *reinterpret_cast<int*>(reinterpret_cast<char*>(lds) + S::FLAG) = 0;
-    stem_weights(a, rw, co_a, kq, W);
+    float A[kStemSteps];
+    int koff[kStemSteps];
+#pragma unroll
+    for (int s = 0; s < kStemSteps; ++s) {
+        const int k = 4 * s + kq;
+        A[s] = load_f32(rw, (uint32_t)(co_a * a.ldw + k) * 4u);
+        const int tap = k / 3, ci = k - tap * 3, ky = tap / 7, kx = tap - ky * 7;
+        koff[s] = k < kStemK ? ci * S::CP + ky * S::LW + kx + 1 + 2 * j : 0;
+    }
     const float bias = a.bias && co_a < a.Co ? a.bias[co_a] : 0.f;
     dma_barrier<0>();  // both windows landed, pad columns written
     for (int i = 0; t < a.tiles; ++i, t += G) {
         const float* B = lds + (i & 1) * S::BUF;
-        char* pieces = reinterpret_cast<char*>(lds);
-        const bool split = stem_cut<BPR>(pieces, B, i + 1) && W.ok;
         f32x4 acc[BPR];
-        stem_row<BPR>(a, rw, pieces, B, W, split, co_a, j, kq, acc);
+#pragma unroll
+        for (int b = 0; b < BPR; ++b) acc[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+        // B values one step ahead of the MFMAs that use them
+        float x[BPR];
+#pragma unroll
+        for (int b = 0; b < BPR; ++b) x[b] = B[koff[0] + 32 * b];
+#pragma unroll
+        for (int s = 0; s < kStemSteps; ++s) {
+            float xn[BPR];
+            if (s + 1 < kStemSteps) {
+#pragma unroll
+                for (int b = 0; b < BPR; ++b) xn[b] = B[koff[s + 1] + 32 * b];
+            }
+            if (s == kStemSteps - 1 && 4 * s + kq >= kStemK) {
+#pragma unroll
+                for (int b = 0; b < BPR; ++b) x[b] = 0.f;  // k past K: no input term, not even 0 * inf
+            }
+#pragma unroll
+            for (int b = 0; b < BPR; ++b) acc[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[b], A[s], acc[b], 0, 0, 0);
+            if (s + 1 < kStemSteps) {
+#pragma unroll
+                for (int b = 0; b < BPR; ++b) x[b] = xn[b];
+                // schedule the next step's LDS reads ahead of this step's
+                // MFMAs (left alone, the scheduler waits on each read right
+                // before its MFMA)
+                __builtin_amdgcn_sched_group_barrier(0x100, (BPR + 1) / 2, 0);  // DS reads (paired)
+                __builtin_amdgcn_sched_group_barrier(0x008, BPR, 0);            // MFMAs
+            }
+        }
         // the next window landed (loaded a whole tile ago) and every wave is
         // done with this one: refill it with the tile after next
         dma_barrier<0>();
@@ -1952,9 +1866,15 @@ conv_stem_pool_k(StemArgs a, PoolBand pb) {
     const int co_a = 16 * wave + j;  // also this lane's output channel
     const __amdgpu_buffer_rsrc_t rw =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.w), (short)0, a.Co * a.ldw * 4, 0x00020000);
-    StemWeights W;
-    if (threadIdx.x == 0) *reinterpret_cast<int*>(reinterpret_cast<char*>(lds) + S::FLAG) = 0;
-    stem_weights(a, rw, co_a, kq, W);
+    float A[kStemSteps];
+    int koff[kStemSteps];
+#pragma unroll
+    for (int s = 0; s < kStemSteps; ++s) {
+        const int k = 4 * s + kq;
+        A[s] = load_f32(rw, (uint32_t)(co_a * a.ldw + k) * 4u);
+        const int tap = k / 3, ci = k - tap * 3, ky = tap / 7, kx = tap - ky * 7;
+        koff[s] = k < kStemK ? ci * S::CP + ky * S::LW + kx + 1 + 2 * j : 0;
+    }
     const float bias = a.bias && co_a < a.Co ? a.bias[co_a] : 0.f;
     dma_barrier<0>();
     float run[BPR][2];  // maxima of the current pool row's rows so far
@@ -1967,10 +1887,32 @@ conv_stem_pool_k(StemArgs a, PoolBand pb) {
     bool first_pending = start_shared;
     for (int t = t0, i = 0; t < t1; ++t, ++i) {
         const float* B = lds + (i & 1) * S::BUF;
-        char* pieces = reinterpret_cast<char*>(lds);
-        const bool split = stem_cut<BPR>(pieces, B, i + 1) && W.ok;
         f32x4 acc[BPR];
-        stem_row<BPR>(a, rw, pieces, B, W, split, co_a, j, kq, acc);
+#pragma unroll
+        for (int b = 0; b < BPR; ++b) acc[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+        float x[BPR];
+#pragma unroll
+        for (int b = 0; b < BPR; ++b) x[b] = B[koff[0] + 32 * b];
+#pragma unroll
+        for (int s = 0; s < kStemSteps; ++s) {
+            float xn[BPR];
+            if (s + 1 < kStemSteps) {
+#pragma unroll
+                for (int b = 0; b < BPR; ++b) xn[b] = B[koff[s + 1] + 32 * b];
+            }
+            if (s == kStemSteps - 1 && 4 * s + kq >= kStemK) {
+#pragma unroll
+                for (int b = 0; b < BPR; ++b) x[b] = 0.f;
+            }
+#pragma unroll
+            for (int b = 0; b < BPR; ++b) acc[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[b], A[s], acc[b], 0, 0, 0);
+            if (s + 1 < kStemSteps) {
+#pragma unroll
+                for (int b = 0; b < BPR; ++b) x[b] = xn[b];
+                __builtin_amdgcn_sched_group_barrier(0x100, (BPR + 1) / 2, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, BPR, 0);
+            }
+        }
         dma_barrier<0>();
         if (t + 2 < t1) stem_window<BPR>(a, rin, lds + (i & 1) * S::BUF, t + 2, wave, lane);
         const int n = t / a.Ho, y = t - n * a.Ho;

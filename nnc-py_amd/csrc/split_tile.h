@@ -50,27 +50,8 @@ namespace nnc {
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u32v2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32v4 __attribute__((ext_vector_type(4)));
-
-struct SplitF16 {
-    static constexpr int PLANES = 2, PRODUCTS = 3;
-    static constexpr int OPS = 6;  // VALU operations per pair (with the row maximum)
-    typedef f16x8 Frag;
-    static __device__ __forceinline__ void cut(float x0, float x1, uint32_t (&p)[PLANES]) {
-        const f16x2 h = __builtin_convertvector(f32x2{x0, x1}, f16x2);
-        const _Float16 m0 = (_Float16)__builtin_fmaf((float)h[0], -2048.f, x0 * 2048.f);
-        const _Float16 m1 = (_Float16)__builtin_fmaf((float)h[1], -2048.f, x1 * 2048.f);
-        p[0] = __builtin_bit_cast(uint32_t, h);
-        p[1] = __builtin_bit_cast(uint32_t, f16x2{m0, m1});
-    }
-    static __device__ __forceinline__ floatx16 mma(Frag a, Frag b, floatx16 c) {
-        return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
-    }
-    static __device__ __forceinline__ float sum(float hi, float lo) { return __builtin_fmaf(lo, 0x1p-11f, hi); }
-};
 
 struct SplitB16 {
     static constexpr int PLANES = 3, PRODUCTS = 6;

@@ -181,6 +181,94 @@ def test_stored_weights(shape, which, hip, abi):
 
 
 # ---------------------------------------------------------------------------
+# the RGB stem's row kernels (512 output rows of 32 pixels): alone and with
+# its max pool
+# ---------------------------------------------------------------------------
+def _stem_case(which):
+    rng = np.random.default_rng(17)
+    x = rng.standard_normal((16, 3, 64, 64)).astype(np.float32)
+    w = (rng.standard_normal((64, 7, 7, 3)) * np.sqrt(2 / 147)).astype(np.float32)
+    if which == "bytes":
+        x = rng.integers(0, 256, x.shape).astype(np.float32)
+    elif which == "sixteen_bit":
+        x = rng.integers(0, 65536, x.shape).astype(np.float32)
+    elif which == "huge":
+        x *= np.float32(1e32)
+    elif which == "tiny":
+        x *= np.float32(1e-30)
+    elif which == "tiny_rows":
+        x[3, :, 20:40] *= np.float32(1e-9)
+        x[5] *= np.float32(1e-36)
+    elif which == "inf":
+        x[2, 1, 30, 30] = np.inf
+        x[4, 0, 0, 0] = -np.inf
+        x[7, 2, 63, 63] = np.inf
+    elif which == "nan":
+        x[2, 1, 30, 31] = np.nan
+    elif which == "lowest":  # the type's lowest value against zero and small weights
+        x[6, 0, 10, 11] = -np.finfo(np.float32).max
+        w[:, :, :, 0] *= np.float32(1e-3)
+        w[::2, :, :, 0] = 0
+    elif which == "tiny_weights":
+        w[9] *= np.float32(1e-12)
+        w[10] *= np.float32(1e-35)
+    elif which == "huge_weights":
+        w[9] *= np.float32(1e9)
+        w[10] *= np.float32(1e35)
+    elif which == "inf_weight":
+        w[11, 3, 3, 1] = np.inf
+    elif which == "nan_weight":
+        w[12, 0, 6, 2] = np.nan
+    elif which == "mixed":  # one channel large, its weights zero
+        x[:, 1:] *= np.float32(2.0 ** -40)
+        w[:, :, :, 0] = 0
+    elif which == "mixed_columns":  # the same within pairs of columns
+        x[..., 1::2] *= np.float32(2.0 ** -40)
+        w[:, :, 1::2] = 0
+    elif which == "mixed_weights":
+        x[:, 0] *= np.float32(2.0 ** -40)
+        w[:, :, :, 1:] *= np.float32(2.0 ** -60)
+    elif which in ("select", "select_one"):
+        x = _spread(rng, x.shape, *((-126, 60) if which == "select" else (0, 0)))
+        w[:] = 0
+        w[np.arange(64), rng.integers(0, 7, 64), rng.integers(0, 7, 64), rng.integers(0, 3, 64)] = 1
+    return x, w
+
+
+def _stem_columns(x):
+    xp = np.pad(x, ((0, 0), (0, 0), (3, 3), (3, 3)))
+    cols = [xp[:, :, r:r + 64:2, q:q + 64:2] for r in range(7) for q in range(7)]  # (tap, channel)
+    return np.stack(cols).transpose(0, 2, 1, 3, 4).reshape(147, -1)
+
+
+STEM = ["unit", "bytes", "sixteen_bit", "huge", "tiny", "tiny_rows", "inf", "nan", "lowest", "tiny_weights",
+        "huge_weights", "inf_weight", "nan_weight", "mixed", "mixed_columns", "mixed_weights", "select", "select_one"]
+
+
+@pytest.mark.parametrize("which", STEM)
+def test_stem_rows(which, hip, abi):
+    print(f"case stem rows {which}", flush=True)
+    x, w = _stem_case(which)
+    rows = np.zeros((64, 160), np.float32)
+    rows[:, :147] = w.reshape(64, 147)
+    got = _call(abi, lambda i, v, o, *s: hip.nnc_hip_conv_packed(i, v, None, None, o, *s), [x, rows],
+                (7, 7, 2, 2, 3, 3, 0), (16, 64, 32, 32))
+    cols = _stem_columns(x)
+    got = got.transpose(1, 0, 2, 3).reshape(64, -1)
+    if which.startswith("select"):
+        assert np.array_equal(got, (w.reshape(64, 147).astype(np.float64) @ cols).astype(np.float32))
+    else:
+        _check(got, w.reshape(64, 147), cols, which)
+    # the same row with its max pool: the pooled relu of those outputs
+    pooled = _call(abi, lambda i, v, o, *s: hip.nnc_hip_conv_maxpool(i, v, None, o, *s), [x, rows], (7, 7, 2, 2, 3, 3),
+                   (16, 64, 16, 16))
+    relu = np.where(got > 0, got, np.float32(0)).reshape(64, 16, 32, 32).transpose(1, 0, 2, 3)
+    rp = np.pad(relu, ((0, 0), (0, 0), (1, 1), (1, 1)))
+    want = np.max([rp[:, :, r:r + 32:2, q:q + 32:2] for r in range(3) for q in range(3)], axis=0)
+    assert np.array_equal(pooled, want)
+
+
+# ---------------------------------------------------------------------------
 # extents past 32-bit byte offsets
 # ---------------------------------------------------------------------------
 def test_output_row_of_2_gib(hip, abi):
