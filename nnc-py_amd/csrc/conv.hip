@@ -769,9 +769,10 @@ __global__ void __launch_bounds__(T::THREADS, DmaStage<T>::MIN_WAVES) conv_dma_k
 // at the output pixel's position times the projection stride (always inside
 // that image). Weights [Co][kh*kw*Ci + pci]; Ci and pci multiples of 32.
 //
-// ResNet-18's 3x3 layer of 128 channels with residual at batch 32, launch and
-// fixup, against the fp32 matrix instruction on direct-to-LDS tiles: 74 -> 59
-// us, error against 64 bits 1.8e-7 -> 0.7e-7.
+// ResNet-18's 3x3 layers at batch 32, launch and fixup, against the fp32
+// matrix instruction on direct-to-LDS tiles: 64 channels 85 -> 57 us, 128 with
+// residual 74 -> 58, 256 73 -> 60, 512 76 -> 64; error against 64 bits 1.8e-7
+// -> 0.7e-7.
 // ---------------------------------------------------------------------------
 template <class T, int KH, int KW, bool PROJ>
 struct SplitTaps : SplitStaged<T, T::BN, T::BN * 16 / T::THREADS> {
@@ -854,7 +855,7 @@ struct ConvSplit {
     const ConvArgs& args;
     const StreamK& sk;
     int wg;
-    KcSplit<T, T::BM, true> a;
+    KcSplit<T, T::BM, kEndSlice> a;
     B b;
     __device__ __forceinline__ ConvSplit(const ConvArgs& c, const StreamK& sk_, int wg_) : args(c), sk(sk_), wg(wg_) {
         a.init();

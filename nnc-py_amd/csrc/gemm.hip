@@ -556,10 +556,12 @@ __global__ void __launch_bounds__(T::THREADS, (GemmDma<T, NS>::MIN_WAVES)) gemm_
 // The tile engine's product on the 16-bit matrix units (split_tile.h).
 // Operand element (x, k) at base[x*ld + k] (KcSplit) or base[k*ld + x]
 // (XcSplit, 4 bytes per lane along x), rows of any alignment. Against the
-// fp32 matrix instruction: Gemm 4096^3 1016 -> 686 us (200 TFLOP/s of fp32
-// products, 1200 of bf16), error against 64 bits 1.1e-6 -> 3.8e-7.
+// fp32 matrix instruction: Gemm 4096^3 1015 -> 669 us (205 TFLOP/s of fp32
+// products, 1230 of bf16; error against 64 bits 1.1e-6 -> 3.8e-7), 2048^3 150
+// -> 101, 1536^3 74 -> 65, 256x4096x4096 84 -> 59, 777x1001x1345 (unaligned)
+// 35.7 -> 34.0.
 // ---------------------------------------------------------------------------
-template <class T, int X, bool FULL>
+template <class T, int X, KEnd END>
 struct XcSplit : SplitStaged<T, X, X * 16 / T::THREADS> {
     typedef SplitStaged<T, X, X * 16 / T::THREADS> S;
     using S::koff;
@@ -586,7 +588,7 @@ struct XcSplit : SplitStaged<T, X, X * 16 / T::THREADS> {
 #pragma unroll
         for (int i = 0; i < PER; ++i)
         {
-            const bool in = FULL || k0 + koff + i < K;  // (past K neither offset reaches the operand)
+            const bool in = END == kEndSlice || k0 + koff + i < K;  // (past K neither offset reaches the operand)
             v[Q][i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
                 r, (int)(in ? o : kOutOfRange), (int)(in ? s0 + (uint32_t)i * ld4 : 0u), 0));
         }
@@ -961,10 +963,11 @@ __global__ void __launch_bounds__(256) gemm_zero_counters_k(int* p, int n) {
 // (16 MFMAs per wave) and keep three slices in flight
 static constexpr int kDmaStages = 4;
 
-// Direct-to-LDS stream-K launch; OA / OB: KcOperand or XcOperand. At most one
-// round of 64x64 tiles over at most 8 slices (gemm_stays_fp32).
+// Direct-to-LDS stream-K launch; OA / OB: KcOperand or XcOperand. One round
+// of 64x64 tiles (plan_gemm_tiles): over a few slices on all resident
+// workgroups, over many on one per CU, whose whole tiles need no partials.
 template <class T, class OA, class OB>
-static void launch_gemm_dma(GemmArgs& g, int batches, const char* name, const char* kname) {
+static void launch_gemm_dma(GemmArgs& g, int batches, bool one_per_cu, const char* name, const char* kname) {
     constexpr int NS = kDmaStages;
     auto kernel = gemm_dma_k<T, NS, OA, OB, true>;
     const size_t lds = (size_t)GemmDma<T, NS>::LDS_FLOATS * sizeof(float);
@@ -982,7 +985,8 @@ static void launch_gemm_dma(GemmArgs& g, int batches, const char* name, const ch
     if ((int64_t)g.tiles_m * g.tiles_n * batches >= (1 << 30))
         return fail(NNC_HIP_EUNSUPP, name, "too many output tiles");
     const int iters = (int)ceil_div(g.K, T::BK);
-    const StreamK sk = plan_streamk(g.tiles_m * g.tiles_n * batches, iters, slots, fixup_slices<T>());
+    const StreamK sk = plan_streamk(g.tiles_m * g.tiles_n * batches, iters, one_per_cu ? std::min(slots, cu_count()) : slots,
+                                    fixup_slices<T>());
     if (sk.G < 1) return;
     const size_t ws_bytes = (size_t)sk.G * 2 * T::BM * T::BN * sizeof(float);
     g.ws = workspace(ws_bytes);
@@ -1002,21 +1006,21 @@ static void launch_gemm_dma(GemmArgs& g, int batches, const char* name, const ch
 }
 
 template <class T, bool A_KC, bool B_KC>
-static void launch_gemm_dma_kinds(GemmArgs& g, int batches, const char* name) {
+static void launch_gemm_dma_kinds(GemmArgs& g, int batches, bool one_per_cu, const char* name) {
     typedef typename std::conditional<A_KC, KcOperand<T, T::BM, 0>, XcOperand<T, T::BM, 0>>::type OA;
     typedef typename std::conditional<B_KC, KcOperand<T, T::BN, T::BM * 32>, XcOperand<T, T::BN, T::BM * 32>>::type
         OB;
     char kname[64];
     snprintf(kname, sizeof kname, "gemm_dma_%dx%d_%s%s", T::BM, T::BN, A_KC ? "k4" : "x4", B_KC ? "k4" : "x4");
-    launch_gemm_dma<T, OA, OB>(g, batches, name, kname);
+    launch_gemm_dma<T, OA, OB>(g, batches, one_per_cu, name, kname);
 }
 
 template <class T>
-static void dispatch_dma(GemmArgs& g, bool a_kc, bool b_kc, int batches, const char* name) {
-    if (a_kc && b_kc) return launch_gemm_dma_kinds<T, true, true>(g, batches, name);
-    if (a_kc) return launch_gemm_dma_kinds<T, true, false>(g, batches, name);
-    if (b_kc) return launch_gemm_dma_kinds<T, false, true>(g, batches, name);
-    return launch_gemm_dma_kinds<T, false, false>(g, batches, name);
+static void dispatch_dma(GemmArgs& g, bool a_kc, bool b_kc, int batches, bool one_per_cu, const char* name) {
+    if (a_kc && b_kc) return launch_gemm_dma_kinds<T, true, true>(g, batches, one_per_cu, name);
+    if (a_kc) return launch_gemm_dma_kinds<T, true, false>(g, batches, one_per_cu, name);
+    if (b_kc) return launch_gemm_dma_kinds<T, false, true>(g, batches, one_per_cu, name);
+    return launch_gemm_dma_kinds<T, false, false>(g, batches, one_per_cu, name);
 }
 
 // Shared tiles of the split kernel with at most this many partials are
@@ -1050,29 +1054,30 @@ static void launch_gemm_split(GemmArgs& g, int batches, const StreamK& sk, const
     }
 }
 
-template <class T, bool A_KC, bool B_KC, bool FULL>
+template <class T, bool A_KC, bool B_KC, KEnd END>
 static void launch_gemm_split_kinds(GemmArgs& g, int batches, const StreamK& sk, const char* name) {
-    typedef typename std::conditional<A_KC, KcSplit<T, T::BM, FULL>, XcSplit<T, T::BM, FULL>>::type OA;
-    typedef typename std::conditional<B_KC, KcSplit<T, T::BN, FULL>, XcSplit<T, T::BN, FULL>>::type OB;
+    typedef typename std::conditional<A_KC, KcSplit<T, T::BM, END>, XcSplit<T, T::BM, END>>::type OA;
+    typedef typename std::conditional<B_KC, KcSplit<T, T::BN, END>, XcSplit<T, T::BN, END>>::type OB;
     char kname[64];
     snprintf(kname, sizeof kname, "gemm_split_%dx%d_%s%s", T::BM, T::BN, A_KC ? "k" : "x", B_KC ? "k" : "x");
     launch_gemm_split<T, OA, OB>(g, batches, sk, name, kname);
 }
 
-template <class T, bool FULL>
-static void dispatch_split_full(GemmArgs& g, bool a_kc, bool b_kc, int batches, const StreamK& sk, const char* name) {
-    if (a_kc && b_kc) return launch_gemm_split_kinds<T, true, true, FULL>(g, batches, sk, name);
-    if (a_kc) return launch_gemm_split_kinds<T, true, false, FULL>(g, batches, sk, name);
-    if (b_kc) return launch_gemm_split_kinds<T, false, true, FULL>(g, batches, sk, name);
-    return launch_gemm_split_kinds<T, false, false, FULL>(g, batches, sk, name);
+template <class T, KEnd END>
+static void dispatch_split_end(GemmArgs& g, bool a_kc, bool b_kc, int batches, const StreamK& sk, const char* name) {
+    if (a_kc && b_kc) return launch_gemm_split_kinds<T, true, true, END>(g, batches, sk, name);
+    if (a_kc) return launch_gemm_split_kinds<T, true, false, END>(g, batches, sk, name);
+    if (b_kc) return launch_gemm_split_kinds<T, false, true, END>(g, batches, sk, name);
+    return launch_gemm_split_kinds<T, false, false, END == kEndSlice ? kEndSlice : kEndAny>(g, batches, sk, name);
 }
 
 template <class T>
 static void dispatch_split(GemmArgs& g, bool a_kc, bool b_kc, int batches, const StreamK& sk, const char* name) {
     g.tiles_m = (int)ceil_div(g.M, T::BM);
     g.tiles_n = (int)ceil_div(g.N, T::BN);
-    if (g.K % 32 == 0) return dispatch_split_full<T, true>(g, a_kc, b_kc, batches, sk, name);
-    return dispatch_split_full<T, false>(g, a_kc, b_kc, batches, sk, name);
+    if (g.K % 32 == 0) return dispatch_split_end<T, kEndSlice>(g, a_kc, b_kc, batches, sk, name);
+    if (g.K % 4 == 0) return dispatch_split_end<T, kEndQuad>(g, a_kc, b_kc, batches, sk, name);
+    return dispatch_split_end<T, kEndAny>(g, a_kc, b_kc, batches, sk, name);
 }
 
 template <int AK, int BKIND>
@@ -1433,11 +1438,12 @@ static void gemm_run(const GemmProblem& p, const char* name) {
     const int bkind = p.b_kc ? ((b_al && p.K % 4 == 0) ? kKC4 : kKC) : ((b_al && p.N % 4 == 0) ? kXC4 : kXC);
     const bool aligned = (akind == kKC4 || akind == kXC4) && (bkind == kKC4 || bkind == kXC4);
     const int64_t tiles64 = ceil_div(p.M, 64) * ceil_div(p.N, 64) * p.batches;
-    const int64_t iters = ceil_div(p.K, 32);
     // (an output row of 2 GiB or more: tiles that store through 64-bit addresses)
     const bool row64 = (int64_t)p.N * 4 >= ((int64_t)1 << 31);
-    if (row64 || gemm_stays_fp32(tiles64, iters, aligned, cu_count())) {
-        if (aligned) return dispatch_dma<GemmT64>(g, akind == kKC4, bkind == kKC4, p.batches, name);
+    if (tiles64 >= (1 << 30)) return fail(NNC_HIP_EUNSUPP, name, "too many output tiles");
+    const GemmTilePlan plan = plan_gemm_tiles(p.M, p.N, p.K, p.batches, aligned, cu_count());
+    if (row64 || plan.fp32) {
+        if (aligned) return dispatch_dma<GemmT64>(g, akind == kKC4, bkind == kKC4, p.batches, plan.one_per_cu, name);
         switch (akind) {
             case kKC4: return dispatch_b_small<kKC4>(g, bkind, p.batches, name);
             case kKC: return dispatch_b_small<kKC>(g, bkind, p.batches, name);
@@ -1458,16 +1464,9 @@ static void gemm_run(const GemmProblem& p, const char* name) {
         }
         return;
     }
-    if (tiles64 >= (1 << 30)) return fail(NNC_HIP_EUNSUPP, name, "too many output tiles");
-    // 64x64 and 128x64 tiles have registers for a second-level sum, which
-    // unaligned rows (formerly summed that way) keep; see split_tile.h
-    auto plan = [&](const SplitTileCost& c) {
-        return plan_split(c, ceil_div(p.M, c.bm) * ceil_div(p.N, c.bn) * p.batches, (int)iters, cu_count(), kGemmFinish);
-    };
-    const SplitPlan small = plan(kSplit64), big = plan(aligned ? kSplit128 : kSplit128x64);
-    if (small.us <= big.us) return dispatch_split<GemmT64>(g, p.a_kc, p.b_kc, p.batches, small.sk, name);
-    if (aligned) return dispatch_split<GemmT128>(g, p.a_kc, p.b_kc, p.batches, big.sk, name);
-    return dispatch_split<GemmT12864>(g, p.a_kc, p.b_kc, p.batches, big.sk, name);
+    if (plan.tile.bm == 64) return dispatch_split<GemmT64>(g, p.a_kc, p.b_kc, p.batches, plan.sk, name);
+    if (plan.tile.bn == 128) return dispatch_split<GemmT128>(g, p.a_kc, p.b_kc, p.batches, plan.sk, name);
+    return dispatch_split<GemmT12864>(g, p.a_kc, p.b_kc, p.batches, plan.sk, name);
 }
 
 static bool args_ok(const char* name, Tensor* a, Tensor* b, Tensor* out) {

@@ -197,41 +197,38 @@ inline bool plan_gemm_ws(int64_t M, int64_t N, int64_t K, int64_t batches, bool 
 constexpr int fixup_slices_for(int bm, int bn) { return (128 * 128) / (bm * bn); }
 
 // ---------------------------------------------------------------------------
-// Tile and schedule of the split kernels (split_tile.h). A tile shape's cost
-// per 32-k slice grows with the workgroups n that share a CU; the estimate of
-// a launch is its longest workgroup's slices at that price, plus finishing
-// the tiles where they are shared (SplitFinish; in the GEMM kernel its price
-// goes with the partials' bytes: 1024^3 split over 256 workgroups 22.2 us,
-// 2048^3 over 512 86 us against 73.6 whole). Prices measured on MI355X: 128x128 from Gemm 2048^3 (256
-// whole tiles, 73.6 us) and 4096^3 (two rounds of 512, 426 us); 64x64 from
-// 1024^3, 1536^3 and 2048^3 at 1 to 4 workgroups per CU; 64x256 from
-// ResNet-18's layer 1 at batch 12 and 32; 128x64 from 2048^3. What the
-// estimate decides, both sides measured: Gemm 2048x1024x256 64x64 12.3 us,
-// 128x128 15.8; 2048^3 102 and 73.6; 2000x2000x200 21.5 and 19.1; 3x3
-// convolutions at batch 32: 128 channels 28x28 as 128x128 tiles split 46.3 us,
-// whole 55.1; 256 channels 14x14 48 and 85; 1x1 256 -> 128 28x28 26.5 and 17.2;
-// layer 1 as 64x256 tiles whole 44.6, split 62.3, as 64x64 tiles 49.8 (batch
-// 12: 32.0, and 25.1 as 64x64). kConvFinish is below what a fixup launch
-// costs (about 12 us with its partials' traffic): at 196 tiles of 18 slices
-// (64 -> 128 channels, stride 2, batch 32) split and whole are 39 and 32 us,
-// and the launch table that the cost model shares has the fixup.
+// Tile and schedule of the split kernels (split_tile.h). The estimate of a
+// launch is its start, its longest workgroup's slices of 32 k at a price that
+// grows with the workgroups n that share a CU, an epilogue for each of that
+// workgroup's whole tiles, and, where tiles are shared, what finishing them
+// takes beside their partials' bytes. Prices in microseconds, fitted by least
+// squares to every tile shape at every n, tiles whole and shared, of 95
+// products and 43 convolutions on MI355X (the estimate's choice takes 1.03
+// times the best one's time for aligned products, 1.02 for others, 1.01 for
+// convolutions). What it decides, both sides measured: Gemm 2048^3 as 128x128
+// tiles 95 us, as 64x64 107; 2048x1024x256 as 64x64 13.9, as 128x128 15.8;
+// 1024x768x1024 64x64 at three per CU shared 24.3, whole 27; 3x3 convolutions
+// at batch 32: 64 channels 56x56 as 64x256 whole 57, shared 68; 64 -> 128
+// stride 2 as 128x128 whole 36, shared 40; 128 channels 28x28 shared 58, whole
+// 61; 1x1 256 -> 128 28x28 whole 20.4.
 // ---------------------------------------------------------------------------
 struct SplitTileCost {
     int bm, bn, max_per_cu;
-    double us[4];   // per slice, at 1..max_per_cu workgroups per CU
-    double shared;  // more for tiles that are shared
+    double start, tile;  // a launch; a workgroup's whole tile beside its slices
+    double us[4];        // a slice, at 1..max_per_cu workgroups per CU
+    double shared[4];    // more for shared tiles
+    double per_mb, per_part;
 };
-constexpr SplitTileCost kSplit128 = {128, 128, 2, {1.02, 1.63, 0, 0}, 0};
-constexpr SplitTileCost kSplit64x256 = {64, 256, 2, {1.25, 1.90, 0, 0}, 20};
-constexpr SplitTileCost kSplit128x64 = {128, 64, 3, {0.80, 1.14, 1.71, 0}, 0};
-constexpr SplitTileCost kSplit64 = {64, 64, 4, {0.65, 0.77, 1.10, 1.48}, 0};
-
-// What finishing shared tiles adds (microseconds): per partial of a tile, per
-// MB of partials written.
-struct SplitFinish {
-    double base, per_part, per_mb;
-};
-constexpr SplitFinish kConvFinish = {2.5, 1.0, 0.0}, kGemmFinish = {3.0, 0.0, 0.35};
+constexpr SplitTileCost kGemm64 = {64, 64, 4, 3.7, 3.6, {0.68, 0.92, 1.38, 2.17}, {8.7, 8.1, 5.7, 6.5}, 0.40, 0};
+constexpr SplitTileCost kGemm128 = {128, 128, 2, 3.8, 7.1, {1.27, 2.54, 0, 0}, {10.6, 5.4, 0, 0}, 0.40, 0};
+// rows off 16-byte boundaries, or K or N no multiple of 4
+constexpr SplitTileCost kGemm64u = {64, 64, 4, 2.2, 4.1, {0.84, 1.15, 1.56, 2.46}, {12.1, 12.9, 14.2, 16.6}, 0.05, 0};
+constexpr SplitTileCost kGemm128x64u = {128, 64, 3, 3.7, 5.3, {1.15, 1.71, 3.58, 0}, {16.9, 15.8, 14.0, 0}, 0.05, 0};
+// the fp32 instruction on 64x64 tiles (gemm_dma_k), one workgroup per CU
+constexpr SplitTileCost kGemmFp32 = {64, 64, 1, 3.9, 2.8, {0.61, 0, 0, 0}, {6.5, 0, 0, 0}, 0.40, 0};
+constexpr SplitTileCost kConv64 = {64, 64, 4, 4.6, 2.3, {0.79, 1.06, 1.38, 2.37}, {5.5, 3.7, 3.9, 0.9}, 0.37, 0.16};
+constexpr SplitTileCost kConv128 = {128, 128, 2, 4.1, 5.4, {1.39, 2.51, 0, 0}, {5.8, 1.6, 0, 0}, 0.37, 0.16};
+constexpr SplitTileCost kConv64x256 = {64, 256, 2, 4.9, 5.1, {1.85, 2.97, 0, 0}, {4.9, 1.9, 0, 0}, 0.37, 0.16};
 
 struct SplitPlan {
     StreamK sk;
@@ -244,31 +241,32 @@ inline int64_t split_parts(const StreamK& sk) {
     return per > 0 ? (sk.iters + per - 1) / per + 1 : sk.iters;
 }
 
-inline double split_estimate(const SplitTileCost& c, const StreamK& sk, int cus, const SplitFinish& f) {
-    auto price = [&](int64_t groups) {
-        int64_t n = (groups + cus - 1) / cus;
-        return c.us[(n < 1 ? 1 : n > c.max_per_cu ? c.max_per_cu : n) - 1];
+inline double split_estimate(const SplitTileCost& c, const StreamK& sk, int cus) {
+    auto at = [&](int64_t groups) {
+        const int64_t n = (groups + cus - 1) / cus;
+        return (n < 1 ? 1 : n > c.max_per_cu ? c.max_per_cu : n) - 1;
     };
     const int64_t whole = sk.tiles - sk.sk_tiles;
     const int64_t full = whole / sk.G, rem = whole % sk.G;
-    double us = (double)full * sk.iters * price(sk.G) + (rem ? sk.iters * price(rem) : 0.0);
-    if (sk.sk_tiles) us += (double)((sk.total() + sk.G - 1) / sk.G) * price(sk.G);
+    double us = c.start + c.tile * (double)(full + (rem != 0));
+    us += (double)full * sk.iters * c.us[at(sk.G)] + (rem ? sk.iters * c.us[at(rem)] : 0.0);
+    if (sk.sk_tiles) us += (double)((sk.total() + sk.G - 1) / sk.G) * c.us[at(sk.G)];
     if (sk.needs_fixup())
-        us += f.base + c.shared + f.per_part * (double)split_parts(sk) +
-              f.per_mb * ((double)sk.G + sk.sk_tiles) * c.bm * c.bn * 4e-6;
+        us += c.shared[at(sk.G)] + c.per_part * (double)split_parts(sk) +
+              c.per_mb * ((double)sk.G + sk.sk_tiles) * c.bm * c.bn * 4e-6;
     return us;
 }
 
 // The cheapest schedule of `tiles` tiles of `iters` slices on 1 to max_per_cu
 // workgroups per CU, tiles whole or shared.
-inline SplitPlan plan_split(const SplitTileCost& c, int64_t tiles, int iters, int cus, const SplitFinish& f) {
+inline SplitPlan plan_split(const SplitTileCost& c, int64_t tiles, int iters, int cus) {
     SplitPlan best{};
     best.us = 1e30;
     for (int n = 1; n <= c.max_per_cu; ++n)
         for (int whole = 0; whole < 2; ++whole) {
             const StreamK sk = plan_streamk((int)tiles, iters, n * cus, whole ? 1 << 20 : 0);
             if (sk.G < 1) continue;
-            const double us = split_estimate(c, sk, cus, f);
+            const double us = split_estimate(c, sk, cus);
             if (us < best.us) best = SplitPlan{sk, us};
         }
     return best;
@@ -278,25 +276,53 @@ inline SplitPlan plan_split(const SplitTileCost& c, int64_t tiles, int iters, in
 struct ConvSplitPlan {
     SplitTileCost tile;
     StreamK sk;
+    double us;
 };
 inline ConvSplitPlan plan_conv_split(int64_t Co, int64_t Npix, int64_t K, int cus) {
     auto plan = [&](const SplitTileCost& c) {
-        return plan_split(c, ((Co + c.bm - 1) / c.bm) * ((Npix + c.bn - 1) / c.bn), (int)(K / 32), cus, kConvFinish);
+        return plan_split(c, ((Co + c.bm - 1) / c.bm) * ((Npix + c.bn - 1) / c.bn), (int)(K / 32), cus);
     };
-    const SplitTileCost& large = Co <= 64 ? kSplit64x256 : kSplit128;
-    const SplitPlan a = plan(kSplit64), b = plan(large);
-    return a.us <= b.us ? ConvSplitPlan{kSplit64, a.sk} : ConvSplitPlan{large, b.sk};
+    const SplitTileCost& large = Co <= 64 ? kConv64x256 : kConv128;
+    const SplitPlan a = plan(kConv64), b = plan(large);
+    return a.us <= b.us ? ConvSplitPlan{kConv64, a.sk, a.us} : ConvSplitPlan{large, b.sk, b.us};
 }
 
-// Products that stay on the fp32 matrix instruction: one round of 64x64
-// tiles over a few slices. The kernel's start, not its products, is what
-// takes the time there, and cutting the operands lengthens it
-// ([64,128,64] x [64,64,128] 6.9 us, split 7.0; unaligned [30,71,71] x [71,32]
-// 7.3 and 7.7; beyond: unaligned 1001x999x333 23.9 and 13.7, aligned
-// 1024x768x1024 27.9 and 22.7). Over one or two slices a few rounds more do
-// ([24,247,25] x [24,25,242] 6.4 and 7.9; 1799x1057x45 8.1 and 9.2).
+// Products that stay on the fp32 matrix instruction whatever the estimate:
+// one round of 64x64 tiles over a few slices. The kernel's start, not its
+// products, is what takes the time there, and cutting the operands lengthens
+// it ([64,128,64] x [64,64,128] 6.9 us, split 7.0; unaligned [30,71,71] x
+// [71,32] 7.3 and 7.7; beyond: unaligned 1001x999x333 24 and 15). Over one or
+// two slices a few rounds more do ([24,247,25] x [24,25,242] 6.4 and 7.9;
+// 1862x2348x41 16.8 and 17.5).
 inline bool gemm_stays_fp32(int64_t tiles64, int64_t iters, bool aligned, int cus) {
-    return tiles64 <= cus ? iters <= (aligned ? 8 : 4) : iters <= 2 && tiles64 <= 4 * cus;
+    return tiles64 <= cus ? iters <= (aligned ? 8 : 4) : iters <= 2 && tiles64 <= (aligned ? 4 : 5) * cus;
+}
+
+// Tiles of a product that no other kernel takes. `aligned`: 16-byte rows on
+// both sides. Unaligned rows keep a second-level sum (they were summed that
+// way before), for which 64x64 and 128x64 tiles have registers.
+struct GemmTilePlan {
+    SplitTileCost tile;
+    bool fp32;     // gemm_dma_k (aligned) or gemm_streamk_k
+    bool one_per_cu;  // gemm_dma_k on one workgroup per CU, else all resident ones
+    StreamK sk;    // of the split kernels
+    double us;
+};
+inline GemmTilePlan plan_gemm_tiles(int64_t M, int64_t N, int64_t K, int64_t batches, bool aligned, int cus) {
+    const int iters = (int)((K + 31) / 32);
+    auto tiles = [&](const SplitTileCost& c) { return ((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn) * batches; };
+    if (gemm_stays_fp32(tiles(kGemmFp32), iters, aligned, cus)) return GemmTilePlan{kGemmFp32, true, false, StreamK{}, 0.0};
+    const SplitTileCost &s = aligned ? kGemm64 : kGemm64u, &l = aligned ? kGemm128 : kGemm128x64u;
+    const SplitPlan a = plan_split(s, tiles(s), iters, cus), b = plan_split(l, tiles(l), iters, cus);
+    GemmTilePlan p = a.us <= b.us ? GemmTilePlan{s, false, false, a.sk, a.us} : GemmTilePlan{l, false, false, b.sk, b.us};
+    if (aligned && tiles(kGemmFp32) <= cus) {
+        // within one round the fp32 tiles need no cutting: 495x320x3072 22.0
+        // us, split 25.0; 355x2592x1152 27.7 and 29.9; but 478x928x2496 35 and 28
+        const StreamK sk = plan_streamk((int)tiles(kGemmFp32), iters, cus, fixup_slices_for(64, 64));
+        const double us = split_estimate(kGemmFp32, sk, cus);
+        if (us < p.us) p = GemmTilePlan{kGemmFp32, true, true, sk, us};
+    }
+    return p;
 }
 
 }  // namespace nnc

@@ -155,22 +155,26 @@ struct SplitStaged {
     }
 };
 
+// How the last 16-k steps of an operand end: K a multiple of 32, of 4, any.
+enum KEnd { kEndSlice, kEndQuad, kEndAny };
+
 // An operand with rows contiguous in k: element (x, k) at base[x*ld + k], rows
 // of any alignment (buffer loads need 4-byte alignment only). Four lanes
 // load a row's 64 bytes of a step, so an instruction touches 16 whole
 // 64-byte pieces; with two lanes per row and 8 k per lane it touched 32
 // half-used ones, twice the L1 accesses (522 per 128x128 step against a step
-// of 384 MFMA cycles). FULL: K is a multiple of 32; otherwise the last steps
-// load their k < K 4 bytes at a time (16 bytes over a row's end would read
-// the next row, and past the matrix in its last).
-template <class T, int X, bool FULL>
+// of 384 MFMA cycles). kEndQuad: a lane's four k are all inside or all past
+// K, a select on its offset; kEndAny: the last steps load their k < K 4 bytes
+// at a time (16 bytes over a row's end would read the next row, and past the
+// matrix in its last) behind a branch in each step.
+template <class T, int X, KEnd END>
 struct KcSplit : SplitStaged<T, X, 4> {
     typedef SplitStaged<T, X, 4> S;
     using S::koff;
     using S::NG;
     using S::v;
     using S::x;
-    static constexpr bool BRANCH = !FULL;
+    static constexpr bool BRANCH = END == kEndAny;
     static __device__ __forceinline__ int64_t origin(int x0, int64_t ld) { return (int64_t)x0 * ld; }
     __amdgpu_buffer_rsrc_t r;
     uint32_t vo[NG];  // byte offsets of this thread's rows at its first k, or kOutOfRange
@@ -188,10 +192,11 @@ struct KcSplit : SplitStaged<T, X, 4> {
     }
     template <int Q>
     __device__ __forceinline__ void load(int k0, int K, bool on) {
+        const bool in = END == kEndQuad ? on & (k0 + koff < K) : on;
 #pragma unroll
         for (int g = 0; g < NG; ++g) {
-            const uint32_t o = on ? vo[g] : kOutOfRange;
-            if (FULL || k0 + 16 <= K) {
+            const uint32_t o = in ? vo[g] : kOutOfRange;
+            if (END != kEndAny || k0 + 16 <= K) {
                 const f32x4 q = __builtin_bit_cast(
                     f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)o, (int)((uint32_t)k0 * 4u), 0));
                 v[Q][4 * g] = q[0], v[Q][4 * g + 1] = q[1], v[Q][4 * g + 2] = q[2], v[Q][4 * g + 3] = q[3];
