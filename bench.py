@@ -43,16 +43,24 @@ ROOT = Path(__file__).resolve().parent
 METRIC = "ResNet-18 fp32 images/s (b1,b32) on 1 GPU; per-op % HBM/MFMA roofline"
 PEAK_HBM_GBS = 8000.0      # MI355X HBM3E
 PEAK_FP32_MFMA_TF = 157.3  # MI355X dense fp32 matrix
-PEAK_SPLIT_TF = 2500.0 / 3  # fp32 products as three f16 products each (csrc/split_tile.h)
+PEAK_SPLIT_TF = 2500.0 / 6  # fp32 products as six bf16 products each (csrc/split_tile.h)
 # kernel-table names of the MFMA kernels (their work is priced in FLOP)
 MFMA_KERNELS = ("conv_igemm", "conv_stem", "conv_ws", "gemm_mfma", "gemm_split", "gemm_dma", "gemm_skinny", "gemm_ws", "attention")
 
 
 def mfma_peak(name: str) -> float:
     """Peak of the matrix instruction a kernel of the timing table uses, in
-    fp32 products."""
-    split = name.startswith("gemm_split") or (name.startswith("conv_igemm") and name.endswith("_dma") and "c3" not in name)
+    fp32 products: the split tiles and the short kernels in pieces (_b16) run
+    on the 16-bit instruction, the others on the fp32 one."""
+    split = (name.startswith("gemm_split") or name.endswith("_b16")
+             or (name.startswith("conv_igemm") and name.endswith("_dma") and "c3" not in name))
     return PEAK_SPLIT_TF if split else PEAK_FP32_MFMA_TF
+
+
+def mfma_frac(rows: list, ms: float) -> float | None:
+    """Share of `ms` that the rows' products would take at the peaks of their
+    own instructions."""
+    return round(sum(r["frac"] * r["ms_per_step"] for r in rows if r["bound"] == "mfma") / ms, 4) if ms else None
 
 
 def load_package():
@@ -217,7 +225,7 @@ def kernel_table(ex, runtime, steps: int) -> list[dict]:
         elif r["name"].endswith("_fixup"):
             # stream-K partial-tile reduction: no algorithmic work of its own,
             # its time counts against the MFMA kernels it completes
-            bound, unit, peak = "mfma-fixup", "TFLOP/s", PEAK_FP32_MFMA_TF
+            bound, unit, peak = "mfma-fixup", "TFLOP/s", PEAK_SPLIT_TF
             achieved = 0.0
         else:
             bound, unit, peak = "hbm", "GB/s", PEAK_HBM_GBS
@@ -320,6 +328,15 @@ def conv_symbol_pattern(name: str) -> re.Pattern | None:
     if m:
         kernel = "conv_stem_k" if m.group(1) == "rows" else "conv_stem_pool_k"
         return re.compile(rf"{kernel}<{int(m.group(2)) // 16}>")
+    m = re.fullmatch(r"conv_igemm_32x32_k(\d+)x(\d+)(_b16)?", name)
+    if m:
+        return re.compile(rf"conv_wss_k<\d+, (true|false), {'true' if m.group(3) else 'false'}>")
+    m = re.fullmatch(r"conv_ws_32x32_k(\d+)x(\d+)(p?)(_b16)?", name)
+    if m:
+        return re.compile(rf"conv_ws_k<\d+, {'true' if m.group(3) else 'false'}, {'true' if m.group(4) else 'false'}>")
+    m = re.fullmatch(r"gemm_split_(\d+)x(\d+)_\w+", name)
+    if m:
+        return re.compile(rf"gemm_split_k<nnc::Tile<{m.group(1)}, {m.group(2)},")
     m = re.fullmatch(r"gemm_mfma_(\d+)x(\d+)_\w+", name)
     if m:
         return re.compile(rf"gemm_streamk_k<nnc::Tile<{m.group(1)}, {m.group(2)},")
@@ -639,9 +656,10 @@ def run_suite() -> int:
     dt = timed_steps(ex, steps, 10, True, runtime)
     ms = dt / steps * 1e3
     flops = zoo.transformer_flops()
-    emit("transformer", "encoder 2 layers, B8 S128 D256 H4 FFN1024, O3, hipGraph", {"kernels": kernel_table(ex, runtime, 5)},
+    rows = kernel_table(ex, runtime, 5)
+    emit("transformer", "encoder 2 layers, B8 S128 D256 H4 FFN1024, O3, hipGraph", {"kernels": rows},
          ms_per_step=round(ms, 4), gflops_per_s=round(flops / (ms * 1e-3) / 1e9, 1),
-         mfma_frac_whole_step=round(flops / (ms * 1e-3) / 1e12 / PEAK_FP32_MFMA_TF, 4))
+         mfma_frac_whole_step=mfma_frac(rows, ms))
     ex.close()
     return 0
 
@@ -768,8 +786,6 @@ def main() -> int:
         roofline["traffic_detail"] = {k: {kk: round(vv, 4) for kk, vv in v.items()} for k, v in traffic_detail.items()}
     gpu_ms = sum(r["ms_per_step"] for r in table)
     conv_ms = sum(r["ms_per_step"] for r in table if r["bound"] in ("mfma", "mfma-fixup"))
-    conv_flops = zoo.resnet18_flops(args.batch)
-
     cpu = None
     if not args.skip_cpu:
         log(f"CPU baseline: ResNet-18 batch 1 ({args.cpu_iters} timed runs) and batch {args.batch} "
@@ -795,7 +811,7 @@ def main() -> int:
         "b1": ({"images_per_s": round(results[1]["images_per_s"], 2),
                 "ms_per_step": round(results[1]["ms_per_step"], 4)} if 1 in results else None),
         "roofline": roofline,
-        "mfma_frac_all_conv": round(conv_flops / (conv_ms * 1e-3) / 1e12 / PEAK_FP32_MFMA_TF, 4) if conv_ms else None,
+        "mfma_frac_all_conv": mfma_frac(table, conv_ms),
         "kernel_ms_per_step": round(gpu_ms, 4),
         "per_kernel": [{k: r[k] for k in ("kernel", "launches_per_step", "avg_us", "bound", "achieved", "unit", "frac")}
                        for r in table],

@@ -1628,10 +1628,11 @@ static bool launch_conv_ws(ConvArgs& a, const char* entry) {
                    (int)tiles);
     }
     char name[64];
+    const char* pieces = wp.pieces ? "_b16" : "";
     if (KIND >= kWsStored)
-        snprintf(name, sizeof name, "conv_igemm_32x32_k%dx%d", a.kh, a.kw);
+        snprintf(name, sizeof name, "conv_igemm_32x32_k%dx%d%s", a.kh, a.kw, pieces);
     else
-        snprintf(name, sizeof name, "conv_ws_32x32_k%dx%d%s", a.kh, a.kw, KIND == kWsProj ? "p" : "");
+        snprintf(name, sizeof name, "conv_ws_32x32_k%dx%d%s%s", a.kh, a.kw, KIND == kWsProj ? "p" : "", pieces);
     set_work(2.0 * a.Co * (double)a.Npix * a.K, 0.0);
     const unsigned grid = (unsigned)(tiles * S);
     switch (wp.NS) {

@@ -58,21 +58,17 @@ struct MfmaKind {
     int bm, bn, per_cu;  // tile, resident workgroups per CU
     double eff, lat_us;  // main loop: fraction of a CU's MFMA rate, slice latency alone
 };
-// Fitted to 97 launches of ResNet-18 at batch 1, 8 and 32 (rocprofv3 kernel
-// trace, hipGraph replay; rms error 11% per launch, 2-6% per step).
-// direct-to-LDS conv kernels (packed 3x3 / 1x1), the 3-channel stem; the
-// register-staged conv kernels (reference-layout weights) and GEMM tiles
-// are priced like the direct-to-LDS ones of their tile shape, the gather
-// kernels 20% slower.
-const MfmaKind kConv128 = {"conv_dma_128", 128, 128, 2, 0.75, 0.47};
-const MfmaKind kConv64x128 = {"conv_dma_64x128", 64, 128, 3, 0.65, 4.0};
-const MfmaKind kConv64 = {"conv_dma_64", 64, 64, 4, 0.60, 1.0};
+// The kernels on the fp32 instruction, stream-K over 64x64 to 128x128 tiles:
+// the 3-channel stem's tiles, reference-layout weights (gather), one round of
+// product tiles. Efficiencies fitted to launches of ResNet-18 at batch 1, 8
+// and 32 (rocprofv3 kernel trace, hipGraph replay; rms error 11% per launch);
+// the gather kernels 20% slower than direct-to-LDS ones of their tile shape.
+// The split kernels take plan.h's own estimate.
 const MfmaKind kStem64x128 = {"stem_64x128", 64, 128, 3, 0.50, 1.26};  // with the in-kernel finish
 const MfmaKind kStem64 = {"stem_64", 64, 64, 4, 0.30, 1.43};
 const MfmaKind kGather128 = {"conv_gather_128", 128, 128, 2, 0.60, 0.6};
 const MfmaKind kGather64x128 = {"conv_gather_64x128", 64, 128, 3, 0.52, 4.0};
 const MfmaKind kGather64 = {"conv_gather_64", 64, 64, 4, 0.48, 1.2};
-const MfmaKind kGemm128 = {"gemm_128", 128, 128, 2, 0.75, 0.47};  // direct-to-LDS, two stages
 const MfmaKind kGemmDma64 = {"gemm_dma_64", 64, 64, 2, 0.60, 1.0};  // direct-to-LDS, four stages
 const MfmaKind kGemm64 = {"gemm_64", 64, 64, 4, 0.60, 1.0};         // register-staged
 // the stem's row kernel (input window in LDS): fraction of a CU's MFMA rate
@@ -195,8 +191,8 @@ MfmaResult mfma_kernel(const MfmaKind& k, int tiles, int64_t K, double hbm_bytes
 
 // finishing shared tiles: the fixup kernel reads every partial tile and
 // writes the finished tiles
-double fixup_us(const MfmaKind& k, const nnc::StreamK& sk) {
-    const double bytes = (2.0 * sk.G + sk.sk_tiles) * k.bm * k.bn * 4;
+double fixup_us(int bm, int bn, const nnc::StreamK& sk) {
+    const double bytes = (2.0 * sk.G + sk.sk_tiles) * bm * bn * 4;
     const double parts = (double)sk.G / (sk.sk_tiles > 0 ? sk.sk_tiles : 1) + 1.0;
     return kLaunchUs + kFixupUsPerMB * bytes * 1e-6 + kFixupUsPerPart * parts;
 }
@@ -209,8 +205,9 @@ bool ws_kernel(const char* op, int kh, int kw, const char* kind, int64_t Co, int
     nnc::WsPlan p;
     if (!(*kind == 's' ? nnc::plan_ws_stored(Co, npix, K, p) : nnc::plan_ws(Co, npix, K, p))) return false;
     char name[64];
-    if (*kind == 's') snprintf(name, sizeof name, "conv_igemm_32x32_k%dx%d", kh, kw);
-    else snprintf(name, sizeof name, "conv_ws_32x32_k%dx%d%s", kh, kw, kind);
+    const char* pieces = p.pieces ? "_b16" : "";
+    if (*kind == 's') snprintf(name, sizeof name, "conv_igemm_32x32_k%dx%d%s", kh, kw, pieces);
+    else snprintf(name, sizeof name, "conv_ws_32x32_k%dx%d%s%s", kh, kw, kind, pieces);
     const int r = (int)ceil_div(p.tiles * p.S, kCUs);  // workgroups sharing a CU
     double us = kLaunchUs + r * p.NS * kWsSliceUs + kColdUsPerMB * weight_bytes * 1e-6;
     if (p.S > 1) us += kWsFinishUs + kWsFinishUsPerPart * p.S;
@@ -221,23 +218,22 @@ bool ws_kernel(const char* op, int kh, int kw, const char* kind, int64_t Co, int
 
 constexpr int kMaxInKernelParts = 4;
 
-// conv.hip conv_split, named by the library's tile. Schedule, fixup launches
-// and prices are those of the fp32-MFMA tiles whose measured times the model
-// is fitted to: an upper bound for the library's split kernels.
+// A split kernel (split_tile.h): the library's own estimate of the schedule
+// that it picks, of which the fixup launch, if there is one, takes its part.
+void split_kernel(const char* op, const char* name, const char* fixup, const nnc::SplitTileCost& tile,
+                  const nnc::StreamK& sk, double us, double flops, double bytes) {
+    const double after = fixup ? fixup_us(tile.bm, tile.bn, sk) : 0.0;
+    record(op, name, fmax(us - after, kLaunchUs + bytes / (kHbm * kStreamEff) * 1e6), flops, bytes);
+    if (fixup) record(op, fixup, after, 0.0, 0.0);
+}
+
+// conv.hip conv_split
 void split_conv(const char* op, int kh, int kw, bool proj, int64_t Co, int64_t npix, int64_t K, double flops,
-                double bytes, double weight_bytes) {
-    const nnc::SplitTileCost tile = nnc::plan_conv_split(Co, npix, K, kCUs).tile;
+                double bytes) {
+    const nnc::ConvSplitPlan p = nnc::plan_conv_split(Co, npix, K, kCUs);
     char name[64];
-    snprintf(name, sizeof name, "conv_igemm_%dx%d_k%dx%d%s_dma", tile.bm, tile.bn, kh, kw, proj ? "p" : "");
-    const MfmaKind& k = (K >= 512 && Co >= 128 && npix >= 1024) ? kConv128
-                        : (K >= 512 && Co <= 64 && npix >= 4096) ? kConv64x128 : kConv64;
-    const int tiles = (int)(ceil_div(Co, k.bm) * ceil_div(npix, k.bn));
-    MfmaResult m = mfma_kernel(k, tiles, K, bytes, weight_bytes);
-    record(op, name, m.us, flops, bytes);
-    if (!m.sk.needs_fixup()) return;
-    const int64_t per = m.sk.total() / m.sk.G;
-    if (&k == &kConv64x128 && (m.sk.iters + per - 1) / per + 1 <= kMaxInKernelParts) return;
-    record(op, "conv_streamk_fixup", fixup_us(k, m.sk), 0.0, 0.0);
+    snprintf(name, sizeof name, "conv_igemm_%dx%d_k%dx%d%s_dma", p.tile.bm, p.tile.bn, kh, kw, proj ? "p" : "");
+    split_kernel(op, name, p.sk.needs_fixup() ? "conv_streamk_fixup" : nullptr, p.tile, p.sk, p.us, flops, bytes);
 }
 
 // ---------------------------------------------------------------------------
@@ -255,7 +251,7 @@ void conv(const char* op, Tensor* in, Tensor* w, Tensor* b, Tensor* res, Tensor*
     const double bytes = nbytes(in) + nbytes(w) + nbytes(b) + nbytes(out) + (res ? nbytes(res) : 0.0);
     const bool stem = packed && w->ndim == 2;
     const bool dma_ok = Ci % 32 == 0 && ((kh == 3 && kw == 3) || (kh == 1 && kw == 1));
-    bool dma = dma_ok && (packed || (kh == 1 && kw == 1));
+    bool dma = dma_ok && K > 0 && (packed || (kh == 1 && kw == 1));
     if (dma_ok && !packed && kh == 3 && flops >= kRepackMinFlops) {
         stream_kernel(op, "conv_repack_taps", 8.0 * Co * K);
         dma = true;
@@ -279,7 +275,7 @@ void conv(const char* op, Tensor* in, Tensor* w, Tensor* b, Tensor* res, Tensor*
     } else {
         if ((dma || kh * kw < 64) && ws_kernel(op, kh, kw, dma ? "" : "s", Co, npix, K, flops, bytes, nbytes(w))) return;
         const int tile = (K >= 512 && Co >= 128 && npix >= 1024) ? 2 : (K >= 512 && Co <= 64 && npix >= 4096) ? 1 : 0;
-        if (dma) return split_conv(op, kh, kw, false, Co, npix, K, flops, bytes, nbytes(w));
+        if (dma) return split_conv(op, kh, kw, false, Co, npix, K, flops, bytes);
         {
             k = tile == 2 ? &kGather128 : tile == 1 ? &kGather64x128 : &kGather64;
             const bool known = (kh == 1 && kw == 1) || (kh == 3 && kw == 3) || (kh == 7 && kw == 7);
@@ -299,7 +295,7 @@ void conv(const char* op, Tensor* in, Tensor* w, Tensor* b, Tensor* res, Tensor*
     const int64_t per = m.sk.total() / m.sk.G;
     // (its cost is inside the kernel's fitted efficiency)
     if (fin && (m.sk.iters + per - 1) / per + 1 <= kMaxInKernelParts) return;
-    record(op, "conv_streamk_fixup", fixup_us(*k, m.sk), 0.0, 0.0);
+    record(op, "conv_streamk_fixup", fixup_us(k->bm, k->bn, m.sk), 0.0, 0.0);
 }
 
 // ---------------------------------------------------------------------------
@@ -364,39 +360,34 @@ void gemm(const char* op, int M, int N, int K, int batches, bool a_kc, bool b_kc
     }
     const bool a4 = a_kc ? K % 4 == 0 : M % 4 == 0;  // 16-byte loads along the contiguous axis
     const bool b4 = b_kc ? K % 4 == 0 : N % 4 == 0;
-    const bool big = (int64_t)M * N * batches >= (int64_t)128 * 128 * 2 * kCUs / 4 && M >= 128 && N >= 128;
     static const char* kinds[4] = {"k4", "k1", "x4", "x1"};
     const int ak = a_kc ? (a4 ? 0 : 1) : (a4 ? 2 : 3), bk = b_kc ? (b4 ? 0 : 1) : (b4 ? 2 : 3);
     char name[64];
-    const bool fp32 = nnc::gemm_stays_fp32(ceil_div(M, 64) * ceil_div(N, 64) * batches, ceil_div(K, kBK), a4 && b4, kCUs);
-    if (!fp32) {
-        // gemm.hip's split kernels, priced as the fp32-MFMA tiles
-        const MfmaKind& k = a4 && b4 && big ? kGemm128 : kGemm64;
-        snprintf(name, sizeof name, "gemm_split_%dx%d_%s%s", k.bm, k.bn, a_kc ? "k" : "x", b_kc ? "k" : "x");
-        const int tiles = (int)(ceil_div(M, k.bm) * ceil_div(N, k.bn) * batches);
-        return record(op, name, mfma_kernel(k, tiles, K, bytes, b_bytes).us, flops, bytes);
+    const nnc::GemmTilePlan p = nnc::plan_gemm_tiles(M, N, K, batches, a4 && b4, kCUs);
+    if (!p.fp32) {
+        snprintf(name, sizeof name, "gemm_split_%dx%d_%s%s", p.tile.bm, p.tile.bn, a_kc ? "k" : "x", b_kc ? "k" : "x");
+        const bool fixup = p.sk.needs_fixup() && nnc::split_parts(p.sk) > nnc::kSplitInKernelParts;
+        return split_kernel(op, name, fixup ? "gemm_streamk_fixup" : nullptr, p.tile, p.sk, p.us, flops, bytes);
     }
     if (a4 && b4) {
-        // direct-to-LDS: 128x128 or 64x64 tiles (one workgroup per CU over
-        // 16 or more K slices); shared tiles of at most four partials are
+        // direct-to-LDS 64x64 tiles; shared tiles of at most four partials are
         // finished in-kernel
-        const MfmaKind& k = big ? kGemm128 : kGemmDma64;
+        const MfmaKind& k = kGemmDma64;
         snprintf(name, sizeof name, "gemm_dma_%dx%d_%s%s", k.bm, k.bn, kinds[ak], kinds[bk]);
         const int tiles = (int)(ceil_div(M, k.bm) * ceil_div(N, k.bn) * batches);
-        const int iters = (int)ceil_div(K, kBK);
-        MfmaResult m = mfma_kernel(k, tiles, K, bytes, b_bytes, !big && iters >= 16 ? kCUs : 0);
+        MfmaResult m = mfma_kernel(k, tiles, K, bytes, b_bytes, p.one_per_cu ? kCUs : 0);
         record(op, name, m.us, flops, bytes);
         if (!m.sk.needs_fixup()) return;
         const int64_t per = m.sk.total() / m.sk.G;
         if ((m.sk.iters + per - 1) / per + 1 <= kMaxInKernelParts) return;
-        return record(op, "gemm_streamk_fixup", fixup_us(k, m.sk), 0.0, 0.0);
+        return record(op, "gemm_streamk_fixup", fixup_us(k.bm, k.bn, m.sk), 0.0, 0.0);
     }
     const MfmaKind& k = kGemm64;
     snprintf(name, sizeof name, "gemm_mfma_%dx%d_%s%s", k.bm, k.bn, kinds[ak], kinds[bk]);
     const int tiles = (int)(ceil_div(M, k.bm) * ceil_div(N, k.bn) * batches);
     MfmaResult m = mfma_kernel(k, tiles, K, bytes, b_bytes);
     record(op, name, m.us, flops, bytes);
-    if (m.sk.needs_fixup()) record(op, "gemm_streamk_fixup", fixup_us(k, m.sk), 0.0, 0.0);
+    if (m.sk.needs_fixup()) record(op, "gemm_streamk_fixup", fixup_us(k.bm, k.bn, m.sk), 0.0, 0.0);
 }
 
 void matmul(const char* op, Tensor* a, Tensor* b, Tensor* bias, Tensor* out) {
@@ -601,7 +592,7 @@ void nnc_hip_conv_proj(Tensor* in, Tensor* w, Tensor* b, Tensor* x, Tensor* out,
     const double flops = 2.0 * Co * (double)npix * K;
     const double bytes = nbytes(in) + nbytes(x) + nbytes(w) + nbytes(b) + nbytes(out);
     if (ws_kernel(op, 3, 3, "p", Co, npix, K, flops, bytes, nbytes(w))) return;
-    split_conv(op, 3, 3, true, Co, npix, K, flops, bytes, nbytes(w));
+    split_conv(op, 3, 3, true, Co, npix, K, flops, bytes);
 }
 void nnc_hip_conv_packed(Tensor* in, Tensor* w, Tensor* b, Tensor* res, Tensor* out, int kh, int kw, int sh, int sw,
                          int ph, int pw, int act) {

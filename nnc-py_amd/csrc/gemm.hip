@@ -1023,10 +1023,6 @@ static void dispatch_dma(GemmArgs& g, bool a_kc, bool b_kc, int batches, bool on
     return launch_gemm_dma_kinds<T, false, false>(g, batches, one_per_cu, name);
 }
 
-// Shared tiles of the split kernel with at most this many partials are
-// finished in it: a second launch costs more than the last workgroup's reads.
-static constexpr int kSplitInKernelParts = 8;
-
 template <class T, class OA, class OB>
 static void launch_gemm_split(GemmArgs& g, int batches, const StreamK& sk, const char* name, const char* kname) {
     auto kernel = gemm_split_k<T, OA, OB>;

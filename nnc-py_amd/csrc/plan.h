@@ -235,6 +235,10 @@ struct SplitPlan {
     double us;
 };
 
+// Shared product tiles with at most this many partials are finished in the
+// split kernel: a second launch costs more than the last workgroup's reads.
+constexpr int kSplitInKernelParts = 8;
+
 // parts of a shared tile at most
 inline int64_t split_parts(const StreamK& sk) {
     const int64_t per = sk.total() / sk.G;

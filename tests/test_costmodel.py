@@ -33,10 +33,13 @@ FIXTURE = json.loads((ROOT / "tests" / "golden" / "costmodel_mi355x.json").read_
 FAMILY = [
     (r"conv_stem_rows_", "conv_stem_k"),
     (r"conv_stem_pool_w", "conv_stem_pool_k"),
-    (r"conv_igemm_.*_dma$", "conv_dma_k"),
+    (r"conv_igemm_.*c3_dma$", "conv_dma_k"),
+    (r"conv_igemm_.*_dma$", "conv_split_k"),
+    (r"conv_igemm_32x32_", "conv_wss_k"),
     (r"conv_ws_32x32_", "conv_ws_k"),
     (r"conv_igemm_", "conv_streamk_k"),
     (r"conv_streamk_fixup$", "conv_fixup_k"),
+    (r"gemm_split_", "gemm_split_k"),
     (r"gemm_dma_", "gemm_dma_k"),
     (r"gemm_ws_32x32_", "gemm_ws_k"),
     (r"attention16_d64$", "attention16_k"),
