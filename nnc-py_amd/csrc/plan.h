@@ -206,11 +206,11 @@ constexpr int fixup_slices_for(int bm, int bn) { return (128 * 128) / (bm * bn);
 // products and 43 convolutions on MI355X (the estimate's choice takes 1.03
 // times the best one's time for aligned products, 1.02 for others, 1.01 for
 // convolutions). What it decides, both sides measured: Gemm 2048^3 as 128x128
-// tiles 95 us, as 64x64 107; 2048x1024x256 as 64x64 13.9, as 128x128 15.8;
+// tiles 101 us, as 64x64 134; 2048x1024x256 as 64x64 13.9, as 128x128 19.0;
 // 1024x768x1024 64x64 at three per CU shared 24.3, whole 27; 3x3 convolutions
 // at batch 32: 64 channels 56x56 as 64x256 whole 57, shared 68; 64 -> 128
 // stride 2 as 128x128 whole 36, shared 40; 128 channels 28x28 shared 58, whole
-// 61; 1x1 256 -> 128 28x28 whole 20.4.
+// 61.
 // ---------------------------------------------------------------------------
 struct SplitTileCost {
     int bm, bn, max_per_cu;
