@@ -77,6 +77,25 @@ def test_gemm_edges(m, n, k, nt, hip, abi):
     _check(_gemm(hip, abi, a, b, nt), a, b, f"{m}x{n}x{k}")
 
 
+# (m, n, k, transposed A, transposed B): K a multiple of 4 and no more (both
+# loaders of either operand), K past 16 by 4; one round of fp32 tiles on one
+# workgroup per CU, shared and whole; unaligned rows over two slices on just
+# more than four rounds of 64x64 tiles
+GEMM_ROUTES = [(1500, 1100, 644, ta, tb) for ta in (0, 1) for tb in (0, 1)] + [
+    (700, 900, 564, 0, 1), (495, 320, 3072, 0, 0), (355, 2592, 1152, 0, 1), (1862, 2348, 41, 0, 0)]
+
+
+@pytest.mark.parametrize("m,n,k,ta,tb", GEMM_ROUTES)
+def test_gemm_routes(m, n, k, ta, tb, hip, abi):
+    print(f"case gemm {m}x{n}x{k} ta={ta} tb={tb}", flush=True)
+    rng = np.random.default_rng(m + k)
+    a, b = rng.uniform(-1, 1, (m, k)).astype(np.float32), rng.uniform(-1, 1, (k, n)).astype(np.float32)
+    c = rng.uniform(-1, 1, n).astype(np.float32)
+    got = _call(abi, lambda x, y, z, o, *s: hip.nnc_gemm(x, y, z, o, *s), [a.T if ta else a, b.T if tb else b, c],
+                (1.0, 1.0, ta, tb), (m, n))
+    _check(got, np.hstack([a, np.ones((m, 1), np.float32)]), np.vstack([b, c]), f"{m}x{n}x{k}")
+
+
 def _scaled(which, a, b):
     if which == "small":
         a *= 1e-6
